@@ -38,6 +38,8 @@ struct List
     int32_t cap = 0;          // entries per i-cluster
     uint32_t *cl = nullptr;   // [ncl * cap] j | mask << 24, in search order
     int32_t *cln = nullptr;   // [ncl]
+    char *plan = nullptr;     // queue layout (BS_PAIR_QUEUES): [ncl * nst] QPLAN_BYTES records
+    int32_t nst = 0;          // records per cluster: (cap + 63) / 64
     uint32_t *rows = nullptr; // row layout (BS_PAIR_ROWS): [row blocks * rcap * 64]
     int32_t *rlen = nullptr;  // [row blocks * 64]
     int32_t rcap = 0;
@@ -141,11 +143,13 @@ struct bs_handle
     float4 *pos[2] = {nullptr, nullptr}, *plo[2] = {nullptr, nullptr};
     float4 *vel = nullptr, *jprm = nullptr, *iprm = nullptr, *xref = nullptr, *fext = nullptr, *fout = nullptr;
     double4 *fnb = nullptr;
-    int32_t *sp_ptr = nullptr, *sp_j = nullptr, *perm_d = nullptr;
-    float *sp_k = nullptr, *sp_l0 = nullptr;
+    int32_t *sp_ptr = nullptr, *perm_d = nullptr;
+    uint2 *sp_e = nullptr;
+    float *sp_k = nullptr;
     bool k_uniform = false; // every spring has the stiffness k_uni: the kernels read no per-edge k
     float k_uni = 0.0f;
-    int64_t nedges = 0;
+    int64_t nedges = 0; // directed edges of the force rows (the null edges not counted)
+    int64_t nunits = 0; // EDGE_PAD-edge units of the force rows
     int32_t ncl = 0;                                  // i-clusters of 8
     // bs_adjoint_forward's record: checkpoints, the last segment's positions
     // and the state at x_T, valid while the state is unchanged
@@ -333,7 +337,7 @@ void free_device(bs_handle *h)
         h->pos[b] = h->plo[b] = nullptr;
     }
     f(h->vel); f(h->fnb); f(h->jprm); f(h->iprm); f(h->xref); f(h->fext); f(h->fout);
-    f(h->sp_ptr); f(h->sp_j); f(h->perm_d); f(h->sp_k); f(h->sp_l0);
+    f(h->sp_ptr); f(h->sp_e); f(h->perm_d); f(h->sp_k);
     f(h->cell_of); f(h->counts); f(h->cstart); f(h->ctmp); f(h->cidx);
     f(h->box_part); f(h->box); f(h->energies_d); f(h->status); f(h->counters);
     f(h->epp); f(h->ese); f(h->seg_start); f(h->sys_seg); f(h->seg_part); f(h->sys_E); f(h->shift);
@@ -362,19 +366,21 @@ void free_device(bs_handle *h)
     {
         f(l.cl);
         f(l.cln);
+        f(l.plan);
         f(l.rows);
         f(l.rlen);
     }
     h->lists.clear();
     h->vel = h->jprm = h->iprm = h->xref = h->fext = h->fout = nullptr;
     h->fnb = nullptr;
-    h->sp_ptr = h->sp_j = h->perm_d = nullptr;
-    h->sp_k = h->sp_l0 = nullptr;
+    h->sp_ptr = h->perm_d = nullptr;
+    h->sp_e = nullptr;
+    h->sp_k = nullptr;
     h->cell_of = h->counts = h->cstart = h->ctmp = h->cidx = nullptr;
     h->box_part = h->box = h->energies_d = nullptr;
     h->status = h->counters = nullptr;
     h->cell_cap = 0;
-    h->nedges = 0;
+    h->nedges = h->nunits = 0;
     h->ready = false;
 }
 
@@ -383,7 +389,7 @@ void free_device(bs_handle *h)
 int check_device(bs_handle *h)
 {
     const void *need[] = {h->pos[0], h->pos[1], h->vel, h->fnb, h->jprm, h->iprm, h->xref, h->fext, h->fout,
-                          h->sp_ptr, h->sp_j, h->sp_k, h->sp_l0, h->perm_d, h->cell_of, h->ctmp, h->cidx,
+                          h->sp_ptr, h->sp_e, h->sp_k, h->perm_d, h->cell_of, h->ctmp, h->cidx,
                           h->counts, h->cstart, h->box, h->box_part, h->epp, h->ese, h->seg_start,
                           h->sys_seg, h->seg_part, h->sys_E, h->energies_d, h->status, h->counters, h->ex_ptr,
                           h->ex_w};
@@ -406,7 +412,8 @@ int check_device(bs_handle *h)
         return fail(h, BS_ERR_STATE, "internal: cluster count mismatch");
     for (const auto &l : h->lists)
         if (!l.cl || !l.cln || l.cap <= 0 || l.ncells > h->cell_cap ||
-            (h->p.pair_layout == BS_PAIR_ROWS && (!l.rows || !l.rlen || l.rcap < l.cap)))
+            (h->p.pair_layout == BS_PAIR_ROWS && (!l.rows || !l.rlen || l.rcap < l.cap)) ||
+            (h->p.pair_layout == BS_PAIR_QUEUES && (!l.plan || l.nst * 64 < l.cap)))
             return fail(h, BS_ERR_STATE, "internal: neighbour list buffers missing");
     return BS_OK;
 }
@@ -515,12 +522,17 @@ uint32_t particle_flags(const bs_handle *h, int64_t i)
     return f;
 }
 
+// A particle's share of the steric size as the kernels take it: two factors'
+// product is R^2 (R = sqrt(r_i r_j) for Amber and Lewitt, r_i r_j for
+// Zacharias); the raw radius for the linear wall, which adds them.
+float radius_factor(int32_t steric_mode, float r) { return steric_mode == BS_STERIC_ZACHARIAS_8_6 ? r * r : r; }
+
 float4 jprm_of(const bs_handle *h, int64_t i)
 {
     const bool sq = h->p.steric_mode == BS_STERIC_AMBER_12_6 || h->p.steric_mode == BS_STERIC_LEWITT_8_6;
     const float r = h->radius[(size_t)i], e = h->eps[(size_t)i];
     float4 q;
-    q.x = sq ? sqrtf(r) : r;
+    q.x = radius_factor(h->p.steric_mode, r);
     q.y = sq ? sqrtf(e) : e;
     q.z = h->hydro[(size_t)i];
     uint32_t fl = particle_flags(h, i);
@@ -695,6 +707,8 @@ void build_list(bs_handle *h, List &l, bool gated, int32_t cap_override)
     a.ex_w = h->ex_w;
     a.cl = l.cl;
     a.cln = l.cln;
+    a.plan = cap_override < 0 ? l.plan : nullptr;
+    a.nst = l.nst;
     a.status = h->status;
     a.n = n;
     a.ncl = h->ncl;
@@ -736,47 +750,61 @@ void rebuild_chain(bs_handle *h, bool gated, bool prepped = false)
 
 float rc2(float rc, double f) { return (float)((double)rc * rc * f); }
 
-// energy: also sum this evaluation's energies (the last step of a call).
-void launch_pairs(bs_handle *h, bool energy)
+// The pair kernel's arguments for list li.  energy: also sum this
+// evaluation's energies (the last step of a call).
+PairArgs pair_args(const bs_handle *h, size_t li, bool energy)
 {
     const int32_t n = (int32_t)h->n;
-    for (size_t li = 0; li < h->lists.size(); ++li)
+    const List &l = h->lists[li];
+    PairArgs a{};
+    a.pos = h->pos[h->cur];
+    a.jprm = h->jprm;
+    a.cl = l.cl;
+    a.cln = l.cln;
+    a.fnb = h->fnb;
+    a.epp = h->epp;
+    a.rows = l.rows;
+    a.rlen = l.rlen;
+    a.rcap = l.rcap;
+    a.plan = l.plan;
+    a.nst = l.nst;
+    a.n = n;
+    a.ncl = h->ncl;
+    a.cap = l.cap;
+    a.accumulate = li > 0 ? 1 : 0;
+    a.energy = energy ? 1 : 0;
+    a.status = h->status;
+    a.rc = l.rc;
+    a.rc2lo = rc2(l.rc, 1.0 - 4e-6);
+    a.rc2hi = rc2(l.rc, 1.0 + 4e-6);
+    a.steric_mode = (l.terms & TERM_STERIC) ? h->p.steric_mode : -1;
+    a.steric_scale = h->p.steric_gridscale;
+    a.elec_scale = h->p.electrostatic_scale;
+    a.diel = h->p.electrostatic_dielectric;
+    // Coulomb prefactors (electrostatic.hpp:16-49): energy e_C q1 q2 / (eps d),
+    // force module q1 q2 / (4 pi eps d^2) * C_elec, both times the scale
+    a.ke = h->k.e_coul / a.diel * a.elec_scale;
+    a.kf = h->k.c_elec / (4.0 * h->k.pi * a.diel) * a.elec_scale;
+    a.hydro_scale = h->p.hydrophobicity_scale;
+    a.i_mask = l.imask;
+    a.j_mask = l.jmask;
+    a.k = h->k;
+    return a;
+}
+
+int32_t elec_mode(const bs_handle *h, const List &l)
+{
+    return (l.terms & TERM_ELEC) ? (h->p.dielectric_model == BS_DIELECTRIC_DISTANCE ? 2 : 1) : 0;
+}
+
+// The pair kernels of the first `count` lists.
+void launch_pairs(bs_handle *h, bool energy, size_t count)
+{
+    for (size_t li = 0; li < count; ++li)
     {
         const List &l = h->lists[li];
-        PairArgs a{};
-        a.pos = h->pos[h->cur];
-        a.jprm = h->jprm;
-        a.cl = l.cl;
-        a.cln = l.cln;
-        a.fnb = h->fnb;
-        a.epp = h->epp;
-        a.rows = l.rows;
-        a.rlen = l.rlen;
-        a.rcap = l.rcap;
-        a.queues = h->p.pair_layout == BS_PAIR_QUEUES ? 1 : 0;
-        a.n = n;
-        a.ncl = h->ncl;
-        a.cap = l.cap;
-        a.accumulate = li > 0 ? 1 : 0;
-        a.energy = energy ? 1 : 0;
-        a.status = h->status;
-        a.rc = l.rc;
-        a.rc2lo = rc2(l.rc, 1.0 - 4e-6);
-        a.rc2hi = rc2(l.rc, 1.0 + 4e-6);
-        a.steric_mode = (l.terms & TERM_STERIC) ? h->p.steric_mode : -1;
-        a.steric_scale = h->p.steric_gridscale;
-        a.elec_scale = h->p.electrostatic_scale;
-        a.diel = h->p.electrostatic_dielectric;
-        // Coulomb prefactors (electrostatic.hpp:16-49): energy e_C q1 q2 / (eps d),
-        // force module q1 q2 / (4 pi eps d^2) * C_elec, both times the scale
-        a.ke = h->k.e_coul / a.diel * a.elec_scale;
-        a.kf = h->k.c_elec / (4.0 * h->k.pi * a.diel) * a.elec_scale;
-        a.hydro_scale = h->p.hydrophobicity_scale;
-        a.i_mask = l.imask;
-        a.j_mask = l.jmask;
-        a.k = h->k;
-        const int em = (l.terms & TERM_ELEC) ? (h->p.dielectric_model == BS_DIELECTRIC_DISTANCE ? 2 : 1) : 0;
-        launch_pair(a, em, (l.terms & TERM_HYDRO) ? 1 : 0, h->pair_blocks, h->stream);
+        launch_pair(pair_args(h, li, energy), elec_mode(h, l), (l.terms & TERM_HYDRO) ? 1 : 0, h->pair_blocks,
+                    h->stream);
     }
 }
 
@@ -811,7 +839,7 @@ ProbeArgs probe_args(const bs_handle *h)
     a.steric_mode = P.steric_mode;
     a.steric_scale = P.steric_gridscale;
     const bool sq = P.steric_mode == BS_STERIC_AMBER_12_6 || P.steric_mode == BS_STERIC_LEWITT_8_6;
-    a.radius = sq ? std::sqrt(P.probe_radius) : P.probe_radius; // as jprm holds the particles'
+    a.radius = radius_factor(P.steric_mode, P.probe_radius); // as jprm holds the particles'
     a.eps = sq ? std::sqrt(P.probe_epsilon) : P.probe_epsilon;
     a.mass = P.probe_mass;
     a.ke = h->k.e_coul / P.electrostatic_dielectric * P.electrostatic_scale;
@@ -821,7 +849,7 @@ ProbeArgs probe_args(const bs_handle *h)
     return a;
 }
 
-void launch_springs(bs_handle *h, bool integrate, bool energy)
+SpringArgs spring_args(const bs_handle *h, bool integrate, bool energy)
 {
     SpringArgs a{};
     a.pos = h->pos[h->cur];
@@ -835,10 +863,9 @@ void launch_springs(bs_handle *h, bool integrate, bool energy)
     a.jprm = h->jprm;
     a.xref = h->xref;
     a.sp_ptr = h->sp_ptr;
-    a.sp_j = h->sp_j;
+    a.sp_e = h->sp_e;
     a.sp_k = h->k_uniform ? nullptr : h->sp_k;
     a.k_uni = h->k_uni;
-    a.sp_l0 = h->sp_l0;
     a.perm = h->perm_d;
     a.fout = h->fout;
     a.eps = h->ese;
@@ -868,7 +895,12 @@ void launch_springs(bs_handle *h, bool integrate, bool energy)
     a.e_field = 1.3806504E-23 * 1.0E-3 * 6.02214169E23; // k_B, J -> kJ, N_A (constants.hpp:70-73)
     a.probe = probe_args(h);
     a.steps_done = h->status + 6;
-    launch_spring(a, h->group, h->spring_blocks, h->stream);
+    return a;
+}
+
+void launch_springs(bs_handle *h, bool integrate, bool energy)
+{
+    launch_spring(spring_args(h, integrate, energy), h->group, h->spring_blocks, h->stream);
 }
 
 // The probe's step after the spring kernel (integrate) or its force and pair
@@ -1066,6 +1098,14 @@ int regrow_lists(bs_handle *h)
         l.cap = need;
         l.cl = dalloc<uint32_t>((size_t)h->ncl * l.cap, e);
         HIPCHK(h, e);
+        if (l.plan)
+        {
+            (void)hipFree(l.plan);
+            l.plan = nullptr;
+            l.nst = (l.cap + 63) / 64;
+            l.plan = dalloc<char>((size_t)h->ncl * l.nst * QPLAN_BYTES, e);
+            HIPCHK(h, e);
+        }
         if (l.rows)
         {
             (void)hipFree(l.rows);
@@ -1083,28 +1123,46 @@ int regrow_lists(bs_handle *h)
     return BS_OK;
 }
 
-// One step: rebuild gate, (gated) list rebuild, pair forces, springs +
-// integration, rigid bodies.  energy: also write the per-particle energies.
-void launch_step(bs_handle *h, bool energy)
+// A step's forces and integration, lists in place: the pair forces, springs,
+// rigid bodies and probe.  In the queue layout the last list's pairs, the
+// springs and the integrator are one kernel; the probe's block sums and a
+// profiled call's timing of the two parts need them apart.
+void launch_forces(bs_handle *h, bool energy)
 {
-    const size_t e0 = h->prof ? prof_mark(h) : SIZE_MAX;
-    launch_gate(h, h->p.rebuild_interval, 1);
-    rebuild_chain(h, true, true);
+    const size_t nl = h->lists.size();
+    if (nl > 0 && h->p.pair_layout == BS_PAIR_QUEUES && !h->p.probe_enable && !h->prof)
+    {
+        const List &l = h->lists[nl - 1];
+        launch_pairs(h, energy, nl - 1);
+        launch_step_kernel(pair_args(h, nl - 1, energy), spring_args(h, true, energy), elec_mode(h, l),
+                           (l.terms & TERM_HYDRO) ? 1 : 0, h->stream);
+        launch_bodies(h);
+        return;
+    }
     const size_t e1 = h->prof ? prof_mark(h) : SIZE_MAX;
-    if (!h->lists.empty())
-        launch_pairs(h, energy);
+    launch_pairs(h, energy, nl);
     const size_t e2 = h->prof ? prof_mark(h) : SIZE_MAX;
     launch_springs(h, true, energy);
     launch_bodies(h);
     launch_probe_step(h, true);
     if (h->prof)
     {
-        const size_t e3 = prof_mark(h);
-        prof_span(h, BS_PROF_REBUILD, e0, e1);
-        if (!h->lists.empty())
+        if (nl > 0)
             prof_span(h, BS_PROF_PAIR, e1, e2);
-        prof_span(h, BS_PROF_SPRING, e2, e3);
+        prof_span(h, BS_PROF_SPRING, e2, prof_mark(h));
     }
+}
+
+// One step: rebuild gate, (gated) list rebuild, forces and integration.
+// energy: also write the per-particle energies.
+void launch_step(bs_handle *h, bool energy)
+{
+    const size_t e0 = h->prof ? prof_mark(h) : SIZE_MAX;
+    launch_gate(h, h->p.rebuild_interval, 1);
+    rebuild_chain(h, true, true);
+    if (h->prof)
+        prof_span(h, BS_PROF_REBUILD, e0, prof_mark(h));
+    launch_forces(h, energy);
     h->cur ^= 1;
 }
 
@@ -1113,19 +1171,7 @@ void launch_step(bs_handle *h, bool energy)
 // counter is not advanced; the recomputation restores the counters.
 void launch_step_unlisted(bs_handle *h)
 {
-    const size_t e1 = h->prof ? prof_mark(h) : SIZE_MAX;
-    if (!h->lists.empty())
-        launch_pairs(h, false);
-    const size_t e2 = h->prof ? prof_mark(h) : SIZE_MAX;
-    launch_springs(h, true, false);
-    launch_bodies(h);
-    launch_probe_step(h, true);
-    if (h->prof)
-    {
-        if (!h->lists.empty())
-            prof_span(h, BS_PROF_PAIR, e1, e2);
-        prof_span(h, BS_PROF_SPRING, e2, prof_mark(h));
-    }
+    launch_forces(h, false);
     h->cur ^= 1;
 }
 
@@ -1296,19 +1342,31 @@ void springs_host_changed(bs_handle *h)
 // both ends are static.  Built once per setup.
 int build_spring_owners(bs_handle *h)
 {
-    const int64_t n = h->n, m = h->nsp, E = h->nedges;
+    const int64_t n = h->n, m = h->nsp, E = h->nunits * EDGE_PAD;
     if (h->nslots >= 0 || m == 0)
         return BS_OK;
     const int hrc = springs_host(h);
     if (hrc)
         return hrc;
-    std::vector<int32_t> hp((size_t)n + 1), hj((size_t)std::max<int64_t>(E, 1)), own((size_t)m, -1);
-    HIPCHK(h, hipMemcpy(hp.data(), h->sp_ptr, sizeof(int32_t) * (n + 1), hipMemcpyDeviceToHost));
+    std::vector<int32_t> hu((size_t)n + 1);
+    std::vector<uint2> he((size_t)std::max<int64_t>(E, 1));
+    HIPCHK(h, hipMemcpy(hu.data(), h->sp_ptr, sizeof(int32_t) * (n + 1), hipMemcpyDeviceToHost));
     if (E > 0)
-        HIPCHK(h, hipMemcpy(hj.data(), h->sp_j, sizeof(int32_t) * E, hipMemcpyDeviceToHost));
+        HIPCHK(h, hipMemcpy(he.data(), h->sp_e, sizeof(uint2) * E, hipMemcpyDeviceToHost));
+    // partners of row i's edges: hj[hp[i]] to hj[hp[i + 1]], without the null
+    // edges (partner i) that end a row
+    std::vector<int32_t> hp((size_t)n + 1, 0), hj, own((size_t)m, -1);
+    hj.reserve((size_t)std::max<int64_t>(h->nedges, 1));
+    for (int64_t i = 0; i < n; ++i)
+    {
+        for (int64_t t = (int64_t)hu[(size_t)i] * EDGE_PAD;
+             t < (int64_t)hu[(size_t)i + 1] * EDGE_PAD && he[(size_t)t].x != (uint32_t)i; ++t)
+            hj.push_back((int32_t)he[(size_t)t].x);
+        hp[(size_t)i + 1] = (int32_t)hj.size();
+    }
     // a slot per owned edge: in a moving row, the edges to static partners
     // and to partners of higher index, numbered in edge order
-    std::vector<int32_t> ord((size_t)std::max<int64_t>(E, 1), -1), sp((size_t)n + 1, 0);
+    std::vector<int32_t> ord(std::max<size_t>(hj.size(), 1), -1), sp((size_t)n + 1, 0);
     for (int64_t i = 0; i < n; ++i)
     {
         int32_t c = sp[(size_t)i];
@@ -1687,10 +1745,9 @@ int adjoint_sweep(bs_handle *h, AdjBufs &b, double *dk, double *dl0, double *dq)
             a.jprm = h->jprm;
             a.iprm = h->iprm;
             a.sp_ptr = h->sp_ptr;
-            a.sp_j = h->sp_j;
+            a.sp_e = h->sp_e;
             a.sp_k = h->k_uniform ? nullptr : h->sp_k;
             a.k_uni = h->k_uni;
-            a.sp_l0 = h->sp_l0;
             a.w = wb[wc];
             a.hwp = hwp;
             a.lx = b.lx;
@@ -1859,67 +1916,63 @@ int do_setup(bs_handle *h)
     int32_t *cnt = S.get<int32_t>((size_t)n, e);
     HIPCHK(h, e);
     HIPCHK(h, hipMemcpyAsync(iperm_d, h->iperm.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, st));
+    // the full rows: the force rows unless there are rigid bodies
     const bool any_rigid = !h->bodies.empty();
-    int32_t *fptr = nullptr; // full rows
+    int2 *slot = S.get<int2>((size_t)m, e);
+    HIPCHK(h, e);
+    int32_t *units = S.get<int32_t>((size_t)n, e);
+    HIPCHK(h, e);
+    launch_fill_i32(cnt, 0, n, nullptr, st);
+    launch_edge_count(h->dsa, h->dsb, m, iperm_d, (int32_t)n, cnt, slot, units, st);
+    ALLOC(h->sp_ptr, int32_t, n + 1);
+    int32_t *fptr = h->sp_ptr;
     if (any_rigid)
     {
         fptr = S.get<int32_t>((size_t)n + 1, e);
         HIPCHK(h, e);
     }
-    else
-    {
-        ALLOC(h->sp_ptr, int32_t, n + 1);
-        fptr = h->sp_ptr;
-    }
-    launch_fill_i32(cnt, 0, n, nullptr, st);
-    launch_edge_count(h->dsa, h->dsb, m, iperm_d, cnt, st);
-    launch_scan(cnt, fptr, (int32_t)n, nullptr, st);
-    int32_t efull = 0;
-    HIPCHK(h, hipMemcpyAsync(&efull, fptr + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    launch_scan(units, fptr, (int32_t)n, nullptr, st);
+    int32_t nu = 0;
+    HIPCHK(h, hipMemcpyAsync(&nu, fptr + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
     HIPCHK(h, hipStreamSynchronize(st));
-    uint64_t *key = S.get<uint64_t>((size_t)efull, e);
+    const size_t full = (size_t)nu * EDGE_PAD;
+    uint2 *key = S.get<uint2>(full, e);
     HIPCHK(h, e);
-    int32_t *fej = nullptr;
-    float *fek = nullptr, *fel = nullptr;
+    uint2 *frow = nullptr;
+    float *frk = nullptr;
     if (any_rigid)
     {
-        fej = S.get<int32_t>((size_t)efull, e);
+        frow = S.get<uint2>(full, e);
         HIPCHK(h, e);
-        fek = S.get<float>((size_t)efull, e);
-        HIPCHK(h, e);
-        fel = S.get<float>((size_t)efull, e);
+        frk = S.get<float>(full, e);
         HIPCHK(h, e);
     }
     else
     {
-        ALLOC(h->sp_j, int32_t, efull);
-        ALLOC(h->sp_k, float, efull);
-        ALLOC(h->sp_l0, float, efull);
-        fej = h->sp_j;
-        fek = h->sp_k;
-        fel = h->sp_l0;
+        ALLOC(h->sp_e, uint2, full);
+        ALLOC(h->sp_k, float, full);
+        frow = h->sp_e;
+        frk = h->sp_k;
     }
-    launch_fill_i32(cnt, 0, n, nullptr, st);
-    launch_edge_fill(h->dsa, h->dsb, m, iperm_d, fptr, cnt, key, st);
-    launch_edge_sort(fptr, (int32_t)n, key, h->jprm, h->dsl, h->dsk, fej, fek, fel, st);
+    launch_edge_sort(h->dsa, h->dsb, m, iperm_d, fptr, cnt, (int32_t)n, slot, key, h->jprm, h->dsl, h->dsk, frow, frk,
+                     st);
+    h->nunits = nu;
+    h->nedges = 2 * m;
     // static exclusions per i-cluster: the union of its 8 rows as sorted
     // (j, bonded-mask) words; springs never change during a run
     {
         const int32_t ncl = (int32_t)((n + CLUSTER - 1) / CLUSTER);
-        uint32_t *merged = S.get<uint32_t>((size_t)efull, e);
-        HIPCHK(h, e);
-        int32_t *ucnt = S.get<int32_t>((size_t)ncl, e);
-        HIPCHK(h, e);
-        launch_ex_merge(fptr, fej, (int32_t)n, ncl, merged, ucnt, st);
+        uint32_t *merged = reinterpret_cast<uint32_t *>(key); // the keys are done with
+        int32_t *ucnt = units;
+        launch_ex_merge(fptr, cnt, frow, (int32_t)n, ncl, merged, ucnt, st);
         ALLOC(h->ex_ptr, int32_t, ncl + 1);
         launch_scan(ucnt, h->ex_ptr, ncl, nullptr, st);
         int32_t nex = 0;
         HIPCHK(h, hipMemcpyAsync(&nex, h->ex_ptr + ncl, sizeof(int32_t), hipMemcpyDeviceToHost, st));
         HIPCHK(h, hipStreamSynchronize(st));
         ALLOC(h->ex_w, uint32_t, nex);
-        launch_ex_fill(fptr, (int32_t)n, ncl, merged, h->ex_ptr, h->ex_w, st);
+        launch_ex_fill(fptr, cnt, (int32_t)n, ncl, merged, h->ex_ptr, h->ex_w, st);
     }
-    h->nedges = efull;
     if (any_rigid)
     {
         std::vector<uint8_t> rg((size_t)n);
@@ -1928,17 +1981,23 @@ int do_setup(bs_handle *h)
         uint8_t *rg_d = S.get<uint8_t>((size_t)n, e);
         HIPCHK(h, e);
         HIPCHK(h, hipMemcpyAsync(rg_d, rg.data(), (size_t)n, hipMemcpyHostToDevice, st));
-        launch_edge_keep(fptr, (int32_t)n, fej, fek, fel, rg_d, nullptr, cnt, nullptr, nullptr, nullptr, st);
-        ALLOC(h->sp_ptr, int32_t, n + 1);
-        launch_scan(cnt, h->sp_ptr, (int32_t)n, nullptr, st);
-        int32_t ekeep = 0;
-        HIPCHK(h, hipMemcpyAsync(&ekeep, h->sp_ptr + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+        int32_t *kept = S.get<int32_t>((size_t)n, e);
+        HIPCHK(h, e);
+        int32_t *kptr = S.get<int32_t>((size_t)n + 1, e);
+        HIPCHK(h, e);
+        launch_edge_keep(fptr, cnt, (int32_t)n, frow, frk, rg_d, kept, nullptr, nullptr, nullptr, st);
+        launch_scan(kept, kptr, (int32_t)n, nullptr, st); // the edges left, for the counters
+        launch_edge_units(kept, (int32_t)n, units, st);
+        launch_scan(units, h->sp_ptr, (int32_t)n, nullptr, st);
+        int32_t tot[2] = {0, 0};
+        HIPCHK(h, hipMemcpyAsync(&tot[0], h->sp_ptr + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+        HIPCHK(h, hipMemcpyAsync(&tot[1], kptr + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
         HIPCHK(h, hipStreamSynchronize(st)); // also: rg outlives its copy
-        ALLOC(h->sp_j, int32_t, ekeep);
-        ALLOC(h->sp_k, float, ekeep);
-        ALLOC(h->sp_l0, float, ekeep);
-        launch_edge_keep(fptr, (int32_t)n, fej, fek, fel, rg_d, h->sp_ptr, nullptr, h->sp_j, h->sp_k, h->sp_l0, st);
-        h->nedges = ekeep;
+        h->nunits = tot[0];
+        h->nedges = tot[1];
+        ALLOC(h->sp_e, uint2, h->nunits * EDGE_PAD);
+        ALLOC(h->sp_k, float, h->nunits * EDGE_PAD);
+        launch_edge_keep(fptr, cnt, (int32_t)n, frow, frk, rg_d, nullptr, h->sp_ptr, h->sp_e, h->sp_k, st);
     }
     // one stiffness for every spring (a network built from a cutoff, an
     // elastic network model): the spring kernels read no per-edge k
@@ -2130,6 +2189,11 @@ int do_setup(bs_handle *h)
         const int32_t mx = st[3];
         l.cap = (std::max<int32_t>(16, (int32_t)std::ceil(mx * 1.25) + 64) + 15) / 16 * 16;
         ALLOC(l.cl, uint32_t, (int64_t)h->ncl * l.cap);
+        if (h->p.pair_layout == BS_PAIR_QUEUES)
+        {
+            l.nst = (l.cap + 63) / 64;
+            ALLOC(l.plan, char, (int64_t)h->ncl * l.nst * QPLAN_BYTES);
+        }
         if (h->p.pair_layout == BS_PAIR_ROWS)
         {
             const int64_t nrb = (n + 63) / 64;
@@ -2474,8 +2538,7 @@ int bs_compute_forces(bs_handle *h, const float *ext_force3, float *force3, doub
     launch_fill_i32(h->status + 2, 0, 1, nullptr, h->stream);
     launch_fill_i32(h->status + 5, 0, 1, nullptr, h->stream);
     rebuild_chain(h, true);
-    if (!h->lists.empty())
-        launch_pairs(h, true);
+    launch_pairs(h, true, h->lists.size());
     launch_springs(h, false, true);
     launch_probe_step(h, false);
     rc = finish_call(h);

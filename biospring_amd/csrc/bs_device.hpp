@@ -106,4 +106,11 @@ __device__ inline int32_t internal_coord(float x, double mn, double len, int32_t
     return c < dim - 1 ? c : dim - 1;
 }
 
+// x[j] at a 32-bit offset (j < 2^24, so the base stays in scalar registers);
+// the shift drops an edge word's static bit.
+__device__ inline float4 partner(const float4 *x, uint32_t j)
+{
+    return *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(x) + (j << 4));
+}
+
 } // namespace bs

@@ -6,12 +6,14 @@
 //   plo[2]   float4[N]  low words of x, y, z      compensated positions only
 //   vel      float4[N]  vx, vy, vz, 0
 //   fnb      double4[N] non-bonded force of the current step (FP64 sums)
-//   jprm     float4[N]  sqrt(radius), sqrt(eps), hydrophobicity, flags (bits)
+//   jprm     float4[N]  steric size factor (two multiply to R^2; linear: the
+//            radius), sqrt(eps) or eps, hydrophobicity, flags (bits)
 //   iprm     float4[N]  mass, sasa, transfer, burying
 //   xref     float4[N]  positions at the last neighbour-list build
-//   springs  CSR over particles, both directions, each row sorted by j:
-//            sp_ptr int32[N+1], sp_j int32[E] (bit31 = j static), sp_k float[E],
-//            sp_l0 float[E]
+//   springs  rows over particles, both directions, each sorted by j and padded
+//            with at least one null edge to a multiple of EDGE_PAD edges: row i
+//            is edges EDGE_PAD sp_ptr[i] to EDGE_PAD sp_ptr[i + 1] (int32[N+1]);
+//            sp_e uint2[E] = j (bit 31: j static), L0 bits; sp_k float[E]
 //   lists    per i-cluster of 8 particles: cl[c * cap + t] = j | mask << 24,
 //            cln[c] entries, zero words up to the next multiple of 16
 //   ex       static exclusions per i-cluster: ex_ptr[c], ex_w = j << 8 | mask
@@ -79,23 +81,19 @@ inline Consts make_consts()
 constexpr int32_t CLUSTER = 8;
 constexpr uint32_t CL_JMASK = 0x00FFFFFFu;
 
-// The queue layout reads a cluster's `kept` entries (in search order) in
-// nch = ceil(kept / QCHUNK) chunks of nearly equal size: chunk c holds
-// q + (c < r) entries from offset c q + min(c, r) (q = kept / nch,
-// r = kept mod nch).
-constexpr int32_t QCHUNK = 128;
-struct Chunks
-{
-    int32_t nch, q, r;
-};
-constexpr Chunks chunks_of(int32_t kept) // constexpr: callable on host and device
-{
-    Chunks d{0, 0, 0};
-    d.nch = kept > 0 ? (kept + QCHUNK - 1) / QCHUNK : 0;
-    d.q = kept > 0 ? kept / d.nch : 0;
-    d.r = kept > 0 ? kept - d.q * d.nch : 0;
-    return d;
-}
+// Edges in a unit of the spring rows (64 bytes of edge words).
+constexpr int32_t EDGE_PAD = 8;
+
+// Waves that share one cluster in the queue layout (a power of two).  A wave
+// is long (a dense cluster's list takes tens of microseconds), so few clusters
+// leave the chip's 1024 SIMDs idle or end in a tail: measured per step with 1,
+// 2 and 4 waves at 1,126 clusters 164, 126 and 118 us, at 3,752 clusters 119,
+// 108 and 112, at 6,250 (short lists) 49, 54 and 68, at 31,250 500, 507 and 598.
+constexpr int32_t pair_waves(int32_t ncl) { return ncl <= 2048 ? 4 : ncl <= 5120 ? 2 : 1; }
+
+// A list's plan for the queue layout: one record per stretch of 64 words
+// (QPlan, bs_pairterm.hpp), (cap + 63) / 64 records per cluster.
+constexpr int32_t QPLAN_BYTES = 80;
 
 // Parameters of one pair kernel launch.
 struct PairArgs
@@ -109,7 +107,8 @@ struct PairArgs
     const uint32_t *rows; // nullable: per-particle lists (row layout), else the cluster lists
     const int32_t *rlen;  // [64 * row blocks] entries per particle
     int32_t rcap;         // entries per particle row
-    int32_t queues;       // cluster lists read through per-particle LDS queues (k_pair_q)
+    const char *plan;     // queue layout (else null): the lists' plans, nst records per cluster
+    int32_t nst;
     int32_t n, ncl, cap;
     int32_t accumulate; // add to fnb instead of overwriting
     int32_t energy;     // also write epp (the last step of a call only)
@@ -180,7 +179,7 @@ struct ProbeArgs
     int32_t steric, elec;  // probe terms on
     int32_t steric_mode;
     float steric_scale;
-    float radius, eps;     // probe radius and epsilon in jprm's form (square roots for Amber / Lewitt)
+    float radius, eps;     // probe radius and epsilon in jprm's form
     float mass;
     double ke, kf;         // Coulomb energy / force prefactors incl. scale and 1/dielectric
     int32_t ddd;           // eps(r) = eps r
@@ -200,9 +199,8 @@ struct SpringArgs
     const float4 *jprm;
     const float4 *xref;
     const int32_t *sp_ptr;
-    const int32_t *sp_j;
+    const uint2 *sp_e;
     const float *sp_k;   // null: every spring has stiffness k_uni (not read per edge)
-    const float *sp_l0;
     float k_uni;
     const int32_t *perm;
     float4 *fout;        // forces-only mode
@@ -255,10 +253,9 @@ struct AdjSpringArgs
     const float4 *jprm;
     const float4 *iprm;
     const int32_t *sp_ptr;
-    const int32_t *sp_j;
+    const uint2 *sp_e;
     const float *sp_k;    // null: every spring has stiffness k_uni
     float k_uni;
-    const float *sp_l0;
     const float4 *w;      // [N] weights of this step (FP32)
     const double4 *hwp;   // nullable: pair part of H w
     double4 *lx, *lv;     // [N] adjoint of x and v (updated in place)
@@ -306,6 +303,8 @@ struct ListArgs
     const int32_t *ex_ptr;     // [ncl + 1] static exclusions per i-cluster
     const uint32_t *ex_w;      // j << 8 | bonded mask, sorted by j
     uint32_t *cl;              // [ncl * cap] search order
+    char *plan;                // nullable: the queue layout's plans, nst records per cluster
+    int32_t nst;               // records per cluster
     int32_t *cln;              // [ncl]
     int32_t *status;           // [2] overflow, [3] max count
     int32_t n, ncl, cap;
@@ -344,6 +343,10 @@ void launch_list_build(const ListArgs &a, hipStream_t s);
 void launch_rows(const uint32_t *cl, const int32_t *cln, int32_t ncl, int32_t cap, uint32_t *rows, int32_t *rlen,
                  int32_t rcap, const int32_t *gate, hipStream_t s);
 void launch_pair(const PairArgs &a, int32_t elec_mode, int32_t hydro, int32_t nblocks, hipStream_t s);
+// One step after the lists (bs_step.hip): the pair forces of list p, added to
+// those of earlier lists (p.accumulate), the springs and the integration, in
+// the queue layout.  No probe (a.probe.state null).
+void launch_step_kernel(const PairArgs &p, const SpringArgs &a, int32_t elec_mode, int32_t hydro, hipStream_t s);
 void launch_spring(const SpringArgs &a, int32_t group, int32_t nblocks, hipStream_t s);
 // Per-system energies from the per-particle ones: segments of contiguous
 // particles (never crossing a system) are summed by one workgroup each, then
@@ -389,28 +392,31 @@ void launch_spring_grads(float *dke, float *dle, int64_t nslots, double *dk, dou
 void launch_spring_out(const int32_t *slot_of, int64_t m, const double *dk, const double *dl0, double *outk,
                        double *outl, hipStream_t s);
 void launch_topo_springs(const TopoArgs &a, hipStream_t s);
-// Spring CSR on the device from the spring table (sa, sb: external ids; m
-// springs; iperm: external -> internal).  Count pass (cnt zeroed: both ends
-// of each spring), fill pass (cursor zeroed; 64-bit keys partner << 32 |
-// spring << 1 | side at the rows' offsets ptr), then the rows sorted by key
-// and written as partner (bit 31: static partner), stiffness, rest length.
-void launch_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t *cnt,
-                       hipStream_t s);
-void launch_edge_fill(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const int32_t *ptr,
-                      int32_t *cursor, uint64_t *key, hipStream_t s);
-void launch_edge_sort(const int32_t *ptr, int32_t n, const uint64_t *key, const float4 *jprm, const float *sl,
-                      const float *sk, int32_t *ej, float *ek, float *el, hipStream_t s);
+// Spring rows on the device from the spring table (sa, sb: external ids; m
+// springs; iperm: external -> internal).  Count pass (cnt zeroed): the edges
+// of each row, every edge's place in its rows, and the units of the padded
+// rows.
+void launch_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t n, int32_t *cnt,
+                       int2 *slot, int32_t *units, hipStream_t s);
+void launch_edge_units(const int32_t *cnt, int32_t n, int32_t *units, hipStream_t s);
+// Then, with the rows' units in ptr: the edges as {partner, spring} into key
+// (as many words as the rows), sorted by partner and written with their rest
+// lengths and stiffnesses, padded with null edges.
+void launch_edge_sort(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const int32_t *ptr,
+                      const int32_t *cnt, int32_t n, const int2 *slot, uint2 *key, const float4 *jprm, const float *sl,
+                      const float *sk, uint2 *rows, float *rk, hipStream_t s);
 // Exclusions of each i-cluster from its rows: merged (j << 8 | row bit, in
-// j order) into merged[ptr[8c] ..) with the count of distinct j per cluster,
-// then the distinct words (row bits of equal j or-ed) at ex_ptr[c].
-void launch_ex_merge(const int32_t *ptr, const int32_t *ej, int32_t n, int32_t ncl, uint32_t *merged,
-                     int32_t *ucount, hipStream_t s);
-void launch_ex_fill(const int32_t *ptr, int32_t n, int32_t ncl, const uint32_t *merged, const int32_t *ex_ptr,
-                    uint32_t *ex_w, hipStream_t s);
-// Rows without the edges joining two rigid members (rigid[i] != 0): fptr
-// null counts them into cnt; otherwise they are copied to fptr's offsets.
-void launch_edge_keep(const int32_t *ptr, int32_t n, const int32_t *ej, const float *ek, const float *el,
-                      const uint8_t *rigid, const int32_t *fptr, int32_t *cnt, int32_t *fej, float *fek, float *fel,
+// j order) from merged[EDGE_PAD ptr[8c]] on with the count of distinct j per
+// cluster, then the distinct words (row bits of equal j or-ed) at ex_ptr[c].
+void launch_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n, int32_t ncl,
+                     uint32_t *merged, int32_t *ucount, hipStream_t s);
+void launch_ex_fill(const int32_t *ptr, const int32_t *cnt, int32_t n, int32_t ncl, const uint32_t *merged,
+                    const int32_t *ex_ptr, uint32_t *ex_w, hipStream_t s);
+// Rows without the edges joining two rigid members (rigid[i] != 0): krows
+// null counts each row's edges into kept; otherwise they are written at
+// kptr's units, padded.
+void launch_edge_keep(const int32_t *ptr, const int32_t *cnt, int32_t n, const uint2 *rows, const float *rk,
+                      const uint8_t *rigid, int32_t *kept, const int32_t *kptr, uint2 *krows, float *kk,
                       hipStream_t s);
 // ida[t] = i for t in [offs[i], offs[i + 1]).
 void launch_rows_expand(const int32_t *offs, int32_t n, uint32_t *ida, hipStream_t s);

@@ -4,7 +4,7 @@
 // Every kernel is wave64-shaped; none uses floating-point atomics, so the
 // forces and energies of a step are bitwise reproducible run to run.  Integer
 // atomics are used only for histogram counts and flags.
-#include "bs_device.hpp"
+#include "bs_spring.hpp"
 
 #include <cmath>
 
@@ -282,179 +282,6 @@ __global__ void k_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *st
 }
 
 // ---------------------------------------------------------------------------
-// IMPALA (imp.hpp:29-159, ForceField.cpp:62-86) in FP64: returns the energy
-// and adds the force (the negated gradient vector times the scale) to f.
-// The curved geometry z' = sqrt(x^2 + (z - c)^2) - R cancels two numbers of
-// the size of the tube radius, so it is formed in double.
-// ---------------------------------------------------------------------------
-__device__ inline double imp_eval(float xf, float zf, float sasa, float tr, float uo, float lo, float uc, float lc,
-                                  float scale, double c_spring, double f[3])
-{
-    const double alpha = (double)1.99f, z0 = 15.75, alip = (double)-0.018f;
-    const bool flat = uo == 0.0f && lo == 0.0f && uc == 0.0f && lc == 0.0f;
-    const double x = xf, z = zf;
-    const double ru = uc == 0.0f ? 1000000.0 : fabs(1.0 / (double)uc);
-    const double rl = lc == 0.0f ? 1000000.0 : fabs(1.0 / (double)lc);
-    const int su = (uc > 0.0f) - (uc < 0.0f), sl = (lc > 0.0f) - (lc < 0.0f);
-    const double cu = (double)uo - su * ru, cl = -(double)lo - sl * rl;
-    const double vu0 = x, vu2 = z - cu, vl0 = x, vl2 = z - cl;
-    const double nu = sqrt(vu0 * vu0 + vu2 * vu2);
-    const double nl = sqrt(vl0 * vl0 + vl2 * vl2);
-    const double zu = su == 0 ? z : (z > cu ? su * nu + uo - ru : -su * nu + uo - ru);
-    const double zl = sl == 0 ? z : (z > cl ? sl * nl - lo - rl : -sl * nl - lo - rl);
-    const double wu = zu - uo, wl = zl + lo;
-    const double xu = exp(alpha * (fabs(wu) - z0)), xl = exp(alpha * (fabs(wl) - z0));
-    const double pre = -(double)sasa * tr + alip * sasa;
-    const double eu = pre * (0.5 - 1.0 / (1.0 + xu));
-    const double el = pre * (0.5 - 1.0 / (1.0 + xl));
-    double dcu = alpha * wu * xu / ((xu + 1.0) * (xu + 1.0) * fabs(wu));
-    double dcl = alpha * wl * xl / ((xl + 1.0) * (xl + 1.0) * fabs(wl));
-    if (!isfinite(dcu))
-        dcu = 0.0;
-    if (!isfinite(dcl))
-        dcl = 0.0;
-    double du[3] = {0.0, 0.0, 1.0}, dl[3] = {0.0, 0.0, 1.0};
-    if (su != 0)
-    {
-        const double inv = nu > 1e-40 ? 1.0 / nu : 0.0;
-        du[0] = vu0 * inv;
-        du[2] = vu2 * inv;
-    }
-    if (sl != 0)
-    {
-        const double inv = nl > 1e-40 ? 1.0 / nl : 0.0;
-        dl[0] = vl0 * inv;
-        dl[2] = vl2 * inv;
-    }
-    const double mu = pre * dcu * c_spring, ml = pre * dcl * c_spring;
-    for (int c = 0; c < 3; ++c)
-        f[c] -= (double)scale * (flat ? du[c] * mu : du[c] * mu + dl[c] * ml);
-    return (double)scale * (flat ? eu : eu + el);
-}
-
-// One spring edge seen from row i: force on i and the energy share.  The
-// extension len - L0 is formed from an FP64 length (rsqrt seed plus one
-// Newton step) so that it keeps full accuracy near rest.
-template <bool COMP>
-__device__ inline void spring_edge(float4 pi, float4 li, float4 pj, const float4 *plo, int32_t j, float k, float l0,
-                                   bool jstatic, double cs, float scale, bool energy, double &fx, double &fy,
-                                   double &fz, double &e)
-{
-    double dx = (double)pj.x - (double)pi.x;
-    double dy = (double)pj.y - (double)pi.y;
-    double dz = (double)pj.z - (double)pi.z;
-    if (COMP)
-    {
-        const float4 lj = plo[j];
-        dx += (double)lj.x - (double)li.x;
-        dy += (double)lj.y - (double)li.y;
-        dz += (double)lj.z - (double)li.z;
-    }
-    const double r2 = dx * dx + dy * dy + dz * dz;
-    double len = 0.0;
-    float inv = 0.0f;
-    if (r2 > 0.0)
-    {
-        inv = rsqrtf((float)r2);
-        const double s = r2 * (double)inv;
-        len = fma(fma(-s, s, r2), 0.5 * (double)inv, s);
-    }
-    const double ext = len - (double)l0;
-    const double y = inv; // 1/len refined in FP64 for the unit vector
-    const double fm = (double)k * ext * cs * (y * fma(-0.5 * r2, y * y, 1.5));
-    fx = fma(dx, fm, fx);
-    fy = fma(dy, fm, fy);
-    fz = fma(dz, fm, fz);
-    if (energy)
-        e += (jstatic ? 1.0 : 0.5) * 0.5 * (double)scale * (double)k * ext * ext;
-}
-
-// Cell of a field grid holding a position, -1 off the grid
-// (GridCoordinatesSystem.hpp:85-93,206-218: off when x < min or x > max - 1e-6).
-__device__ inline int64_t grid_cell(const GridView &g, float x, float y, float z)
-{
-    const double p[3] = {x, y, z};
-    int64_t q[3];
-    for (int c = 0; c < 3; ++c)
-    {
-        if (!(p[c] >= g.origin[c]) || p[c] > g.bmax[c] - 1e-6)
-            return -1;
-        q[c] = (int64_t)(int32_t)((p[c] - g.origin[c]) / g.cell[c]);
-        if (q[c] >= g.shape[c])
-            return -1;
-    }
-    return (q[0] * g.shape[1] + q[1]) * g.shape[2] + q[2];
-}
-
-// One particle's interactions with the probe (Particle::addStericProbeForce /
-// addElectrostaticProbeForce, Particle.cpp:434-465), in FP64: the force on
-// the particle goes to f; the pair energies (in full) to es, ee.  The
-// formulas are the pair kernel's (energy/steric.hpp, electrostatic.hpp) with
-// the probe as the first particle; no cutoff and no spring exclusion.
-__device__ inline void probe_pair(const ProbeArgs &p, const float4 q, float4 pi, float4 ri, double cs, double f[3],
-                                  double &es, double &ee)
-{
-    const double dx = (double)q.x - (double)pi.x, dy = (double)q.y - (double)pi.y, dz = (double)q.z - (double)pi.z;
-    const double r = sqrt(dx * dx + dy * dy + dz * dz);
-    const double inv = r > 1e-40 ? 1.0 / r : 0.0; // a zero vector stays zero (Vector3f::normalize)
-    double fm = 0.0;
-    if (p.steric)
-    {
-        double e = 0.0, m = 0.0;
-        if (p.steric_mode == 0)
-        { // linear: overlap of the raw radii
-            const double dv = r - ((double)p.radius + (double)ri.x);
-            if (!(dv > 0.0))
-            {
-                e = 0.5 * dv * dv;
-                m = -fabs(dv) * cs;
-            }
-        }
-        else if (r >= 0.1)
-        {
-            const bool prod = p.steric_mode == 3; // Zacharias: raw products; else square-root factors
-            const double eij = (double)p.eps * (double)ri.y;
-            const double R = (double)p.radius * (double)ri.x;
-            const double sr = R * inv, s2 = sr * sr, s6 = s2 * s2 * s2;
-            if (p.steric_mode == 1)
-            { // Amber 12-6
-                e = eij * s6 * s6 - 2.0 * eij * s6;
-                m = (-12.0 * eij * s6 * s6 + 12.0 * eij * s6) * inv * cs;
-            }
-            else if (p.steric_mode == 2)
-            { // Lewitt 8-6
-                e = 3.0 * eij * s6 * s2 - 4.0 * eij * s6;
-                m = (-24.0 * eij * s6 * s2 + 24.0 * eij * s6) * inv * cs;
-            }
-            else if (prod)
-            { // Zacharias 8-6
-                e = eij * s6 * s2 - eij * s6;
-                m = (-8.0 * eij * s6 * s2 + 6.0 * eij * s6) * inv * cs;
-            }
-        }
-        es += (double)p.steric_scale * e;
-        fm += (double)p.steric_scale * m;
-    }
-    if (p.elec && r >= 0.001)
-    {
-        const double qq = (double)q.w * (double)pi.w;
-        if (p.ddd)
-        { // eps(r) = eps r
-            ee += p.ke * qq * inv * inv;
-            fm += -2.0 * p.kf * qq * inv * inv * inv;
-        }
-        else
-        {
-            ee += p.ke * qq * inv;
-            fm += -p.kf * qq * inv * inv;
-        }
-    }
-    f[0] += dx * inv * fm;
-    f[1] += dy * inv * fm;
-    f[2] += dz * inv * fm;
-}
-
-// ---------------------------------------------------------------------------
 // Springs (CSR gather, G lanes per row, 8 edges in flight per lane) fused with
 // viscosity, external and IMPALA forces and the viscous semi-implicit Euler
 // step (SpringNetwork.cpp:63-90,202-241; Spring.cpp:20-34; Particle.cpp:80-128).
@@ -477,9 +304,7 @@ __global__ void __launch_bounds__(BLOCK) k_spring(SpringArgs a)
     }
     if (INTEGRATE && tid == 0 && a.steps_done)
         atomicAdd(a.steps_done, 1);
-    double espr = 0.0, eke = 0.0, eimp = 0.0, efld = 0.0;
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    double pf[3] = {0.0, 0.0, 0.0}, pes = 0.0, pee = 0.0; // force on the probe, probe pair energies
+    RowOut o;
     const bool active = row < a.n;
     float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), li = make_float4(0.f, 0.f, 0.f, 0.f);
     uint32_t fli = PF_STATIC;
@@ -491,55 +316,15 @@ __global__ void __launch_bounds__(BLOCK) k_spring(SpringArgs a)
             li = a.plo[row];
     }
     const bool dyn = active && !(fli & PF_STATIC);
-    if (dyn && a.spring_enable)
+    RowSum<COMP> sum(pi, li);
+    const int32_t row0 = __builtin_amdgcn_readfirstlane(row);
+    if (row0 < a.n && a.spring_enable) // wave-uniform
     {
-        const int32_t beg = a.sp_ptr[row], end = a.sp_ptr[row + 1];
-        const double cs = a.k.c_spring * (double)a.spring_scale;
-        constexpr int U = 8;
-        // the edge words of the next iteration load while this one gathers
-        // and computes (two dependent loads per edge: the word, then x_j)
-        int32_t jr[U];
-        float kk[U], ll[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-        {
-            const int32_t e = beg + lane + u * G;
-            const bool ok = e < end;
-            jr[u] = ok ? a.sp_j[e] : 0;
-            kk[u] = ok ? (a.sp_k ? a.sp_k[e] : a.k_uni) : 0.0f;
-            ll[u] = ok ? a.sp_l0[e] : 0.0f;
-        }
-        for (int32_t e0 = beg + lane; e0 < end; e0 += U * G)
-        {
-            float4 pj[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                pj[u] = a.pos[jr[u] & 0x7fffffff];
-            int32_t jn[U];
-            float kn[U], ln[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const int32_t e = e0 + (U + u) * G;
-                const bool ok = e < end;
-                jn[u] = ok ? a.sp_j[e] : 0;
-                kn[u] = ok ? (a.sp_k ? a.sp_k[e] : a.k_uni) : 0.0f;
-                ln[u] = ok ? a.sp_l0[e] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (e0 + u * G < end)
-                    spring_edge<COMP>(pi, li, pj[u], a.plo, jr[u] & 0x7fffffff, kk[u], ll[u], jr[u] < 0, cs,
-                                      a.spring_scale, a.energy != 0, fx, fy, fz, espr);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                jr[u] = jn[u];
-                kk[u] = kn[u];
-                ll[u] = ln[u];
-            }
-        }
+        EdgeRow er(a, row0, row, lane, G, dyn);
+        row_springs<8, COMP>(a, er, sum, a.energy != 0);
     }
+    const double cs = a.k.c_spring * (double)a.spring_scale;
+    double fx = sum.fx * cs, fy = sum.fy * cs, fz = sum.fz * cs, espr = sum.e;
     // reduce the force (and the spring energy) over the G lanes of the row
     for (int off = G / 2; off > 0; off >>= 1)
     {
@@ -551,145 +336,21 @@ __global__ void __launch_bounds__(BLOCK) k_spring(SpringArgs a)
     }
     if (dyn && lane == 0)
     {
-        float4 v = a.vel[row];
-        double sx = fx, sy = fy, sz = fz;
         if (a.fnb)
         {
             const double4 fn = a.fnb[row];
-            sx += fn.x;
-            sy += fn.y;
-            sz += fn.z;
+            fx += fn.x;
+            fy += fn.y;
+            fz += fn.z;
         }
-        if (a.fext)
-        {
-            const float4 fe = a.fext[row];
-            sx += fe.x;
-            sy += fe.y;
-            sz += fe.z;
-        }
-        if (a.probe.state)
-        { // the probe: the particle's share here, the opposite on the probe
-            double f[3] = {0.0, 0.0, 0.0};
-            probe_pair(a.probe, a.probe.state->x, pi, a.jprm[row], a.k.c_spring, f, pes, pee);
-            sx += f[0];
-            sy += f[1];
-            sz += f[2];
-            pf[0] = -f[0];
-            pf[1] = -f[1];
-            pf[2] = -f[2];
-        }
-        const float4 ip = a.iprm[row];
-        // field forces: nearest-lower-cell lookup, no interpolation
-        // (Particle.cpp:136-189); off-grid particles get nothing
-        if (a.gpot.cells)
-        {
-            const int64_t c = grid_cell(a.gpot, pi.x, pi.y, pi.z);
-            if (c >= 0)
-            {
-                const float4 g = a.gpot.cells[c];
-                const double qs = (double)pi.w * (double)a.gpot.scale;
-                sx += (double)g.x * qs;
-                sy += (double)g.y * qs;
-                sz += (double)g.z * qs;
-                efld += (double)g.w * qs * a.e_field;
-            }
-        }
-        if (a.gden.cells)
-        {
-            const int64_t c = grid_cell(a.gden, pi.x, pi.y, pi.z);
-            if (c >= 0)
-            {
-                const float4 g = a.gden.cells[c];
-                const double bs = (double)ip.w * (double)a.gden.scale;
-                sx += (double)g.x * bs;
-                sy += (double)g.y * bs;
-                sz += (double)g.z * bs;
-            }
-        }
-        if (a.imp_enable)
-        {
-            double f[3] = {sx, sy, sz};
-            eimp += imp_eval(pi.x, pi.z, ip.y, ip.z, a.imp_uo, a.imp_lo, a.imp_uc, a.imp_lc, a.imp_scale,
-                             a.k.c_spring, f);
-            sx = f[0];
-            sy = f[1];
-            sz = f[2];
-        }
-        // the position-dependent sum is rounded once; the viscous term
-        // -gamma v follows in FP32 (Particle.cpp:80-84)
-        float fxf = (float)sx, fyf = (float)sy, fzf = (float)sz;
-        if (a.visc_enable)
-        {
-            fxf -= v.x * a.visc;
-            fyf -= v.y * a.visc;
-            fzf -= v.z * a.visc;
-        }
-        const float fx = fxf, fy = fyf, fz = fzf;
-        if (!INTEGRATE)
-        {
-            a.fout[row] = make_float4(fx, fy, fz, 0.0f);
-        }
-        else if (fli & PF_RIGID)
-        {
-            // placed by its body after the body solve (k_rigid_place); a rigid
-            // particle's kinetic energy is reset before it is summed
-            // (RigidBody.cpp:629, SpringNetwork.cpp:232)
-            a.frig[row] = make_double4(fx, fy, fz, 0.0);
-        }
-        else
-        {
-            const float m = ip.x;
-            const float dt = a.dt;
-            if (m > 0.0f)
-            {
-                v.x = v.x + (fx / m) * dt;
-                v.y = v.y + (fy / m) * dt;
-                v.z = v.z + (fz / m) * dt;
-            }
-            eke += 0.5 * (double)m * ((double)v.x * v.x + (double)v.y * v.y + (double)v.z * v.z) * a.k.c_kinetic;
-            float4 xn = pi;
-            if (COMP)
-            {
-                // two-sum of hi + v*dt, carried into the low word
-                float4 ln = li;
-                const float u[3] = {v.x * dt, v.y * dt, v.z * dt};
-                float *hp[3] = {&xn.x, &xn.y, &xn.z};
-                float *lp[3] = {&ln.x, &ln.y, &ln.z};
-                for (int c = 0; c < 3; ++c)
-                {
-                    const float h = *hp[c];
-                    const float s = h + u[c];
-                    const float bb = s - h;
-                    const float err = (h - (s - bb)) + (u[c] - bb);
-                    const float lo = *lp[c] + err;
-                    const float h2 = s + lo;
-                    *lp[c] = lo - (h2 - s);
-                    *hp[c] = h2;
-                }
-                a.plo_out[row] = ln;
-            }
-            else
-            {
-                xn.x = pi.x + v.x * dt;
-                xn.y = pi.y + v.y * dt;
-                xn.z = pi.z + v.z * dt;
-            }
-            if (!isfinite(xn.x) || !isfinite(xn.y) || !isfinite(xn.z))
-                atomicMin(&a.status[1], a.perm[row]);
-            const float4 xr = a.xref[row];
-            const float ex = xn.x - xr.x, ey = xn.y - xr.y, ez = xn.z - xr.z;
-            if (!(ex * ex + ey * ey + ez * ez <= a.half_skin2))
-                atomicOr(&a.status[7], 1);
-            a.vel[row] = v;
-            a.pos_out[row] = xn;
-        }
+        finish_row<INTEGRATE, COMP>(a, row, pi, li, fli, fx, fy, fz, o);
     }
     if (a.energy && active && lane == 0)
-        a.eps[row] = make_double4(espr, eke, eimp, efld);
+        a.eps[row] = make_double4(espr, o.eke, o.eimp, o.efld);
     if (a.probe.state)
     { // block sums of the probe's force and pair energies, in a fixed order
         __shared__ double psh[BLOCK / 64];
-        const double v[5] = {pf[0], pf[1], pf[2], pes, pee};
+        const double v[5] = {o.pf[0], o.pf[1], o.pf[2], o.pes, o.pee};
         for (int k = 0; k < 5; ++k)
         {
             const double t = block_sum(v[k], psh);
@@ -1139,62 +800,52 @@ __global__ void __launch_bounds__(BLOCK) k_adj_spring(AdjSpringArgs a)
         wi = make_double4(wf.x, wf.y, wf.z, 0.0);
     }
     const bool dyn = active && !(fli & PF_STATIC);
-    if (dyn && a.spring_enable)
+    const int32_t row0 = __builtin_amdgcn_readfirstlane(row);
+    if (row0 < a.n && a.spring_enable) // wave-uniform
     {
         const double C = a.k.c_spring * (double)a.spring_scale;
-        const int32_t beg = a.sp_ptr[row], end = a.sp_ptr[row + 1];
+        EdgeRow er(a, row0, row, lane, G, dyn);
         // the row's next slot: owned edges take consecutive slots in edge
         // order, counted over the row's G lanes with a ballot per batch
-        int32_t next_slot = a.dk ? a.slot_ptr[row] : 0;
+        int32_t next_slot = a.dk ? a.slot_ptr[min(row, a.n - 1)] : 0;
         const int32_t gbase = (int32_t)(threadIdx.x & 63u) - lane; // first lane of the row in the wave
         const uint64_t gmask = ((1ull << G) - 1ull) << gbase; // G <= 32
+        const bool own = a.dk && dyn;
+        const double px = pi.x, py = pi.y, pz = pi.z;
         constexpr int U = 4; // edges in flight per lane
         // the edge words of the next iteration load while this one gathers
         // and computes
-        int32_t jr[U];
+        uint32_t jr[U];
         float kk[U], ll[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
+            er.word(u, jr[u], ll[u], kk[u]);
+        for (int32_t it = (er.steps() + U - 1) / U; it > 0; --it)
         {
-            const int32_t e = beg + lane + u * G;
-            const bool ok = e < end;
-            jr[u] = ok ? a.sp_j[e] : row;
-            kk[u] = ok ? (a.sp_k ? a.sp_k[e] : a.k_uni) : 0.0f;
-            ll[u] = ok ? a.sp_l0[e] : 0.0f;
-        }
-        for (int32_t e0 = beg + lane; e0 < end; e0 += U * G)
-        {
-            int32_t jn[U];
+            uint32_t jn[U];
             float kn[U], ln[U];
             float4 pj[U], wj[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
-                pj[u] = a.pos[jr[u] & 0x7fffffff];
-                wj[u] = a.w[jr[u] & 0x7fffffff];
+                pj[u] = partner(a.pos, jr[u]);
+                wj[u] = partner(a.w, jr[u]);
             }
+            er.off += U * er.step;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                er.word(u, jn[u], ln[u], kn[u]);
 #pragma unroll
             for (int u = 0; u < U; ++u)
             {
-                const int32_t e = e0 + (U + u) * G;
-                const bool ok = e < end;
-                jn[u] = ok ? a.sp_j[e] : row;
-                kn[u] = ok ? (a.sp_k ? a.sp_k[e] : a.k_uni) : 0.0f;
-                ln[u] = ok ? a.sp_l0[e] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                const int32_t e = e0 + u * G;
-                const int32_t j = jr[u] & 0x7fffffff;
-                const bool owned = a.dk && e < end && (jr[u] < 0 || j > row);
+                // a null edge's partner is the row itself: not owned
+                const bool owned = own && (int32_t)jr[u] != row && ((int32_t)jr[u] < 0 || (int32_t)jr[u] > row);
                 const uint64_t ob = __ballot(owned) & gmask;
                 const int32_t slot = next_slot + (int32_t)__popcll(ob & ((1ull << (threadIdx.x & 63u)) - 1ull));
                 next_slot += (int32_t)__popcll(ob);
-                const double dx = (double)pj[u].x - (double)pi.x, dy = (double)pj[u].y - (double)pi.y,
-                             dz = (double)pj[u].z - (double)pi.z;
+                const double dx = (double)pj[u].x - px, dy = (double)pj[u].y - py, dz = (double)pj[u].z - pz;
                 const double r2 = dx * dx + dy * dy + dz * dz;
-                if (!(e < end && r2 > 0.0))
+                if (!(r2 > 0.0))
                     continue;
                 const double k = kk[u], l0 = ll[u];
                 const double ir = rsqrt_d(r2), r = r2 * ir;
@@ -1553,78 +1204,132 @@ __global__ void k_fill_i32(int32_t *p, int32_t v, int64_t n, const int32_t *gate
 }
 
 // ---------------------------------------------------------------------------
-// Spring CSR built on the device from the spring table (external ids): both
-// directions, each row sorted by (partner, spring, side); the exclusions of
-// each i-cluster merged from its rows; springs between two rigid members
-// left out of the force rows.
+// Spring rows built on the device from the spring table (external ids): both
+// directions, each row sorted by partner and padded with null edges (EdgeRow,
+// bs_spring.hpp); the exclusions of each i-cluster merged from its rows;
+// springs between two rigid members left out of the force rows.
 // ---------------------------------------------------------------------------
-__global__ void k_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t *cnt)
+// Counts each row's edges and gives every edge its (arbitrary) place in the
+// row: slot[2 s] in the row of the spring's first end, slot[2 s + 1] in that of
+// its second.  Tables are often ordered by the first end, so equal first ends
+// of neighbouring lanes share one atomic.
+__global__ void k_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t *cnt,
+                             int2 *slot)
 {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (s >= m)
-        return;
-    atomicAdd(&cnt[iperm[sa[s]]], 1);
-    atomicAdd(&cnt[iperm[sb[s]]], 1);
+    const int lane = threadIdx.x & 63;
+    const bool in = s < m;
+    const int32_t a = in ? iperm[sa[s]] : -1;
+    const int32_t before = __shfl_up(a, 1, 64); // every lane takes part
+    const bool first = lane == 0 || a != before;
+    const uint64_t heads = __ballot(first);
+    const int lead = 63 - __clzll(heads & (~0ull >> (63 - lane)));
+    const uint64_t later = lead == 63 ? 0ull : heads >> (lead + 1);
+    const int run = later ? __builtin_ctzll(later) + 1 : 64 - lead;
+    int32_t base = 0;
+    if (in && first)
+        base = atomicAdd(&cnt[a], run);
+    base = __shfl(base, lead, 64);
+    if (in)
+        slot[s] = make_int2(base + lane - lead, atomicAdd(&cnt[iperm[sb[s]]], 1));
 }
 
-// key = partner << 32 | (spring << 1 | side), placed at an arbitrary slot of
-// the row (k_edge_sort orders it)
+// Units of each padded row: its edges and at least one null edge.
+__global__ void k_edge_units(const int32_t *cnt, int32_t n, int32_t *units)
+{
+    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        units[i] = (cnt[i] + EDGE_PAD) / EDGE_PAD;
+}
+
+// Every edge as {partner, spring} at its place.
 __global__ void k_edge_fill(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm,
-                            const int32_t *ptr, int32_t *cursor, uint64_t *key)
+                            const int32_t *ptr, const int2 *slot, uint2 *key)
 {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= m)
         return;
     const int32_t a = iperm[sa[s]], b = iperm[sb[s]];
-    const uint32_t w = (uint32_t)s << 1;
-    key[ptr[a] + atomicAdd(&cursor[a], 1)] = (uint64_t)(uint32_t)b << 32 | w;
-    key[ptr[b] + atomicAdd(&cursor[b], 1)] = (uint64_t)(uint32_t)a << 32 | (w | 1u);
+    const int2 at = slot[s];
+    key[(size_t)ptr[a] * EDGE_PAD + at.x] = make_uint2((uint32_t)b, (uint32_t)s);
+    key[(size_t)ptr[b] * EDGE_PAD + at.y] = make_uint2((uint32_t)a, (uint32_t)s);
 }
 
 constexpr int32_t EDGE_WAVES = BLOCK / 64;
-constexpr int32_t EDGE_LDS = 1024; // keys per wave held in LDS; longer rows rank from global memory
+constexpr int32_t EDGE_KEYS = 4;             // keys per lane held in registers
+constexpr int32_t EDGE_LDS = 64 * EDGE_KEYS; // longer rows rank from global memory
 
-// One wave per row: each key's rank is the number of smaller keys in the row
-// (keys are distinct).  Writes the partner (bit 31: static partner), its
-// stiffness and rest length at the rank.
-__global__ void __launch_bounds__(BLOCK) k_edge_sort(const int32_t *ptr, int32_t n, const uint64_t *key,
-                                                     const float4 *jprm, const float *sl, const float *sk, int32_t *ej,
-                                                     float *ek, float *el)
+// One wave per row: each key's rank is the number of smaller partners in the
+// row (partners are distinct).  Writes the edge words and stiffnesses in rank
+// order, then the null edges.  Rows up to EDGE_LDS keep their keys in
+// registers and compare all of them with each partner read from LDS: 3.4
+// reads of four partners per key instead of one 64-bit key per pair (1.81 ->
+// 0.62 ms at 100,000 rows of 182).
+__global__ void __launch_bounds__(BLOCK) k_edge_sort(const int32_t *ptr, const int32_t *cnt, int32_t n,
+                                                     const uint2 *key, const float4 *jprm, const float *sl,
+                                                     const float *sk, uint2 *rows, float *rk)
 {
-    __shared__ uint64_t lk[EDGE_WAVES][EDGE_LDS];
+    __shared__ __align__(16) uint32_t lj[EDGE_WAVES][EDGE_LDS];
     const int32_t lane = (int32_t)(threadIdx.x & 63u), w = (int32_t)(threadIdx.x >> 6);
     const int32_t row = (int32_t)blockIdx.x * EDGE_WAVES + w;
     if (row >= n)
         return; // whole wave; no block barrier below
-    const int32_t b = ptr[row], len = ptr[row + 1] - b;
-    const uint64_t *src = key + b;
+    const size_t b = (size_t)ptr[row] * EDGE_PAD;
+    const int32_t len = cnt[row], room = (ptr[row + 1] - ptr[row]) * EDGE_PAD;
+    auto put = [&](uint2 kv, int32_t rank) {
+        const bool st = (fbits(jprm[kv.x].w) & PF_STATIC) != 0u;
+        rows[b + rank] = make_uint2(st ? kv.x | 0x80000000u : kv.x, fbits(sl[kv.y]));
+        rk[b + rank] = sk[kv.y];
+    };
     if (len <= EDGE_LDS)
     {
-        for (int32_t t = lane; t < len; t += 64)
-            lk[w][t] = key[b + t];
+        uint2 kv[EDGE_KEYS];
+        int32_t rank[EDGE_KEYS];
+#pragma unroll
+        for (int q = 0; q < EDGE_KEYS; ++q)
+        {
+            const int32_t t = lane + 64 * q;
+            kv[q] = t < len ? key[b + t] : make_uint2(0xffffffffu, 0u); // past the end: larger than any partner
+            rank[q] = 0;
+            lj[w][t] = kv[q].x;
+        }
         wave_lds_sync();
-        src = lk[w];
+        for (int32_t t = 0; t < len; t += 4)
+        {
+            const uint4 o = *reinterpret_cast<const uint4 *>(&lj[w][t]);
+#pragma unroll
+            for (int q = 0; q < EDGE_KEYS; ++q)
+                rank[q] += (o.x < kv[q].x) + (o.y < kv[q].x) + (o.z < kv[q].x) + (o.w < kv[q].x);
+        }
+#pragma unroll
+        for (int q = 0; q < EDGE_KEYS; ++q)
+            if (lane + 64 * q < len)
+                put(kv[q], rank[q]);
     }
-    for (int32_t e = lane; e < len; e += 64)
+    else
+        for (int32_t e = lane; e < len; e += 64)
+        {
+            const uint2 kv = key[b + e];
+            int32_t rank = 0;
+            for (int32_t t = 0; t < len; ++t)
+                rank += key[b + t].x < kv.x ? 1 : 0;
+            put(kv, rank);
+        }
+    for (int32_t t = len + lane; t < room; t += 64)
     {
-        const uint64_t kv = src[e];
-        int32_t rank = 0;
-        for (int32_t t = 0; t < len; ++t)
-            rank += src[t] < kv ? 1 : 0;
-        const int32_t j = (int32_t)(kv >> 32);
-        const uint32_t s = (uint32_t)kv >> 1;
-        ej[b + rank] = (fbits(jprm[j].w) & PF_STATIC) ? (int32_t)((uint32_t)j | 0x80000000u) : j;
-        ek[b + rank] = sk[s];
-        el[b + rank] = sl[s];
+        rows[b + t] = make_uint2((uint32_t)row, 0u);
+        rk[b + t] = 0.0f;
     }
 }
 
-__device__ inline int32_t row_lower_bound(const int32_t *ej, int32_t lo, int32_t hi, int32_t j, bool upper)
+// Edge words before the first with partner >= j (upper: > j).
+template <class Row> __device__ inline int32_t row_lower_bound(const Row &partner_at, int32_t len, int32_t j, bool upper)
 {
+    int32_t lo = 0, hi = len;
     while (lo < hi)
     {
         const int32_t mid = (lo + hi) >> 1;
-        const int32_t v = ej[mid] & 0x7fffffff;
+        const int32_t v = partner_at(mid);
         if (v < j || (upper && v == j))
             lo = mid + 1;
         else
@@ -1633,103 +1338,150 @@ __device__ inline int32_t row_lower_bound(const int32_t *ej, int32_t lo, int32_t
     return lo;
 }
 
+constexpr int32_t EX_STAGE = 2048; // partners of a cluster's rows held in LDS
+
 // One wave per i-cluster: the words j << 8 | 1 << k of its rows k = 0..7
-// merged in j order (stable in k) into merged[ptr[8c] ..), then the number
-// of distinct j.
-__global__ void k_ex_merge(const int32_t *ptr, const int32_t *ej, int32_t n, int32_t ncl, uint32_t *merged,
-                           int32_t *ucount)
+// merged in j order (stable in k) from merged[EDGE_PAD ptr[8c]] on, then the
+// number of distinct j.  The binary searches run on a copy of the rows in LDS
+// when they fit (0.96 -> 0.45 ms at 100,000 rows of 182).
+__global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n,
+                                                    int32_t ncl, uint32_t *merged, int32_t *ucount)
 {
-    const int32_t lane = (int32_t)(threadIdx.x & 63u);
-    const int32_t c = (int32_t)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
+    __shared__ int32_t stage[EDGE_WAVES][EX_STAGE];
+    const int32_t lane = (int32_t)(threadIdx.x & 63u), w = (int32_t)(threadIdx.x >> 6);
+    const int32_t c = (int32_t)blockIdx.x * EDGE_WAVES + w;
     if (c >= ncl)
-        return;
-    int32_t rb[CLUSTER + 1];
+        return; // whole wave
+    // row k: edges from[k] on, words off[k] to off[k + 1] of the cluster
+    size_t from[CLUSTER];
+    int32_t off[CLUSTER + 1];
+    off[0] = 0;
 #pragma unroll
-    for (int k = 0; k <= CLUSTER; ++k)
-        rb[k] = ptr[min(c * CLUSTER + k, n)];
-    const int32_t base = rb[0], end = rb[CLUSTER];
-    for (int32_t e = base + lane; e < end; e += 64)
+    for (int k = 0; k < CLUSTER; ++k)
     {
-        int32_t k = 0;
+        const int32_t i = c * CLUSTER + k;
+        from[k] = (size_t)ptr[min(i, n)] * EDGE_PAD;
+        off[k + 1] = off[k] + (i < n ? cnt[i] : 0);
+    }
+    const int32_t total = off[CLUSTER];
+    const size_t base = from[0];
+    const bool staged = total <= EX_STAGE;
+    if (staged)
+    {
+#pragma unroll
+        for (int k = 0; k < CLUSTER; ++k)
+            for (int32_t t = lane; t < off[k + 1] - off[k]; t += 64)
+                stage[w][off[k] + t] = (int32_t)(rows[from[k] + t].x & 0x7fffffffu);
+        wave_lds_sync();
+    }
+    for (int32_t e = lane; e < total; e += 64)
+    {
+        int32_t k = 0, start = 0;
+        size_t row = from[0];
 #pragma unroll
         for (int q = 1; q < CLUSTER; ++q)
-            k = e >= rb[q] ? q : k;
-        const int32_t j = ej[e] & 0x7fffffff;
+        {
+            k = e >= off[q] ? q : k;
+            start = e >= off[q] ? off[q] : start;
+            row = e >= off[q] ? from[q] : row;
+        }
+        const int32_t j = staged ? stage[w][e] : (int32_t)(rows[row + (e - start)].x & 0x7fffffffu);
         // rank: its place in its own row, plus the smaller words of the
         // other rows (for rows before its own, the equal ones too)
-        int32_t r = e - rb[k];
+        int32_t r = e - start;
 #pragma unroll
         for (int q = 0; q < CLUSTER; ++q)
             if (q != k)
-                r += row_lower_bound(ej, rb[q], rb[q + 1], j, q < k) - rb[q];
+                r += staged ? row_lower_bound([&](int32_t t) { return stage[w][off[q] + t]; }, off[q + 1] - off[q], j,
+                                              q < k)
+                            : row_lower_bound([&](int32_t t) { return (int32_t)(rows[from[q] + t].x & 0x7fffffffu); },
+                                              off[q + 1] - off[q], j, q < k);
         merged[base + r] = (uint32_t)j << 8 | 1u << k;
     }
     // the wave reads back what its own lanes stored (one CU)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    int32_t cnt = 0;
-    for (int32_t t0 = base; t0 < end; t0 += 64)
+    int32_t u = 0;
+    for (int32_t t0 = 0; t0 < total; t0 += 64)
     {
         const int32_t t = t0 + lane;
-        const bool first = t < end && (t == base || (merged[t - 1] >> 8) != (merged[t] >> 8));
-        cnt += (int32_t)__popcll(__ballot(first));
+        const bool first = t < total && (t == 0 || (merged[base + t - 1] >> 8) != (merged[base + t] >> 8));
+        u += (int32_t)__popcll(__ballot(first));
     }
     if (lane == 0)
-        ucount[c] = cnt;
+        ucount[c] = u;
 }
 
 // The distinct words of each cluster, masks of equal j or-ed, at ex_ptr[c].
-__global__ void k_ex_fill(const int32_t *ptr, int32_t n, int32_t ncl, const uint32_t *merged, const int32_t *ex_ptr,
-                          uint32_t *ex_w)
+__global__ void k_ex_fill(const int32_t *ptr, const int32_t *cnt, int32_t n, int32_t ncl, const uint32_t *merged,
+                          const int32_t *ex_ptr, uint32_t *ex_w)
 {
     const int32_t lane = (int32_t)(threadIdx.x & 63u);
     const int32_t c = (int32_t)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
     if (c >= ncl)
         return;
-    const int32_t base = ptr[min(c * CLUSTER, n)], end = ptr[min(c * CLUSTER + CLUSTER, n)];
+    const uint32_t *mw = merged + (size_t)ptr[c * CLUSTER] * EDGE_PAD;
+    int32_t total = 0;
+    for (int k = 0; k < CLUSTER && c * CLUSTER + k < n; ++k)
+        total += cnt[c * CLUSTER + k];
     int32_t out = ex_ptr[c];
-    for (int32_t t0 = base; t0 < end; t0 += 64)
+    for (int32_t t0 = 0; t0 < total; t0 += 64)
     {
         const int32_t t = t0 + lane;
-        const bool first = t < end && (t == base || (merged[t - 1] >> 8) != (merged[t] >> 8));
+        const bool first = t < total && (t == 0 || (mw[t - 1] >> 8) != (mw[t] >> 8));
         const uint64_t bal = __ballot(first);
         if (first)
         {
-            uint32_t wv = merged[t];
-            for (int32_t u = t + 1; u < end && (merged[u] >> 8) == (wv >> 8); ++u)
-                wv |= merged[u] & 0xFFu;
+            uint32_t wv = mw[t];
+            for (int32_t u = t + 1; u < total && (mw[u] >> 8) == (wv >> 8); ++u)
+                wv |= mw[u] & 0xFFu;
             ex_w[out + (int32_t)__popcll(bal & ((1ull << lane) - 1ull))] = wv;
         }
         out += (int32_t)__popcll(bal);
     }
 }
 
-// Force rows: a row's edges but those joining two rigid-body members.
-__global__ void k_edge_keep(const int32_t *ptr, int32_t n, const int32_t *ej, const float *ek, const float *el,
-                            const uint8_t *rigid, const int32_t *fptr, int32_t *cnt, int32_t *fej, float *fek,
-                            float *fel)
+// Force rows with rigid bodies, one wave per row: the full row's edges but
+// those joining two members, then null edges up to the row's units.
+__global__ void __launch_bounds__(BLOCK) k_edge_keep(const int32_t *ptr, const int32_t *cnt, int32_t n,
+                                                     const uint2 *rows, const float *rk, const uint8_t *rigid,
+                                                     int32_t *kept, const int32_t *kptr, uint2 *krows, float *kk)
 {
-    const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int32_t lane = (int32_t)(threadIdx.x & 63u);
+    const int32_t i = (int32_t)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
     if (i >= n)
-        return;
+        return; // whole wave
+    const size_t b = (size_t)ptr[i] * EDGE_PAD, o = krows ? (size_t)kptr[i] * EDGE_PAD : 0;
+    const int32_t len = cnt[i];
     const bool ri = rigid[i] != 0;
-    int32_t o = fptr ? fptr[i] : 0, c = 0;
-    for (int32_t t = ptr[i]; t < ptr[i + 1]; ++t)
+    int32_t c = 0;
+    for (int32_t t0 = 0; t0 < len; t0 += 64)
     {
-        if (ri && rigid[ej[t] & 0x7fffffff])
-            continue;
-        if (fptr)
+        const int32_t t = t0 + lane;
+        const uint2 e = t < len ? rows[b + t] : make_uint2(0u, 0u);
+        const bool keep = t < len && !(ri && rigid[e.x & 0x7fffffffu]);
+        const uint64_t bal = __ballot(keep);
+        if (krows && keep)
         {
-            fej[o] = ej[t];
-            fek[o] = ek[t];
-            fel[o] = el[t];
-            ++o;
+            const size_t s = o + (size_t)(c + (int32_t)__popcll(bal & ((1ull << lane) - 1ull)));
+            krows[s] = e;
+            kk[s] = rk[b + t];
         }
-        ++c;
+        c += (int32_t)__popcll(bal);
     }
-    if (!fptr)
-        cnt[i] = c;
+    if (!krows)
+    {
+        if (lane == 0)
+            kept[i] = c;
+        return;
+    }
+    const int32_t room = (kptr[i + 1] - kptr[i]) * EDGE_PAD;
+    for (int32_t t = c + lane; t < room; t += 64)
+    {
+        krows[o + (size_t)t] = make_uint2((uint32_t)i, 0u);
+        kk[o + (size_t)t] = 0.0f;
+    }
 }
 
 // Row i of the constructed springs at offs[i]: id1 = i.
@@ -1947,47 +1699,50 @@ void launch_fill_i32(int32_t *p, int32_t v, int64_t n, const int32_t *gate, hipS
     }
 }
 
-void launch_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t *cnt,
-                       hipStream_t s)
+void launch_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t n, int32_t *cnt,
+                       int2 *slot, int32_t *units, hipStream_t s)
 {
     if (m > 0)
-        k_edge_count<<<(int32_t)((m + BLOCK - 1) / BLOCK), BLOCK, 0, s>>>(sa, sb, m, iperm, cnt);
+        k_edge_count<<<(int32_t)((m + BLOCK - 1) / BLOCK), BLOCK, 0, s>>>(sa, sb, m, iperm, cnt, slot);
+    launch_edge_units(cnt, n, units, s);
 }
 
-void launch_edge_fill(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const int32_t *ptr,
-                      int32_t *cursor, uint64_t *key, hipStream_t s)
+void launch_edge_units(const int32_t *cnt, int32_t n, int32_t *units, hipStream_t s)
+{
+    if (n > 0)
+        k_edge_units<<<nblk(n), BLOCK, 0, s>>>(cnt, n, units);
+}
+
+void launch_edge_sort(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const int32_t *ptr,
+                      const int32_t *cnt, int32_t n, const int2 *slot, uint2 *key, const float4 *jprm, const float *sl,
+                      const float *sk, uint2 *rows, float *rk, hipStream_t s)
 {
     if (m > 0)
-        k_edge_fill<<<(int32_t)((m + BLOCK - 1) / BLOCK), BLOCK, 0, s>>>(sa, sb, m, iperm, ptr, cursor, key);
-}
-
-void launch_edge_sort(const int32_t *ptr, int32_t n, const uint64_t *key, const float4 *jprm, const float *sl,
-                      const float *sk, int32_t *ej, float *ek, float *el, hipStream_t s)
-{
+        k_edge_fill<<<(int32_t)((m + BLOCK - 1) / BLOCK), BLOCK, 0, s>>>(sa, sb, m, iperm, ptr, slot, key);
     if (n > 0)
-        k_edge_sort<<<(n + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, n, key, jprm, sl, sk, ej, ek, el);
+        k_edge_sort<<<(n + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, cnt, n, key, jprm, sl, sk, rows, rk);
 }
 
-void launch_ex_merge(const int32_t *ptr, const int32_t *ej, int32_t n, int32_t ncl, uint32_t *merged,
-                     int32_t *ucount, hipStream_t s)
+void launch_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n, int32_t ncl,
+                     uint32_t *merged, int32_t *ucount, hipStream_t s)
 {
     if (ncl > 0)
-        k_ex_merge<<<(ncl + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, ej, n, ncl, merged, ucount);
+        k_ex_merge<<<(ncl + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, cnt, rows, n, ncl, merged, ucount);
 }
 
-void launch_ex_fill(const int32_t *ptr, int32_t n, int32_t ncl, const uint32_t *merged, const int32_t *ex_ptr,
-                    uint32_t *ex_w, hipStream_t s)
+void launch_ex_fill(const int32_t *ptr, const int32_t *cnt, int32_t n, int32_t ncl, const uint32_t *merged,
+                    const int32_t *ex_ptr, uint32_t *ex_w, hipStream_t s)
 {
     if (ncl > 0)
-        k_ex_fill<<<(ncl + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, n, ncl, merged, ex_ptr, ex_w);
+        k_ex_fill<<<(ncl + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, cnt, n, ncl, merged, ex_ptr, ex_w);
 }
 
-void launch_edge_keep(const int32_t *ptr, int32_t n, const int32_t *ej, const float *ek, const float *el,
-                      const uint8_t *rigid, const int32_t *fptr, int32_t *cnt, int32_t *fej, float *fek, float *fel,
-                      hipStream_t s)
+void launch_edge_keep(const int32_t *ptr, const int32_t *cnt, int32_t n, const uint2 *rows, const float *rk,
+                      const uint8_t *rigid, int32_t *kept, const int32_t *kptr, uint2 *krows, float *kk, hipStream_t s)
 {
     if (n > 0)
-        k_edge_keep<<<nblk(n), BLOCK, 0, s>>>(ptr, n, ej, ek, el, rigid, fptr, cnt, fej, fek, fel);
+        k_edge_keep<<<(n + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, cnt, n, rows, rk, rigid, kept, kptr, krows,
+                                                                        kk);
 }
 
 void launch_rows_expand(const int32_t *offs, int32_t n, uint32_t *ida, hipStream_t s)

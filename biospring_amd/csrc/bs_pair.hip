@@ -7,7 +7,7 @@
 // per i-cluster with lanes laid out as 8 i x 8 entries, so that every load of
 // a j's data serves 8 lanes, and accumulate forces on i only (each pair is
 // visited from both sides): no atomics, bitwise reproducible.
-#include "bs_device.hpp"
+#include "bs_pairterm.hpp"
 
 #include <cmath>
 
@@ -16,8 +16,6 @@ namespace bs
 
 namespace
 {
-
-constexpr int WAVES = BLOCK / 64;
 
 __device__ inline uint32_t bonded_mask(const int32_t *ex_ptr, const uint32_t *ex_w, int32_t ci, int32_t j)
 {
@@ -339,6 +337,14 @@ __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListArgs a)
         for (int32_t slot = count + lane; slot < pad; slot += 64)
             a.cl[(size_t)ci * a.cap + slot] = 0u;
     }
+    if (a.plan)
+    { // the wave reads back what its own lanes stored (one CU)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        queue_plan(a.cl + (size_t)ci * a.cap, min(count, a.cap), pair_waves(a.ncl),
+                   reinterpret_cast<QPlan *>(a.plan + (size_t)ci * a.nst * QPLAN_BYTES));
+    }
     if (lane == 0)
     {
         a.cln[ci] = count < a.cap ? count : a.cap;
@@ -347,187 +353,6 @@ __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListArgs a)
         if (count > 0)
             atomicMax(&a.status[3], count);
     }
-}
-
-// ---------------------------------------------------------------------------
-// One pair from i's side.  Energies are weighted 1/2 for a dynamic partner
-// and 1 for a static one (Particle.cpp:231-249).  Formulas: energy/steric.hpp,
-// electrostatic.hpp, hydrophobic.hpp; per-bead sqrt(r), sqrt(eps) for the
-// Lorentz-Berthelot / Good-Hope modes (CombinationRules.hpp:18-31).  The
-// force is accumulated in FP64 (same rate as FP32 on CDNA4), which keeps
-// small net forces accurate when many pair terms cancel.
-//
-// Branch-free: every lane evaluates the terms with a safe distance and the
-// results are selected by the pair's predicates.  Across a wave the pairs are
-// half inside the cutoff at best, so branching would not skip work; it only
-// costs exec-mask bookkeeping and keeps loads from being issued early.  The
-// exact two-stage test runs for pairs in the guard band around rc^2 only.
-//
-// The kernel is bound by VALU issue, so the per-pair instruction count is
-// what is minimised: the force prefactors carry C_spring, the term scales
-// and i's own factor (PairI, formed once per lane); the pair predicates gate
-// FP32 values (one select each) instead of FP64 results; a charge that is
-// zero, or a pair gated off, zeroes the Coulomb term through q_j.
-// ---------------------------------------------------------------------------
-struct PairI
-{
-    float ks;  // steric force: C_spring x scale x {12 eps_i', 24 eps_i', eps_i} (Amber, Lewitt, Zacharias), C_spring x scale (linear)
-    float kh;  // hydrophobic force: scale x C_spring x h_i
-    double qe; // Coulomb energy: q_i ke
-    double qf; // Coulomb force: q_i kf, doubled for eps(r) = eps r
-};
-
-// An FP32 value kept as computed: a select of it stays one FP32 select
-// instead of being sunk past a later FP64 conversion (two selects).
-__device__ inline float keep(float x)
-{
-    asm("" : "+v"(x));
-    return x;
-}
-
-template <int SMODE, int EMODE>
-__device__ inline PairI pair_i(float4 pi, float4 ri, const PairArgs &a)
-{
-    PairI c;
-    const float cs = (float)a.k.c_spring;
-    const float m = SMODE == 1 ? 12.0f : SMODE == 2 ? 24.0f : 1.0f;
-    c.ks = SMODE == 0 ? cs * a.steric_scale : m * cs * a.steric_scale * ri.y;
-    c.kh = a.hydro_scale * cs * ri.z;
-    c.qe = (double)pi.w * a.ke;
-    c.qf = (double)pi.w * a.kf * (EMODE == 2 ? 2.0 : 1.0);
-    return c;
-}
-
-template <int SMODE, int EMODE, int HYDRO, bool ENERGY>
-__device__ inline void interact(bool masked, float4 pi, float4 ri, float4 pj, float4 rj, const PairArgs &a,
-                                const PairI &c, double &fx, double &fy, double &fz, double &es, double &ee,
-                                double &eh)
-{
-    const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-    const float r2 = dx * dx + dy * dy + dz * dz;
-    const bool lo = r2 < a.rc2lo;
-    bool on = masked && lo;
-    if (masked && !lo && r2 < a.rc2hi) // rare: decide exactly
-        on = exact_two_stage(pi, pj, a.rc);
-    const bool pos2 = r2 > 0.0f;
-    const float r2s = pos2 ? r2 : 1.0f;
-    // the distance itself is needed by the vacuum Coulomb term, the linear
-    // steric wall and the hydrophobic term; the others need 1/r^2 only
-    constexpr bool NEED_D = EMODE == 1 || SMODE == 0 || HYDRO != 0;
-    float inv = 0.0f, inv2;
-    double invd = 0.0, i2d = 0.0;
-    if (EMODE > 0)
-    {
-        // 1/d or 1/r^2 to ~1e-13: the FP32 seed (its input kept at or above
-        // the smallest normal float, so it is finite) and one FP64 Newton
-        // step on the exact r^2 of the float components.  The FP32 values of
-        // the other terms are its rounding.  r2 >= 0, so the larger bit
-        // pattern is the larger value (one integer max).
-        const double xd = dx, yd = dy, zd = dz;
-        const double r2d = fma(xd, xd, fma(yd, yd, zd * zd));
-        const float seed = __int_as_float(max(__float_as_int(r2), 0x00800000));
-        if (NEED_D)
-        {
-            const double y = (double)__builtin_amdgcn_rsqf(seed);
-            invd = y * fma(-0.5 * r2d, y * y, 1.5);
-            i2d = invd * invd;
-            inv = (float)invd;
-            inv2 = inv * inv;
-        }
-        else
-        {
-            const double y = (double)__builtin_amdgcn_rcpf(seed);
-            i2d = y * fma(-r2d, y, 2.0);
-            inv2 = (float)i2d;
-        }
-    }
-    else
-    {
-        inv = __builtin_amdgcn_rsqf(r2s);
-        inv = inv * (1.5f - 0.5f * r2s * inv * inv);
-        inv2 = inv * inv;
-    }
-    const uint32_t flj = fbits(rj.w);
-    const float wgt = (flj & PF_STATIC) ? 1.0f : 0.5f;
-    float fs = 0.0f; // FP32 terms of the force scalar: force on i = (dx, dy, dz) * (fs + fsd)
-    if (SMODE >= 0)
-    {
-        float en = 0.0f, f = 0.0f;
-        if (SMODE == 0)
-        { // linear: ri + rj from raw radii; a coincident pair has energy, no force
-            const float sr = ri.x + rj.x;
-            const float d = r2s * inv;
-            const float dv = pos2 ? d - sr : -sr;
-            const bool ov = !(dv > 0.0f);
-            en = ov ? 0.5f * dv * dv : 0.0f;
-            f = (on && ov && pos2) ? dv * c.ks * inv : 0.0f; // -|dv| * C / d
-        }
-        else
-        {
-            const float R = ri.x * rj.x;
-            const float s2 = R * R * inv2, s6 = s2 * s2 * s2;
-            float g, e0 = 0.0f;
-            if (SMODE == 1)
-            { // Amber 12-6: F = 12 eps (s6 - s12) / r^2, E = eps (s12 - 2 s6)
-                g = fmaf(-s6, s6, s6);
-                if (ENERGY)
-                    e0 = ri.y * rj.y * (s6 * s6 - 2.0f * s6);
-            }
-            else if (SMODE == 2)
-            { // Lewitt 8-6: F = 24 eps (s6 - s8) / r^2, E = eps (3 s8 - 4 s6)
-                const float s8 = s6 * s2;
-                g = s6 - s8;
-                if (ENERGY)
-                    e0 = ri.y * rj.y * (3.0f * s8 - 4.0f * s6);
-            }
-            else
-            { // Zacharias 8-6: raw r, eps, product rules
-                const float s8 = s6 * s2;
-                g = 6.0f * s6 - 8.0f * s8;
-                if (ENERGY)
-                    e0 = ri.y * rj.y * (s8 - s6);
-            }
-            const bool far = r2 >= 0.01f; // 0.1 A floor (steric.hpp:62)
-            en = far ? e0 : 0.0f;
-            f = (on && far) ? c.ks * rj.y * g * inv2 : 0.0f;
-        }
-        if (ENERGY)
-            es += on ? (double)(wgt * a.steric_scale * en) : 0.0;
-        fs += f;
-    }
-    double fsd = 0.0;
-    if (EMODE > 0)
-    {
-        // Coulomb dominates the non-bonded force: its scalar is formed in FP64
-        const double qj = (double)keep((on && r2 >= 1.0e-6f) ? pj.w : 0.0f);
-        if (EMODE == 1)
-        {
-            if (ENERGY)
-                ee += (double)wgt * c.qe * qj * invd;
-            fsd = -(c.qf * qj) * (i2d * invd);
-        }
-        else
-        { // eps(r) = eps * r
-            if (ENERGY)
-                ee += (double)wgt * c.qe * qj * i2d;
-            fsd = -(c.qf * qj) * (i2d * i2d);
-        }
-    }
-    if (HYDRO)
-    {
-        // h_i h_j vanishes unless both are hydrophobic
-        const float e = __expf(-(r2s * inv));
-        if (ENERGY)
-        {
-            const float hh = pos2 ? ri.z * rj.z * e : 0.0f;
-            eh += on ? (double)(wgt * a.hydro_scale) * (-(double)hh * 6.02214169E23 * 1.0E-3) : 0.0;
-        }
-        fs += (on && pos2) ? c.kh * rj.z * e * inv : 0.0f;
-    }
-    const double s = EMODE > 0 ? fsd + (double)keep(fs) : (double)fs;
-    fx = fma((double)dx, s, fx);
-    fy = fma((double)dy, s, fy);
-    fz = fma((double)dz, s, fz);
 }
 
 // Pair forces of one i-cluster per wave.  A block is 16 list words, two per
@@ -680,8 +505,8 @@ __device__ inline void adj_pair_term(bool masked, float4 pi, float4 ri, uint32_t
     }
     else if (SMODE > 0)
     {
-        const float eij = ri.y * rj.y, R = ri.x * rj.x;
-        const float s2 = R * R * ir2, s6 = s2 * s2 * s2, s8 = s6 * s2;
+        const float eij = ri.y * rj.y;
+        const float s2 = ri.x * rj.x * ir2, s6 = s2 * s2 * s2, s8 = s6 * s2;
         float f0, d0;
         if (SMODE == 1)
         {
@@ -899,123 +724,45 @@ void launch_list_build(const ListArgs &a, hipStream_t s)
         k_cluster_list<<<cluster_blocks(a.ncl), BLOCK, 0, s>>>(a);
 }
 
-// ---------------------------------------------------------------------------
-// Queue layout (BS_PAIR_QUEUES).  A wave takes its cluster's list one chunk
-// (at most QCHUNK = 128 words) at a time.  Each word's j data is loaded
-// once (one lane per word) into LDS, and each of the 8 cluster particles gets
-// an LDS queue of the chunk's words it sees (one ballot per particle and 64
-// words).  The 8 lanes of a particle then drain its queue, 8 entries per
-// round, so the lanes evaluate listed pairs instead of idling on entries
-// their particle does not see (an entry is seen by about half of a
-// cluster's particles when springs empty the inner shell).  A chunk takes as
-// many rounds as its fullest queue.  Each
-// lane sums a fixed subset of its particle's entries in a fixed order and
-// the 8 partial sums are combined as in k_pair: deterministic.  The next
-// chunk's words and j data are loaded while the current one is evaluated.
-// ---------------------------------------------------------------------------
-__device__ inline int32_t lanes_below(uint64_t b)
+// Pair forces in the queue layout: a block of W waves per cluster
+// (queue_walk), whose partial sums are added in wave order.  Small blocks: a
+// slot is free as soon as its cluster is done.
+template <bool WIDE, bool ENERGY> struct PairLds
 {
-    return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u));
-}
+    QueueLds<WIDE> q;
+    double sum[CLUSTER][ENERGY ? 6 : 3];
+};
 
 template <int SMODE, int EMODE, int HYDRO, bool ENERGY>
 __global__ void __launch_bounds__(BLOCK) k_pair_q(PairArgs a)
 {
     if (a.status && halted(a.status))
         return;
-    __shared__ float4 qpos[WAVES][QCHUNK], qprm[WAVES][QCHUNK];
-    __shared__ uint8_t qidx[WAVES][CLUSTER][QCHUNK];
-    const int wv = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int32_t ci = __builtin_amdgcn_readfirstlane(blockIdx.x * WAVES + wv);
-    if (ci >= a.ncl)
-        return; // whole wave
-    const int32_t il = lane & 7, sl = lane >> 3;
+    extern __shared__ __align__(16) char lds[];
+    auto *part = reinterpret_cast<PairLds<ENERGY || HYDRO, ENERGY> *>(lds); // one per wave
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int W = blockDim.x >> 6;
+    const int32_t ci = blockIdx.x;
+    const int il = lane & 7;
     const int32_t i = ci * CLUSTER + il;
-    const bool iv = i < a.n;
-    const float4 pi = iv ? a.pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 ri = iv ? a.jprm[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const PairI c = pair_i<SMODE, EMODE>(pi, ri, a);
-    double es = 0.0, ee = 0.0, eh = 0.0;
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    const Chunks d = chunks_of(__builtin_amdgcn_readfirstlane(a.cln[ci]));
-    const uint32_t *L = a.cl + (size_t)ci * a.cap;
-    // chunk 0 in flight (a chunk holds at least one word)
-    int32_t cs = 0, cn = d.q + (d.r > 0 ? 1 : 0);
-    uint32_t w0 = 0u, w1 = 0u;
-    if (d.nch > 0)
+    PairSums s;
+    queue_walk<SMODE, EMODE, HYDRO, ENERGY>(a, ci, w, W, part[w].q, s);
+    s.reduce<ENERGY>();
+    if (W > 1)
     {
-        w0 = lane < cn ? L[lane] : 0u;
-        w1 = 64 + lane < cn ? L[64 + lane] : 0u;
+        if (lane < CLUSTER)
+            s.store<ENERGY>(part[w].sum[il]);
+        __syncthreads();
+        if (w != 0)
+            return;
+        for (int v = 1; v < W; ++v)
+            s.add<ENERGY>(part[v].sum[il]);
     }
-    float4 p0 = a.pos[w0 & CL_JMASK], r0 = a.jprm[w0 & CL_JMASK];
-    float4 p1 = a.pos[w1 & CL_JMASK], r1 = a.jprm[w1 & CL_JMASK];
-    for (int32_t ch = 0; ch < d.nch; ++ch)
-    {
-        qpos[wv][lane] = p0;
-        qprm[wv][lane] = r0;
-        qpos[wv][64 + lane] = p1;
-        qprm[wv][64 + lane] = r1;
-        int32_t cnt[CLUSTER];
-#pragma unroll
-        for (int k = 0; k < CLUSTER; ++k)
-        {
-            const bool s0 = (w0 >> (24 + k)) & 1u, s1 = (w1 >> (24 + k)) & 1u;
-            const uint64_t b0 = __ballot(s0), b1 = __ballot(s1);
-            const int32_t n0 = __popcll(b0);
-            if (s0)
-                qidx[wv][k][lanes_below(b0)] = (uint8_t)lane;
-            if (s1)
-                qidx[wv][k][n0 + lanes_below(b1)] = (uint8_t)(64 + lane);
-            cnt[k] = n0 + __popcll(b1);
-        }
-        // the next chunk in flight while this one is evaluated
-        if (ch + 1 < d.nch)
-        {
-            cs += cn;
-            cn = d.q + (ch + 1 < d.r ? 1 : 0);
-            w0 = lane < cn ? L[cs + lane] : 0u;
-            w1 = 64 + lane < cn ? L[cs + 64 + lane] : 0u;
-            p0 = a.pos[w0 & CL_JMASK];
-            r0 = a.jprm[w0 & CL_JMASK];
-            p1 = a.pos[w1 & CL_JMASK];
-            r1 = a.jprm[w1 & CL_JMASK];
-        }
-        wave_lds_sync();
-        int32_t mine = cnt[0], most = cnt[0];
-#pragma unroll
-        for (int k = 1; k < CLUSTER; ++k)
-        {
-            mine = il == k ? cnt[k] : mine;
-            most = max(most, cnt[k]);
-        }
-        for (int32_t e0 = 0; e0 < most; e0 += 8) // wave-uniform rounds
-        {
-            const int32_t e = e0 + sl;
-            const bool valid = e < mine;
-            const int32_t src = valid ? (int32_t)qidx[wv][il][e] : 0;
-            interact<SMODE, EMODE, HYDRO, ENERGY>(valid, pi, ri, qpos[wv][src], qprm[wv][src], a, c, fx, fy, fz, es,
-                                                  ee, eh);
-        }
-        wave_lds_sync();
-    }
-    for (int off = 8; off < 64; off <<= 1)
-    {
-        fx += __shfl_xor(fx, off, 64);
-        fy += __shfl_xor(fy, off, 64);
-        fz += __shfl_xor(fz, off, 64);
-        if (ENERGY)
-        {
-            es += __shfl_xor(es, off, 64);
-            ee += __shfl_xor(ee, off, 64);
-            eh += __shfl_xor(eh, off, 64);
-        }
-    }
-    if (sl != 0 || !iv)
+    if (lane >= CLUSTER || i >= a.n)
         return;
     if (ENERGY)
     {
-        double4 en = make_double4(es, ee, eh, 0.0);
+        double4 en = make_double4(s.es, s.ee, s.eh, 0.0);
         if (a.accumulate)
         {
             const double4 o = a.epp[i];
@@ -1025,7 +772,7 @@ __global__ void __launch_bounds__(BLOCK) k_pair_q(PairArgs a)
         }
         a.epp[i] = en;
     }
-    double4 f = make_double4(fx, fy, fz, 0.0);
+    double4 f = make_double4(s.fx, s.fy, s.fz, 0.0);
     if (a.accumulate)
     {
         const double4 o = a.fnb[i];
@@ -1171,12 +918,13 @@ __global__ void __launch_bounds__(BLOCK) k_pair_rows(PairArgs a)
 
 template <int S, int E, int H> static void pair3(const PairArgs &a, int32_t nb, hipStream_t s)
 {
-    if (a.queues)
+    if (a.plan)
     {
+        const int32_t W = pair_waves(a.ncl);
         if (a.energy)
-            k_pair_q<S, E, H, true><<<nb, BLOCK, 0, s>>>(a);
+            k_pair_q<S, E, H, true><<<a.ncl, 64 * W, W * sizeof(PairLds<true, true>), s>>>(a);
         else
-            k_pair_q<S, E, H, false><<<nb, BLOCK, 0, s>>>(a);
+            k_pair_q<S, E, H, false><<<a.ncl, 64 * W, W * sizeof(PairLds<H != 0, false>), s>>>(a);
         return;
     }
     if (a.rows)

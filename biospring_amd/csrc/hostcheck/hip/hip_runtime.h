@@ -18,6 +18,16 @@ struct float4
 {
     float x, y, z, w;
 };
+struct uint2
+{
+    unsigned x, y;
+};
+struct int2
+{
+    int x, y;
+};
+inline int2 make_int2(int x, int y) { return int2{x, y}; }
+inline uint2 make_uint2(unsigned x, unsigned y) { return uint2{x, y}; }
 inline float4 make_float4(float x, float y, float z, float w) { return float4{x, y, z, w}; }
 struct double4
 {

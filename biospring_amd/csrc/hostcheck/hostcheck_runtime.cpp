@@ -475,6 +475,12 @@ void launch_list_build(const ListArgs &a, hipStream_t)
     if (a.cap > 0)
     {
         need(a.cl, sizeof(uint32_t) * (size_t)a.ncl * a.cap, "list: cl");
+        if (a.plan)
+        {
+            if (a.nst * 64 < a.cap)
+                hc_fail("list: plan shorter than the list");
+            need(a.plan, (size_t)a.ncl * a.nst * QPLAN_BYTES, "list: plan");
+        }
     }
     if ((int64_t)a.ncl * CLUSTER < a.n || (int64_t)(a.ncl - 1) * CLUSTER >= a.n)
         hc_fail("list: bad cluster count");
@@ -624,6 +630,8 @@ void launch_pair(const PairArgs &a, int32_t, int32_t, int32_t nb, hipStream_t)
     need(a.jprm, sizeof(float4) * a.n, "pair: jprm");
     need(a.cln, sizeof(int32_t) * a.ncl, "pair: cln");
     need(a.cl, sizeof(uint32_t) * (size_t)a.ncl * a.cap, "pair: cl");
+    if (a.plan)
+        need(a.plan, (size_t)a.ncl * a.nst * QPLAN_BYTES, "pair: plan");
     need(a.fnb, sizeof(double4) * a.n, "pair: fnb");
     if (a.energy)
         need(a.epp, sizeof(double4) * a.n, "pair: epp");
@@ -656,6 +664,33 @@ void launch_pair(const PairArgs &a, int32_t, int32_t, int32_t nb, hipStream_t)
             if (a.energy)
                 a.epp[i] = make_double4(0, 0, 0, 0);
         }
+}
+
+// The force rows as EdgeRow reads them: partners in range, the last edge of
+// every row a null edge.
+static void check_rows(const int32_t *ptr, const uint2 *rows, const float *rk, int32_t n, const char *who)
+{
+    const size_t ne = (size_t)ptr[n] * EDGE_PAD;
+    need(rows, sizeof(uint2) * ne, who);
+    if (rk)
+        need(rk, sizeof(float) * ne, who);
+    for (size_t e = 0; e < ne; ++e)
+        if ((int32_t)(rows[e].x & 0x7fffffffu) >= n)
+            hc_fail("edge index out of range");
+    for (int32_t i = 0; i < n; ++i)
+    {
+        const uint2 last = rows[(size_t)ptr[i + 1] * EDGE_PAD - 1];
+        if (ptr[i + 1] <= ptr[i] || last.x != (uint32_t)i || last.y != 0u)
+            hc_fail("row without a null edge at its end");
+    }
+}
+
+void launch_step_kernel(const PairArgs &p, const SpringArgs &a, int32_t em, int32_t h, hipStream_t s)
+{
+    if (!p.plan || !a.integrate || a.probe.state)
+        hc_fail("step kernel: queue layout, integration and no probe only");
+    launch_pair(p, em, h, (p.ncl + BLOCK / 64 - 1) / (BLOCK / 64), s);
+    launch_spring(a, 16, (int32_t)(((int64_t)a.n * 16 + BLOCK - 1) / BLOCK), s);
 }
 
 void launch_spring(const SpringArgs &a, int32_t group, int32_t nb, hipStream_t)
@@ -700,17 +735,7 @@ void launch_spring(const SpringArgs &a, int32_t group, int32_t nb, hipStream_t)
         need(a.probe.state, sizeof(ProbeDev), "spring: probe state");
         need(a.probe.part, sizeof(double) * 8 * nb, "spring: probe block sums");
     }
-    const int32_t ne = a.sp_ptr[n];
-    if (ne > 0)
-    {
-        need(a.sp_j, sizeof(int32_t) * ne, "spring: sp_j");
-        if (a.sp_k)
-            need(a.sp_k, sizeof(float) * ne, "spring: sp_k");
-        need(a.sp_l0, sizeof(float) * ne, "spring: sp_l0");
-    }
-    for (int32_t e = 0; e < ne; ++e)
-        if ((a.sp_j[e] & 0x7fffffff) >= n)
-            hc_fail("spring: edge index out of range");
+    check_rows(a.sp_ptr, a.sp_e, a.sp_k, n, "spring");
     need(a.status, 32, "spring: status");
     if (a.integrate && halted(a.status))
     { // a stopped call carries every position over
@@ -778,14 +803,7 @@ void launch_adj_spring(const AdjSpringArgs &a, int32_t group, int32_t nb, hipStr
         need(a.hwp, sizeof(double4) * n, "adj_spring: hwp");
     if ((int64_t)nb * BLOCK < (int64_t)n * group)
         hc_fail("adj_spring: grid too small");
-    const int32_t ne = a.sp_ptr[n];
-    if (ne > 0)
-    {
-        need(a.sp_j, sizeof(int32_t) * ne, "adj_spring: sp_j");
-        if (a.sp_k)
-            need(a.sp_k, sizeof(float) * ne, "adj_spring: sp_k");
-        need(a.sp_l0, sizeof(float) * ne, "adj_spring: sp_l0");
-    }
+    check_rows(a.sp_ptr, a.sp_e, a.sp_k, n, "adj_spring");
     if (a.dk)
     {
         need(a.slot_ptr, sizeof(int32_t) * (n + 1), "adj_spring: slot_ptr");
@@ -797,11 +815,9 @@ void launch_adj_spring(const AdjSpringArgs &a, int32_t group, int32_t nb, hipStr
         const bool dyn = !(fbits(a.jprm[i].w) & PF_STATIC);
         int32_t slot = a.dk ? a.slot_ptr[i] : 0;
         if (dyn && a.spring_enable)
-            for (int32_t e = a.sp_ptr[i]; e < a.sp_ptr[i + 1]; ++e)
+            for (size_t e = (size_t)a.sp_ptr[i] * EDGE_PAD; e < (size_t)a.sp_ptr[i + 1] * EDGE_PAD; ++e)
             {
-                if ((a.sp_j[e] & 0x7fffffff) >= n)
-                    hc_fail("adj_spring: edge index out of range");
-                if (a.dk && (a.sp_j[e] < 0 || a.sp_j[e] > i))
+                if (a.dk && ((int32_t)a.sp_e[e].x < 0 || (int32_t)a.sp_e[e].x > i))
                 {
                     if (slot >= a.slot_ptr[i + 1])
                         hc_fail("adj_spring: more owned edges than slots in a row");
@@ -920,170 +936,171 @@ void launch_unperm_f64(const double *in, const int32_t *perm, int32_t n, double 
 // Springs from a cutoff, computed like the kernel (same grid walk and test).
 // Spring CSR, exclusions and construction expansion: the device kernels'
 // results computed serially, with every access checked.
-void launch_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t *cnt,
-                       hipStream_t)
+void launch_edge_units(const int32_t *cnt, int32_t n, int32_t *units, hipStream_t)
+{
+    need(cnt, sizeof(int32_t) * n, "edge_units: cnt");
+    need(units, sizeof(int32_t) * n, "edge_units: units");
+    for (int32_t i = 0; i < n; ++i)
+        units[i] = (cnt[i] + EDGE_PAD) / EDGE_PAD;
+}
+
+void launch_edge_count(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, int32_t n, int32_t *cnt,
+                       int2 *slot, int32_t *units, hipStream_t s)
 {
     need(sa, sizeof(uint32_t) * m, "edge_count: sa");
     need(sb, sizeof(uint32_t) * m, "edge_count: sb");
-    for (int64_t s = 0; s < m; ++s)
-        for (uint32_t id : {sa[s], sb[s]})
-        {
-            need(iperm + id, 4, "edge_count: iperm");
-            need(cnt + iperm[id], 4, "edge_count: cnt");
-            ++cnt[iperm[id]];
-        }
-}
-
-void launch_edge_fill(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const int32_t *ptr,
-                      int32_t *cursor, uint64_t *key, hipStream_t)
-{
-    need(sa, sizeof(uint32_t) * m, "edge_fill: sa");
-    need(sb, sizeof(uint32_t) * m, "edge_fill: sb");
-    for (int64_t s = 0; s < m; ++s)
+    need(slot, sizeof(int2) * m, "edge_count: slot");
+    need(cnt, sizeof(int32_t) * n, "edge_count: cnt");
+    for (int64_t t = 0; t < m; ++t)
     {
-        const int32_t a = iperm[sa[s]], b = iperm[sb[s]];
-        for (int side = 0; side < 2; ++side)
-        {
-            const int32_t r = side ? b : a, o = side ? a : b;
-            need(ptr + r, 8, "edge_fill: ptr");
-            need(cursor + r, 4, "edge_fill: cursor");
-            const int32_t slot = ptr[r] + cursor[r]++;
-            if (slot >= ptr[r + 1])
-                hc_fail("edge_fill: row overflow");
-            need(key + slot, 8, "edge_fill: key");
-            key[slot] = (uint64_t)(uint32_t)o << 32 | ((uint32_t)s << 1 | (uint32_t)side);
-        }
+        need(iperm + sa[t], 4, "edge_count: iperm");
+        need(iperm + sb[t], 4, "edge_count: iperm");
+        slot[t].x = cnt[iperm[sa[t]]]++;
+        slot[t].y = cnt[iperm[sb[t]]]++;
     }
+    launch_edge_units(cnt, n, units, s);
 }
 
-void launch_edge_sort(const int32_t *ptr, int32_t n, const uint64_t *key, const float4 *jprm, const float *sl,
-                      const float *sk, int32_t *ej, float *ek, float *el, hipStream_t)
+void launch_edge_sort(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const int32_t *ptr,
+                      const int32_t *cnt, int32_t n, const int2 *slot, uint2 *key, const float4 *jprm, const float *sl,
+                      const float *sk, uint2 *rows, float *rk, hipStream_t)
 {
     need(ptr, sizeof(int32_t) * (n + 1), "edge_sort: ptr");
-    const int32_t E = n > 0 ? ptr[n] : 0;
-    need(key, sizeof(uint64_t) * E, "edge_sort: key");
-    need(ej, sizeof(int32_t) * E, "edge_sort: ej");
-    need(ek, sizeof(float) * E, "edge_sort: ek");
-    need(el, sizeof(float) * E, "edge_sort: el");
-    need(jprm, sizeof(float4) * n, "edge_sort: jprm");
+    const size_t E = (size_t)ptr[n] * EDGE_PAD;
+    need(key, sizeof(uint2) * E, "edge_sort: key");
+    need(rows, sizeof(uint2) * E, "edge_sort: rows");
+    need(rk, sizeof(float) * E, "edge_sort: rk");
+    need(sl, sizeof(float) * m, "edge_sort: rest lengths");
+    need(sk, sizeof(float) * m, "edge_sort: stiffnesses");
+    for (int64_t t = 0; t < m; ++t)
+        for (int side = 0; side < 2; ++side)
+        {
+            const int32_t r = iperm[side ? sb[t] : sa[t]], o = iperm[side ? sa[t] : sb[t]];
+            const int32_t at = side ? slot[t].y : slot[t].x;
+            if (at < 0 || at >= cnt[r] || cnt[r] >= (ptr[r + 1] - ptr[r]) * EDGE_PAD)
+                hc_fail("edge_sort: row overflow");
+            key[(size_t)ptr[r] * EDGE_PAD + at] = make_uint2((uint32_t)o, (uint32_t)t);
+        }
     for (int32_t i = 0; i < n; ++i)
     {
-        std::vector<uint64_t> row(key + ptr[i], key + ptr[i + 1]);
-        std::sort(row.begin(), row.end());
+        const size_t b = (size_t)ptr[i] * EDGE_PAD;
+        std::vector<uint2> row(key + b, key + b + cnt[i]);
+        std::sort(row.begin(), row.end(), [](const uint2 &x, const uint2 &y) { return x.x < y.x; });
         for (size_t t = 0; t < row.size(); ++t)
         {
-            if (t > 0 && row[t] == row[t - 1])
-                hc_fail("edge_sort: repeated key");
-            const int32_t j = (int32_t)(row[t] >> 32);
-            const uint32_t s = (uint32_t)row[t] >> 1;
-            if (j < 0 || j >= n)
+            if (t > 0 && row[t].x == row[t - 1].x)
+                hc_fail("edge_sort: repeated partner");
+            if (row[t].x >= (uint32_t)n)
                 hc_fail("edge_sort: partner out of range");
-            need(sl + s, 4, "edge_sort: rest length");
-            need(sk + s, 4, "edge_sort: stiffness");
-            const int32_t o = ptr[i] + (int32_t)t;
-            ej[o] = (fbits(jprm[j].w) & PF_STATIC) ? (int32_t)((uint32_t)j | 0x80000000u) : j;
-            ek[o] = sk[s];
-            el[o] = sl[s];
+            const bool st = (fbits(jprm[row[t].x].w) & PF_STATIC) != 0;
+            rows[b + t] = make_uint2(st ? row[t].x | 0x80000000u : row[t].x, fbits(sl[row[t].y]));
+            rk[b + t] = sk[row[t].y];
+        }
+        for (size_t t = row.size(); t < (size_t)(ptr[i + 1] - ptr[i]) * EDGE_PAD; ++t)
+        {
+            rows[b + t] = make_uint2((uint32_t)i, 0u);
+            rk[b + t] = 0.0f;
         }
     }
 }
 
-static std::vector<uint32_t> hc_cluster_words(const int32_t *ptr, const int32_t *ej, int32_t n, int32_t c)
-{
-    std::vector<uint32_t> w;
-    for (int32_t k = 0; k < CLUSTER && c * CLUSTER + k < n; ++k)
-    {
-        const int32_t i = c * CLUSTER + k;
-        for (int32_t t = ptr[i]; t < ptr[i + 1]; ++t)
-            w.push_back((uint32_t)(ej[t] & 0x7fffffff) << 8 | (1u << k));
-    }
-    std::sort(w.begin(), w.end());
-    return w;
-}
-
-void launch_ex_merge(const int32_t *ptr, const int32_t *ej, int32_t n, int32_t ncl, uint32_t *merged,
-                     int32_t *ucount, hipStream_t)
+void launch_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n, int32_t ncl,
+                     uint32_t *merged, int32_t *ucount, hipStream_t)
 {
     need(ptr, sizeof(int32_t) * (n + 1), "ex_merge: ptr");
-    need(ej, sizeof(int32_t) * (n > 0 ? ptr[n] : 0), "ex_merge: ej");
-    need(merged, sizeof(uint32_t) * (n > 0 ? ptr[n] : 0), "ex_merge: merged");
+    need(rows, sizeof(uint2) * EDGE_PAD * (size_t)ptr[n], "ex_merge: rows");
+    need(merged, sizeof(uint32_t) * EDGE_PAD * (size_t)ptr[n], "ex_merge: merged");
     need(ucount, sizeof(int32_t) * ncl, "ex_merge: ucount");
     if (ncl != (n + CLUSTER - 1) / CLUSTER)
         hc_fail("ex_merge: cluster count");
     for (int32_t c = 0; c < ncl; ++c)
     {
-        const std::vector<uint32_t> w = hc_cluster_words(ptr, ej, n, c);
-        const int32_t base = ptr[c * CLUSTER];
+        std::vector<uint32_t> w;
+        for (int32_t k = 0; k < CLUSTER && c * CLUSTER + k < n; ++k)
+        {
+            const int32_t i = c * CLUSTER + k;
+            for (int32_t t = 0; t < cnt[i]; ++t)
+                w.push_back((rows[(size_t)ptr[i] * EDGE_PAD + t].x & 0x7fffffffu) << 8 | (1u << k));
+        }
+        std::sort(w.begin(), w.end());
+        const size_t base = (size_t)ptr[c * CLUSTER] * EDGE_PAD;
         int32_t u = 0;
         for (size_t t = 0; t < w.size(); ++t)
         {
-            merged[base + (int32_t)t] = w[t];
+            merged[base + t] = w[t];
             u += (t == 0 || (w[t] >> 8) != (w[t - 1] >> 8)) ? 1 : 0;
         }
         ucount[c] = u;
     }
 }
 
-void launch_ex_fill(const int32_t *ptr, int32_t n, int32_t ncl, const uint32_t *merged, const int32_t *ex_ptr,
-                    uint32_t *ex_w, hipStream_t)
+void launch_ex_fill(const int32_t *ptr, const int32_t *cnt, int32_t n, int32_t ncl, const uint32_t *merged,
+                    const int32_t *ex_ptr, uint32_t *ex_w, hipStream_t)
 {
     need(ex_ptr, sizeof(int32_t) * (ncl + 1), "ex_fill: ex_ptr");
     need(ex_w, sizeof(uint32_t) * ex_ptr[ncl], "ex_fill: ex_w");
     for (int32_t c = 0; c < ncl; ++c)
     {
-        const int32_t base = ptr[std::min(c * CLUSTER, n)], end = ptr[std::min(c * CLUSTER + CLUSTER, n)];
-        int32_t o = ex_ptr[c];
-        for (int32_t t = base; t < end; ++t)
+        const uint32_t *mw = merged + (size_t)ptr[c * CLUSTER] * EDGE_PAD;
+        int32_t total = 0, o = ex_ptr[c];
+        for (int32_t k = 0; k < CLUSTER && c * CLUSTER + k < n; ++k)
+            total += cnt[c * CLUSTER + k];
+        for (int32_t t = 0; t < total; ++t)
         {
-            if (t > base && (merged[t] >> 8) == (merged[t - 1] >> 8))
+            if (t > 0 && (mw[t] >> 8) == (mw[t - 1] >> 8))
             {
-                ex_w[o - 1] |= merged[t] & 0xFFu;
+                ex_w[o - 1] |= mw[t] & 0xFFu;
                 continue;
             }
             if (o >= ex_ptr[c + 1])
                 hc_fail("ex_fill: more words than counted");
-            ex_w[o++] = merged[t];
+            ex_w[o++] = mw[t];
         }
         if (o != ex_ptr[c + 1])
             hc_fail("ex_fill: fewer words than counted");
     }
 }
 
-void launch_edge_keep(const int32_t *ptr, int32_t n, const int32_t *ej, const float *ek, const float *el,
-                      const uint8_t *rigid, const int32_t *fptr, int32_t *cnt, int32_t *fej, float *fek, float *fel,
-                      hipStream_t)
+void launch_edge_keep(const int32_t *ptr, const int32_t *cnt, int32_t n, const uint2 *rows, const float *rk,
+                      const uint8_t *rigid, int32_t *kept, const int32_t *kptr, uint2 *krows, float *kk, hipStream_t)
 {
-    need(ptr, sizeof(int32_t) * (n + 1), "edge_keep: ptr");
     need(rigid, (size_t)n, "edge_keep: rigid");
-    if (fptr)
+    if (krows)
     {
-        need(fptr, sizeof(int32_t) * (n + 1), "edge_keep: fptr");
-        need(fej, sizeof(int32_t) * fptr[n], "edge_keep: fej");
-        need(fek, sizeof(float) * fptr[n], "edge_keep: fek");
-        need(fel, sizeof(float) * fptr[n], "edge_keep: fel");
+        need(kptr, sizeof(int32_t) * (n + 1), "edge_keep: kptr");
+        need(krows, sizeof(uint2) * EDGE_PAD * (size_t)kptr[n], "edge_keep: krows");
+        need(kk, sizeof(float) * EDGE_PAD * (size_t)kptr[n], "edge_keep: kk");
     }
     else
-        need(cnt, sizeof(int32_t) * n, "edge_keep: cnt");
+        need(kept, sizeof(int32_t) * n, "edge_keep: kept");
     for (int32_t i = 0; i < n; ++i)
     {
-        int32_t o = fptr ? fptr[i] : 0, c = 0;
-        for (int32_t t = ptr[i]; t < ptr[i + 1]; ++t)
+        int32_t c = 0;
+        const size_t b = (size_t)ptr[i] * EDGE_PAD, o = krows ? (size_t)kptr[i] * EDGE_PAD : 0;
+        for (int32_t t = 0; t < cnt[i]; ++t)
         {
-            if (rigid[i] && rigid[ej[t] & 0x7fffffff])
+            if (rigid[i] && rigid[rows[b + t].x & 0x7fffffffu])
                 continue;
-            if (fptr)
+            if (krows)
             {
-                fej[o] = ej[t];
-                fek[o] = ek[t];
-                fel[o] = el[t];
-                ++o;
+                krows[o + c] = rows[b + t];
+                kk[o + c] = rk[b + t];
             }
             ++c;
         }
-        if (fptr && o != fptr[i + 1])
-            hc_fail("edge_keep: row length differs from its count");
-        if (!fptr)
-            cnt[i] = c;
+        if (!krows)
+        {
+            kept[i] = c;
+            continue;
+        }
+        const int32_t room = (kptr[i + 1] - kptr[i]) * EDGE_PAD;
+        if (c >= room)
+            hc_fail("edge_keep: no room for the null edge");
+        for (; c < room; ++c)
+        {
+            krows[o + c] = make_uint2((uint32_t)i, 0u);
+            kk[o + c] = 0.0f;
+        }
     }
 }
 

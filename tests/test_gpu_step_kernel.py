@@ -1,0 +1,116 @@
+"""The step kernel (queue layout: the last list's pairs, the springs and the
+integrator in one launch) against the separate kernels of the cluster layout,
+and the spring rows it reads, where its parts change: clusters that are not
+full, one stretch of 64 list words and more than the ring holds, the sizes at
+which the number of waves per cluster changes, rows on both sides of the sort's
+register path, several lists, compensated positions, fixed beads.
+
+Both layouts sum the same terms in FP64 in another order (differences of about
+1e-14), round the force once to FP32 and integrate in FP32, so a step may differ
+by one rounding of the force: 6e-8 of the largest velocity change, grown over
+three steps by the springs (a factor below 4); 1e-6 is allowed.
+"""
+import numpy as np
+import pytest
+
+from biospring_amd import _abi, workloads
+from biospring_amd.network import SpringNetwork
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-6
+
+
+def _state(s, params, steps=3):
+    net = SpringNetwork.from_system(s, params)
+    net.run(steps)
+    x, v = net.getState()
+    return x, v, net.getEnergies()
+
+
+def _compare(s, **over):
+    got = []
+    for layout in (_abi.PAIR_QUEUES, _abi.PAIR_CLUSTERS):
+        p = s.params.copy()
+        for k, v in over.items():
+            setattr(p, k, v)
+        p.pair_layout = layout
+        got.append(_state(s, p))
+    (xq, vq, eq), (xc, vc, ec) = got
+    assert np.abs(vq - vc).max() <= TOL * max(np.abs(vc).max(), 1e-12)
+    assert np.abs(xq - xc).max() <= TOL * max(np.abs(xc).max(), 1.0)
+    assert np.allclose(eq, ec, rtol=TOL, atol=TOL * np.abs(ec).max())
+
+
+def _perturbed(config, n, seed):
+    s = workloads.generate(config, seed=seed, n=n)
+    rng = np.random.default_rng(seed)
+    s.x = (s.x + rng.normal(scale=0.02, size=s.x.shape)).astype(np.float32)
+    return s
+
+
+# 16,384 and 40,960 beads are 2,048 and 5,120 clusters
+@pytest.mark.parametrize("n", [9, 63, 1001, 16384, 16385, 40960, 40967])
+def test_sizes(n):
+    print("n", n, flush=True)
+    _compare(_perturbed(1, n, 3))
+
+
+@pytest.mark.parametrize("over", [
+    {"steric_cutoff": 10.0, "dielectric_model": 0, "electrostatic_dielectric": 20.0},
+    {"steric_mode": _abi.STERIC_ZACHARIAS_8_6, "dielectric_model": 0},
+    {"steric_mode": _abi.STERIC_LEWITT_8_6, "compensated_positions": 1},
+    {"steric_mode": _abi.STERIC_LINEAR, "hydrophobicity_enable": 1},
+    {"steric_enable": 0},
+    {"spring_enable": 0, "steric_cutoff": 6.0, "electrostatic_cutoff": 6.0},
+], ids=["two_lists", "zacharias", "lewitt_comp", "linear_hydro", "coulomb_only", "no_springs"])
+def test_terms(over):
+    s = _perturbed(1, 1501, 5)
+    rng = np.random.default_rng(5)
+    s.flags = (rng.random(s.n) < 0.2).astype(np.uint8)
+    if over.get("steric_mode") == _abi.STERIC_ZACHARIAS_8_6:
+        s.radius = np.sqrt(s.radius).astype(np.float32)  # products of radii
+    if over.get("hydrophobicity_enable"):
+        s.hydro = rng.uniform(-1.0, 1.0, s.n).astype(np.float32) * 1e-18
+    _compare(s, **over)
+
+
+def test_distant_beads_have_empty_lists():
+    s = _perturbed(1, 200, 7)
+    s.x[-30:] += np.float32(500.0) * np.repeat(np.arange(1, 11, dtype=np.float32), 3)
+    far = set(range(190, 200))
+    keep = np.array([a not in far and b not in far for a, b in zip(s.id1, s.id2)])
+    s.id1, s.id2, s.l0, s.k = s.id1[keep], s.id2[keep], s.l0[keep], s.k[keep]
+    _compare(s)
+
+
+@pytest.mark.parametrize("spokes", [1, 7, 8, 255, 256, 257, 300])
+def test_row_lengths(spokes):
+    """One hub with `spokes` springs, given in a shuffled order: its force is
+    their sum, and every spoke's the opposite."""
+    rng = np.random.default_rng(spokes)
+    n = spokes + 1
+    x = rng.normal(size=(n, 3)).astype(np.float32) * 5.0
+    x[0] = 0.0
+    order = rng.permutation(spokes) + 1
+    flip = rng.random(spokes) < 0.5
+    a = np.where(flip, order, 0).astype(np.uint32)
+    b = np.where(flip, 0, order).astype(np.uint32)
+    l0 = rng.uniform(1.0, 4.0, spokes).astype(np.float32)
+    k = rng.uniform(0.1, 1.0, spokes).astype(np.float32)
+    p = _abi.default_params()
+    p.spring_enable, p.timestep = 1, 1.0
+    net = SpringNetwork(p)
+    net.setParticles(x.reshape(-1))
+    net.setSprings(a, b, l0, k)
+    f, e = net.computeForces()
+    d = x[order].astype(np.float64)
+    r = np.linalg.norm(d, axis=1)
+    c = 1.0e3 / 6.02214169e23 * 1.0e10 * (1.0e10 / 1.66054e-27 * 1e-30)
+    pull = (k.astype(np.float64) * (r - l0) * c / r)[:, None] * d
+    want = np.zeros((n, 3))
+    want[0] = pull.sum(0)
+    want[order] = -pull
+    # FP64 sums rounded to FP32: half an ulp of each component
+    assert np.abs(f - want).max() <= 1.2e-7 * np.abs(want).max()
+    assert abs(e[_abi.E_SPRING] - (0.5 * k.astype(np.float64) * (r - l0) ** 2).sum()) <= 1e-9 * abs(e[_abi.E_SPRING])
