@@ -35,6 +35,7 @@ struct List
     uint32_t imask = 0, jmask = 0;
     int32_t dims[3] = {1, 1, 1};
     int32_t ncells = 1;
+    int32_t *bstart = nullptr, *bidx = nullptr; // a small system's cells (k_bin): [ncells + 1], [n]
     int32_t cap = 0;          // entries per i-cluster
     uint32_t *cl = nullptr;   // [ncl * cap] j | mask << 24, in search order
     int32_t *cln = nullptr;   // [ncl]
@@ -367,6 +368,8 @@ void free_device(bs_handle *h)
         f(l.cl);
         f(l.cln);
         f(l.plan);
+        f(l.bstart);
+        f(l.bidx);
         f(l.rows);
         f(l.rlen);
     }
@@ -648,6 +651,17 @@ void plan_grid(bs_handle *h, List &l, const std::vector<float4> &shift)
         l.dims[c] = (int32_t)d;
         total *= d;
     }
+    // a small system is binned by one workgroup, its cell counts in LDS
+    while (h->n <= BIN_MAX && total > BIN_CELLS)
+    {
+        const double f = std::cbrt((double)BIN_CELLS / (double)total) * 0.999;
+        total = 1;
+        for (int c = 0; c < 3; ++c)
+        {
+            l.dims[c] = std::max(1, (int)(l.dims[c] * f));
+            total *= l.dims[c];
+        }
+    }
     while (total > (1 << 22))
     { // keep the grid modest for sparse, spread-out systems
         for (int c = 0; c < 3; ++c)
@@ -681,6 +695,45 @@ int ensure_cells(bs_handle *h, int32_t ncells)
 
 const int32_t *gate_of(bs_handle *h, bool gated) { return gated ? h->status : nullptr; }
 
+// The build arguments of list l from the cells at start, idx.
+ListArgs list_args(const bs_handle *h, const List &l, const int32_t *start, const int32_t *idx, const int32_t *gate,
+                   int32_t cap_override)
+{
+    ListArgs a{};
+    a.pos = h->pos[h->cur];
+    a.shift = h->shift;
+    a.jprm = h->jprm;
+    a.cell_start = start;
+    a.cell_idx = idx;
+    a.box = h->box;
+    a.ex_ptr = h->ex_ptr;
+    a.ex_w = h->ex_w;
+    a.cl = l.cl;
+    a.cln = l.cln;
+    a.plan = cap_override < 0 ? l.plan : nullptr;
+    a.nst = l.nst;
+    a.status = h->status;
+    a.n = (int32_t)h->n;
+    a.ncl = h->ncl;
+    a.cap = cap_override >= 0 ? cap_override : l.cap;
+    for (int c = 0; c < 3; ++c)
+        a.dims[c] = l.dims[c];
+    a.cell_edge = 0.5f * l.radius;
+    a.radius = l.radius;
+    a.r2list = (float)((double)l.radius * l.radius * (1.0 + 1e-5));
+    a.i_mask = l.imask;
+    a.j_mask = l.jmask;
+    a.exclude_bonded = h->p.spring_enable ? 1 : 0;
+    a.gate = gate;
+    return a;
+}
+
+void expand_rows(bs_handle *h, const List &l, const int32_t *gate)
+{
+    if (l.rows)
+        launch_rows(l.cl, l.cln, h->ncl, l.cap, l.rows, l.rlen, l.rcap, gate, h->stream);
+}
+
 // Engine cell grid + Verlet list of list l.  gated: skipped on the device
 // unless the rebuild gate (status[0]) is set.
 void build_list(bs_handle *h, List &l, bool gated, int32_t cap_override)
@@ -696,56 +749,74 @@ void build_list(bs_handle *h, List &l, bool gated, int32_t cap_override)
     launch_scan(h->counts, h->cstart, l.ncells, g, s);
     launch_scatter(h->cell_of, n, h->cstart, h->counts, 1, h->ctmp, g, s);
     launch_cell_sort(h->cell_of, n, h->cstart, h->ctmp, nullptr, h->cidx, g, s);
-    ListArgs a{};
-    a.pos = h->pos[h->cur];
-    a.shift = h->shift;
-    a.jprm = h->jprm;
-    a.cell_start = h->cstart;
-    a.cell_idx = h->cidx;
-    a.box = h->box;
-    a.ex_ptr = h->ex_ptr;
-    a.ex_w = h->ex_w;
-    a.cl = l.cl;
-    a.cln = l.cln;
-    a.plan = cap_override < 0 ? l.plan : nullptr;
-    a.nst = l.nst;
-    a.status = h->status;
-    a.n = n;
-    a.ncl = h->ncl;
-    a.cap = cap_override >= 0 ? cap_override : l.cap;
-    for (int c = 0; c < 3; ++c)
-        a.dims[c] = l.dims[c];
-    a.cell_edge = 0.5f * l.radius;
-    a.radius = l.radius;
-    a.r2list = (float)((double)l.radius * l.radius * (1.0 + 1e-5));
-    a.i_mask = l.imask;
-    a.j_mask = l.jmask;
-    a.exclude_bonded = h->p.spring_enable ? 1 : 0;
-    a.gate = g;
-    launch_list_build(a, s);
-    if (l.rows && cap_override < 0)
-        launch_rows(l.cl, l.cln, h->ncl, l.cap, l.rows, l.rlen, l.rcap, g, s);
+    const ListArgs a = list_args(h, l, h->cstart, h->cidx, g, cap_override);
+    launch_list_build(&a, 1, s);
+    if (cap_override < 0)
+        expand_rows(h, l, g);
 }
 
+// Whether one workgroup bins this system (setup gave its lists their cells).
+bool small_bins(const bs_handle *h) { return !h->lists.empty() && h->lists.front().bidx; }
+
 // The gate kernel: with lists, it also writes the box partials of the
-// current positions for the chain's cell binning.
+// current positions for the chain's cell binning, or does the whole binning
+// of a small system.
 void launch_gate(bs_handle *h, int32_t interval, int32_t advance)
 {
     const bool lists = !h->lists.empty();
+    int32_t *log = advance ? h->gate_log : nullptr;
+    if (small_bins(h))
+    {
+        BinArgs a{};
+        a.pos = h->pos[h->cur];
+        a.shift = h->shift;
+        a.jprm = h->jprm;
+        a.xref = h->xref;
+        a.box = h->box;
+        a.status = h->status;
+        a.counters = h->counters;
+        a.log = log;
+        a.n = (int32_t)h->n;
+        a.nlists = (int32_t)h->lists.size();
+        a.interval = interval;
+        a.advance = advance;
+        for (int32_t li = 0; li < a.nlists; ++li)
+        {
+            const List &l = h->lists[(size_t)li];
+            for (int c = 0; c < 3; ++c)
+                a.list[li].dims[c] = l.dims[c];
+            a.list[li].edge = 0.5f * l.radius;
+            a.list[li].mask = l.jmask;
+            a.list[li].start = l.bstart;
+            a.list[li].idx = l.bidx;
+        }
+        launch_bin(a, h->stream);
+        return;
+    }
     launch_prestep(h->status, h->counters, interval, advance, lists ? h->pos[h->cur] : nullptr, h->shift,
-                   (int32_t)h->n, lists ? h->box_part : nullptr, h->box_blocks, advance ? h->gate_log : nullptr,
-                   h->stream);
+                   (int32_t)h->n, lists ? h->box_part : nullptr, h->box_blocks, log, h->stream);
 }
 
-// The gated list rebuild.  prepped: the gate (and the box partials) were
-// just set by a step's prestep; otherwise they are set here from the drift
-// flag alone.
-void rebuild_chain(bs_handle *h, bool gated, bool prepped = false)
+// The gated list rebuild.  prepped: the gate (and the box partials or a small
+// system's cells) were just set by a step's prestep; otherwise they are set
+// here from the drift flag alone.
+void rebuild_chain(bs_handle *h, bool prepped = false)
 {
     if (!prepped)
         launch_gate(h, 0, 0);
+    if (small_bins(h))
+    {
+        ListArgs a[MAX_LISTS];
+        int32_t nl = 0;
+        for (auto &l : h->lists)
+            a[nl++] = list_args(h, l, l.bstart, l.bidx, h->status, -1);
+        launch_list_build(a, nl, h->stream);
+        for (auto &l : h->lists)
+            expand_rows(h, l, h->status);
+        return;
+    }
     for (auto &l : h->lists)
-        build_list(h, l, gated, -1);
+        build_list(h, l, true, -1);
 }
 
 float rc2(float rc, double f) { return (float)((double)rc * rc * f); }
@@ -1159,7 +1230,7 @@ void launch_step(bs_handle *h, bool energy)
 {
     const size_t e0 = h->prof ? prof_mark(h) : SIZE_MAX;
     launch_gate(h, h->p.rebuild_interval, 1);
-    rebuild_chain(h, true, true);
+    rebuild_chain(h, true);
     if (h->prof)
         prof_span(h, BS_PROF_REBUILD, e0, prof_mark(h));
     launch_forces(h, energy);
@@ -1725,7 +1796,7 @@ int adjoint_sweep(bs_handle *h, AdjBufs &b, double *dk, double *dl0, double *dq)
             if (!still)
             {
                 launch_drift_check(h->pos[h->cur], h->xref, (int32_t)n, half_skin2, h->status, st);
-                rebuild_chain(h, true);
+                rebuild_chain(h);
             }
             if (s == s1 - 1 && s > s0 && !h->lists.empty())
             {
@@ -2181,6 +2252,11 @@ int do_setup(bs_handle *h)
     for (auto &l : h->lists)
     {
         ALLOC(l.cln, int32_t, h->ncl);
+        if (n <= BIN_MAX)
+        {
+            ALLOC(l.bstart, int32_t, l.ncells + 1);
+            ALLOC(l.bidx, int32_t, n);
+        }
         launch_fill_i32(h->status + 3, 0, 1, nullptr, h->stream);
         build_list(h, l, false, 0);
         int32_t st[4];
@@ -2205,7 +2281,7 @@ int do_setup(bs_handle *h)
     }
     const int32_t st1[8] = {0, INT_MAX, 0, 0, 0, 0, 0, 1};
     HIPCHK(h, hipMemcpyAsync(h->status, st1, sizeof st1, hipMemcpyHostToDevice, h->stream));
-    rebuild_chain(h, true);
+    rebuild_chain(h);
     HIPCHK(h, hipStreamSynchronize(h->stream));
 #undef ALLOC
     h->ready = true;
@@ -2537,7 +2613,7 @@ int bs_compute_forces(bs_handle *h, const float *ext_force3, float *force3, doub
         return rc;
     launch_fill_i32(h->status + 2, 0, 1, nullptr, h->stream);
     launch_fill_i32(h->status + 5, 0, 1, nullptr, h->stream);
-    rebuild_chain(h, true);
+    rebuild_chain(h);
     launch_pairs(h, true, h->lists.size());
     launch_springs(h, false, true);
     launch_probe_step(h, false);
@@ -2795,7 +2871,7 @@ int bs_get_pairs(bs_handle *h, int32_t kind, uint32_t *ij, int64_t cap, int64_t 
             lst = &l;
     if (!lst)
         return BS_OK;
-    rebuild_chain(h, true);
+    rebuild_chain(h);
     const int32_t n = (int32_t)h->n;
     const uint32_t mask = kind == BS_NS_ELECTROSTATIC ? PF_CHARGED : kind == BS_NS_HYDROPHOBIC ? PF_HYDRO : 0u;
     const float rc_k = kind == BS_NS_ELECTROSTATIC ? h->p.electrostatic_cutoff

@@ -317,6 +317,30 @@ struct ListArgs
     const int32_t *gate;       // nullable: skip unless *gate != 0
 };
 
+// Binning of a small system for all of its lists in one workgroup (k_bin).
+constexpr int32_t BIN_MAX = 16384;   // particles
+constexpr int32_t BIN_CELLS = 12288; // cells per list
+constexpr int32_t MAX_LISTS = 3;     // steric, Coulomb, hydrophobic
+
+struct BinArgs
+{
+    const float4 *pos;
+    const float4 *shift; // nullable
+    const float4 *jprm;
+    float4 *xref;
+    double *box;
+    int32_t *status, *counters;
+    int32_t *log;        // nullable
+    int32_t n, nlists, interval, advance;
+    struct
+    {
+        int32_t dims[3];
+        float edge;
+        uint32_t mask;
+        int32_t *start, *idx; // [cells + 1], [n]
+    } list[MAX_LISTS];
+};
+
 // ---- launchers (bs_kernels.hip) ----
 // shift (nullable): per-particle offset added to positions for binning, which
 // keeps independent systems of a batch apart on the engine's grid.
@@ -335,7 +359,11 @@ void launch_scatter(const int32_t *cell_of, int32_t n, const int32_t *start, int
                     int32_t *tmp_idx, const int32_t *gate, hipStream_t s);
 void launch_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *start, const int32_t *tmp_idx,
                       const int32_t *key, int32_t *out_idx, const int32_t *gate, hipStream_t s);
-void launch_list_build(const ListArgs &a, hipStream_t s);
+void launch_list_build(const ListArgs *a, int32_t nlists, hipStream_t s);
+// A small system's gate (as launch_prestep) and, when it is set, the reference
+// positions, the box and every list's cells (n <= BIN_MAX, at most BIN_CELLS
+// cells a list).
+void launch_bin(const BinArgs &a, hipStream_t s);
 // Row layout: the cluster lists expanded into one list per particle.  Blocks
 // of 64 consecutive particles; entry t of particle i is
 // rows[((i / 64) * rcap + t) * 64 + i % 64], in the order of the cluster list;

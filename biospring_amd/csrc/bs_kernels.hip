@@ -1195,6 +1195,168 @@ __global__ void __launch_bounds__(BLOCK) k_prestep(int32_t *status, int32_t *cou
         box_partial_block(pos, shift, n, partial);
 }
 
+// A small system's whole binning in one workgroup: the gate, then (when set)
+// the reference positions, the box and, for each list, cell counts, starts and
+// the members in order.  A gated-off step costs one launch instead of one for
+// the gate and four for each list (1.4 us and a gap of 1 us each), a rebuild
+// about 10 us a list at 9,000 beads, as the separate kernels.  Counts and
+// starts are 16-bit halves of LDS words (n <= BIN_MAX).
+constexpr int32_t BIN_BLOCK = 1024;
+constexpr int32_t BIN_EACH = BIN_MAX / BIN_BLOCK; // particles per lane
+
+__global__ void __launch_bounds__(BIN_BLOCK) k_bin(BinArgs a)
+{
+    __shared__ uint32_t half[BIN_CELLS / 2];
+    __shared__ uint16_t member[BIN_MAX];
+    __shared__ double red[6][BIN_BLOCK / 64];
+    __shared__ int32_t wsum[BIN_BLOCK / 64];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if (t == 0)
+    {
+        prestep_gate(a.status, a.counters, a.interval, a.advance, a.log);
+        wsum[0] = gated_off(a.status) ? 0 : 1;
+    }
+    __syncthreads();
+    if (wsum[0] == 0)
+        return;
+    auto at = [&](int32_t i) {
+        float4 p = a.pos[i];
+        if (a.shift)
+        {
+            const float4 o = a.shift[i];
+            p.x += o.x;
+            p.y += o.y;
+            p.z += o.z;
+        }
+        return p;
+    };
+    // the box (exact: minima and maxima of floats), and the reference positions
+    float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int32_t i = t; i < a.n; i += BIN_BLOCK)
+    {
+        a.xref[i] = a.pos[i];
+        const float4 p = at(i);
+        mn[0] = fminf(mn[0], p.x);
+        mn[1] = fminf(mn[1], p.y);
+        mn[2] = fminf(mn[2], p.z);
+        mx[0] = fmaxf(mx[0], p.x);
+        mx[1] = fmaxf(mx[1], p.y);
+        mx[2] = fmaxf(mx[2], p.z);
+    }
+    for (int c = 0; c < 3; ++c)
+    {
+        for (int off = 32; off > 0; off >>= 1)
+        {
+            mn[c] = fminf(mn[c], __shfl_xor(mn[c], off, 64));
+            mx[c] = fmaxf(mx[c], __shfl_xor(mx[c], off, 64));
+        }
+        if (lane == 0)
+        {
+            red[c][wave] = mn[c];
+            red[3 + c][wave] = mx[c];
+        }
+    }
+    __syncthreads();
+    if (t < 6)
+    {
+        double r = red[t][0];
+        for (int w = 1; w < BIN_BLOCK / 64; ++w)
+            r = t < 3 ? fmin(r, red[t][w]) : fmax(r, red[t][w]);
+        a.box[t] = r;
+        red[t][0] = r;
+    }
+    __syncthreads();
+    const double box[6] = {red[0][0], red[1][0], red[2][0], red[3][0], red[4][0], red[5][0]};
+    for (int32_t l = 0; l < a.nlists; ++l)
+    {
+        const auto &L = a.list[l];
+        const int32_t ncells = L.dims[0] * L.dims[1] * L.dims[2];
+        for (int32_t w = t; w < BIN_CELLS / 2; w += BIN_BLOCK)
+            half[w] = 0u;
+        __syncthreads();
+        // cell and (arbitrary) place in it of each of the lane's particles
+        uint16_t cell[BIN_EACH], place[BIN_EACH];
+#pragma unroll
+        for (int q = 0; q < BIN_EACH; ++q)
+        {
+            const int32_t i = t + q * BIN_BLOCK;
+            cell[q] = 0xffffu;
+            place[q] = 0u;
+            if (i < a.n && (L.mask == 0u || (fbits(a.jprm[i].w) & L.mask)))
+            {
+                const float4 p = at(i);
+                const float xs[3] = {p.x, p.y, p.z};
+                int32_t c[3];
+                for (int d = 0; d < 3; ++d)
+                    c[d] = internal_coord(xs[d], box[d], box[3 + d] - box[d], L.dims[d], L.edge);
+                const int32_t id = c[0] + c[1] * L.dims[0] + c[2] * L.dims[0] * L.dims[1];
+                const int sh = 16 * (id & 1);
+                cell[q] = (uint16_t)id;
+                place[q] = (uint16_t)(atomicAdd(&half[id >> 1], 1u << sh) >> sh);
+            }
+        }
+        __syncthreads();
+        // exclusive scan of the counts into starts, BIN_CELLS / 1024 per lane
+        constexpr int PER = BIN_CELLS / 2 / BIN_BLOCK; // words per lane
+        uint32_t w[PER];
+        int32_t sum = 0;
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+        {
+            w[q] = half[t * PER + q];
+            sum += (int32_t)(w[q] & 0xffffu) + (int32_t)(w[q] >> 16);
+        }
+        int32_t inc = sum;
+        for (int off = 1; off < 64; off <<= 1)
+        {
+            const int32_t y = __shfl_up(inc, off, 64);
+            inc += lane >= off ? y : 0;
+        }
+        if (lane == 63)
+            wsum[wave] = inc;
+        __syncthreads();
+        int32_t run = inc - sum;
+        for (int v = 0; v < wave; ++v)
+            run += wsum[v];
+#pragma unroll
+        for (int q = 0; q < PER; ++q)
+        {
+            const int32_t lo = run, hi = run + (int32_t)(w[q] & 0xffffu), id = 2 * (t * PER + q);
+            run = hi + (int32_t)(w[q] >> 16);
+            half[t * PER + q] = (uint32_t)lo | (uint32_t)hi << 16;
+            if (id <= ncells)
+                L.start[id] = lo;
+            if (id + 1 <= ncells)
+                L.start[id + 1] = hi;
+        }
+        if (t == BIN_BLOCK - 1 && ncells == BIN_CELLS)
+            L.start[ncells] = run;
+        __syncthreads();
+        auto start = [&](int32_t id) { return (int32_t)(half[id >> 1] >> (16 * (id & 1)) & 0xffffu); };
+        int32_t total = 0;
+        for (int v = 0; v < BIN_BLOCK / 64; ++v)
+            total += wsum[v];
+#pragma unroll
+        for (int q = 0; q < BIN_EACH; ++q)
+            if (cell[q] != 0xffffu)
+                member[start(cell[q]) + place[q]] = (uint16_t)(t + q * BIN_BLOCK);
+        __syncthreads();
+        // each member's rank by index within its cell
+#pragma unroll
+        for (int q = 0; q < BIN_EACH; ++q)
+            if (cell[q] != 0xffffu)
+            {
+                const int32_t i = t + q * BIN_BLOCK, b = start(cell[q]),
+                              end = cell[q] + 1 < BIN_CELLS ? start(cell[q] + 1) : total;
+                int32_t rank = 0;
+                for (int32_t m = b; m < end; ++m)
+                    rank += (int32_t)member[m] < i ? 1 : 0;
+                L.idx[b + rank] = i;
+            }
+        __syncthreads();
+    }
+}
+
 __global__ void k_fill_i32(int32_t *p, int32_t v, int64_t n, const int32_t *gate)
 {
     if (gated_off(gate))
@@ -1672,6 +1834,11 @@ void launch_prestep(int32_t *status, int32_t *counters, int32_t interval, int32_
         k_prestep<<<nblocks, BLOCK, 0, s>>>(status, counters, interval, advance, pos, shift, n, partial, log);
     else
         k_prestep<<<1, BLOCK, 0, s>>>(status, counters, interval, advance, nullptr, nullptr, 0, nullptr, log);
+}
+
+void launch_bin(const BinArgs &a, hipStream_t s)
+{
+    k_bin<<<1, BIN_BLOCK, 0, s>>>(a);
 }
 
 void launch_rigid(const RigidArgs &a, hipStream_t s)

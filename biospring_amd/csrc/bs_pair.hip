@@ -64,8 +64,14 @@ __device__ inline float lane_f(float x, int k) { return __int_as_float(__builtin
 // come from the cells covering the cluster's bounding box grown by the list
 // radius, so the search is complete for any cluster shape.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(BLOCK) k_cluster_list(ListArgs a)
+struct ListSet
 {
+    ListArgs list[MAX_LISTS];
+};
+
+__global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
+{
+    const ListArgs &a = set.list[blockIdx.y];
     if (gated_off(a.gate))
         return;
     __shared__ uint32_t ex_tab[WAVES][EX_SLOTS];
@@ -718,10 +724,13 @@ inline int32_t cluster_blocks(int32_t ncl) { return (ncl + WAVES - 1) / WAVES; }
 
 } // namespace
 
-void launch_list_build(const ListArgs &a, hipStream_t s)
+void launch_list_build(const ListArgs *a, int32_t nlists, hipStream_t s)
 {
-    if (a.ncl > 0)
-        k_cluster_list<<<cluster_blocks(a.ncl), BLOCK, 0, s>>>(a);
+    ListSet set{};
+    for (int32_t l = 0; l < nlists; ++l)
+        set.list[l] = a[l];
+    if (nlists > 0 && a[0].ncl > 0)
+        k_cluster_list<<<dim3(cluster_blocks(a[0].ncl), nlists), BLOCK, 0, s>>>(set);
 }
 
 // Pair forces in the queue layout: a block of W waves per cluster

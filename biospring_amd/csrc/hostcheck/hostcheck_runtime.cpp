@@ -462,7 +462,7 @@ void launch_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *start, c
 
 // Cluster list build on the CPU with the kernel's semantics (search range =
 // cells covering the cluster bounding box grown by the radius).
-void launch_list_build(const ListArgs &a, hipStream_t)
+static void list_build_one(const ListArgs &a)
 {
     const int64_t nc = (int64_t)a.dims[0] * a.dims[1] * a.dims[2];
     need(a.pos, sizeof(float4) * a.n, "list: pos");
@@ -581,6 +581,14 @@ void launch_list_build(const ListArgs &a, hipStream_t)
             a.status[2] |= 1;
         a.status[3] = std::max(a.status[3], count);
     }
+}
+
+void launch_list_build(const ListArgs *a, int32_t nlists, hipStream_t)
+{
+    if (nlists > MAX_LISTS)
+        hc_fail("list: too many lists");
+    for (int32_t l = 0; l < nlists; ++l)
+        list_build_one(a[l]);
 }
 
 void launch_rows(const uint32_t *cl, const int32_t *cln, int32_t ncl, int32_t cap, uint32_t *rows, int32_t *rlen,
@@ -1368,6 +1376,64 @@ void launch_prestep(int32_t *status, int32_t *counters, int32_t interval, int32_
         counters[0] += 1;
     if (log)
         *log = r;
+}
+
+// A small system's gate and binning, as the separate stand-ins do them.
+void launch_bin(const BinArgs &a, hipStream_t s)
+{
+    if (a.n > BIN_MAX || a.nlists > MAX_LISTS)
+        hc_fail("bin: too large");
+    launch_prestep(a.status, a.counters, a.interval, a.advance, nullptr, nullptr, 0, nullptr, 0, a.log, s);
+    if (gated_off(a.status))
+        return;
+    need(a.xref, sizeof(float4) * a.n, "bin: xref");
+    need(a.box, sizeof(double) * 6, "bin: box");
+    for (int c = 0; c < 3; ++c)
+    {
+        a.box[c] = INFINITY;
+        a.box[3 + c] = -INFINITY;
+    }
+    for (int32_t i = 0; i < a.n; ++i)
+    {
+        const float4 p = shifted(a.pos, a.shift, i);
+        const float xs[3] = {p.x, p.y, p.z};
+        for (int c = 0; c < 3; ++c)
+        {
+            a.box[c] = std::min(a.box[c], (double)xs[c]);
+            a.box[3 + c] = std::max(a.box[3 + c], (double)xs[c]);
+        }
+    }
+    for (int32_t l = 0; l < a.nlists; ++l)
+    {
+        const auto &L = a.list[l];
+        const int32_t nc = L.dims[0] * L.dims[1] * L.dims[2];
+        if (nc > BIN_CELLS)
+            hc_fail("bin: too many cells");
+        need(L.start, sizeof(int32_t) * (nc + 1), "bin: start");
+        need(L.idx, sizeof(int32_t) * a.n, "bin: idx");
+        std::vector<std::vector<int32_t>> cells((size_t)nc);
+        for (int32_t i = 0; i < a.n; ++i)
+        {
+            if (L.mask != 0u && (fbits(a.jprm[i].w) & L.mask) == 0u)
+                continue;
+            const float4 p = shifted(a.pos, a.shift, i);
+            const float xs[3] = {p.x, p.y, p.z};
+            int32_t c[3];
+            for (int q = 0; q < 3; ++q)
+                c[q] = internal_coord(xs[q], a.box[q], a.box[3 + q] - a.box[q], L.dims[q], L.edge);
+            cells[(size_t)(c[0] + c[1] * L.dims[0] + c[2] * L.dims[0] * L.dims[1])].push_back(i);
+        }
+        int32_t at = 0;
+        for (int32_t c = 0; c < nc; ++c)
+        {
+            L.start[c] = at;
+            for (const int32_t i : cells[(size_t)c])
+                L.idx[at++] = i;
+        }
+        L.start[nc] = at;
+    }
+    for (int32_t i = 0; i < a.n; ++i)
+        a.xref[i] = a.pos[i];
 }
 
 void launch_fill_i32(int32_t *p, int32_t v, int64_t n, const int32_t *gate, hipStream_t)
