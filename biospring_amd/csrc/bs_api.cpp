@@ -662,11 +662,18 @@ void plan_grid(bs_handle *h, List &l, const std::vector<float4> &shift)
             total *= l.dims[c];
         }
     }
-    while (total > (1 << 22))
-    { // keep the grid modest for sparse, spread-out systems
+    // no more cells than particles: in sparse or spread-out systems finer ones
+    // are mostly empty, and the scan reads every one (coarse-grained beads with
+    // a 5 A radius: 205,000 cells for 50,000 beads)
+    while (h->n > BIN_MAX && total > h->n)
+    {
+        const double f = std::cbrt((double)h->n / (double)total) * 0.999;
+        total = 1;
         for (int c = 0; c < 3; ++c)
-            l.dims[c] = std::max(1, l.dims[c] / 2);
-        total = (int64_t)l.dims[0] * l.dims[1] * l.dims[2];
+        {
+            l.dims[c] = std::max(1, (int)(l.dims[c] * f));
+            total *= l.dims[c];
+        }
     }
     l.ncells = (int32_t)total;
 }
@@ -1896,7 +1903,8 @@ void launch_adj_pairs(bs_handle *h, const float4 *w, double4 *hw, double *dq)
         a.ncl = h->ncl;
         a.cap = l.cap;
         a.accumulate = li > 0 ? 1 : 0;
-        a.queues = h->p.pair_layout == BS_PAIR_QUEUES ? 1 : 0;
+        a.plan = l.plan;
+        a.nst = l.nst;
         a.rc = l.rc;
         a.rc2lo = rc2(l.rc, 1.0 - 4e-6);
         a.rc2hi = rc2(l.rc, 1.0 + 4e-6);

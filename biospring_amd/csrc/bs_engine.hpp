@@ -237,7 +237,8 @@ struct AdjPairArgs
     double4 *hw;          // [N] H w of this list (overwritten, or added with accumulate)
     double *dq;           // [N] dL/dq accumulator
     int32_t n, ncl, cap, accumulate;
-    int32_t queues;       // the lists read in chunks through per-particle LDS queues (k_adj_pair_q)
+    const char *plan;     // queue layout (else null): the lists' plans, nst records per cluster
+    int32_t nst;
     float rc, rc2lo, rc2hi;
     float steric_scale;
     double kf;            // Coulomb force prefactor incl. scale and 1/eps

@@ -754,9 +754,10 @@ __global__ void __launch_bounds__(BLOCK) k_pair_q(PairArgs a)
     const int32_t ci = blockIdx.x;
     const int il = lane & 7;
     const int32_t i = ci * CLUSTER + il;
-    PairSums s;
-    queue_walk<SMODE, EMODE, HYDRO, ENERGY>(a, ci, w, W, part[w].q, s);
-    s.reduce<ENERGY>();
+    PairEval<SMODE, EMODE, HYDRO, ENERGY> ev(a, ci, part[w].q);
+    queue_walk(a, ci, w, W, part[w].q.idx, ev);
+    PairSums &s = ev.s;
+    s.template reduce<ENERGY>();
     if (W > 1)
     {
         if (lane < CLUSTER)
@@ -981,116 +982,126 @@ void launch_pair(const PairArgs &a, int32_t elec_mode, int32_t hydro, int32_t nb
 }
 
 // ---------------------------------------------------------------------------
-// The adjoint's pair terms in the queue layout (as k_pair_q):
-// each chunk's j data (position, parameters, adjoint weight; the index j in
-// the weight's unused fourth word, for a static partner's dq) is staged in
-// LDS once, queued per cluster particle, and drained 8 entries per round.
-// The terms and their FP64 sums are k_adj_pair's.
+// The adjoint's pair terms in the queue layout: the walk of the pair forces
+// (queue_walk) with k_adj_pair's terms and FP64 sums, W waves per cluster.  A
+// ring entry also holds j's adjoint weight; its fourth word is the index j,
+// with bit 31 for a static partner (whose dq takes an atomic).  jprm's flags
+// are not needed beside it: a charge is 0 where the flag is clear.
+// At 40,000 beads 75 -> 52 us a launch, at 2,000 (one wave per cluster left
+// the chip idle) 33 -> 12 us.
 // ---------------------------------------------------------------------------
-constexpr int32_t ACHUNK = 64; // entries per chunk: three float4 per entry in LDS
+struct AdjLds
+{
+    float4 pos[QRING], w[QRING];
+    float2 prm[QRING];
+    QueueIdx idx;
+    double sum[CLUSTER][4];
+};
+
+template <int SMODE, int EMODE> struct AdjEval
+{
+    const AdjPairArgs &a;
+    AdjLds &q;
+    float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), ri = pi, wi = pi;
+    uint32_t fli;
+    float cs, kf;
+    uint32_t j;
+    float4 pj, rj, vj;
+    double hx = 0.0, hy = 0.0, hz = 0.0, dqi = 0.0;
+
+    __device__ AdjEval(const AdjPairArgs &args, int32_t ci, AdjLds &lds)
+        : a(args), q(lds), cs((float)args.k.c_spring), kf((float)args.kf)
+    {
+        const int32_t i = ci * CLUSTER + (int32_t)(threadIdx.x & 7u);
+        if (i < a.n)
+        {
+            pi = a.pos[i];
+            ri = a.jprm[i];
+            wi = a.w[i];
+        }
+        fli = fbits(ri.w);
+    }
+    __device__ void fetch(uint32_t jn)
+    {
+        j = jn;
+        pj = partner(a.pos, j);
+        rj = partner(a.jprm, j);
+        vj = partner(a.w, j);
+    }
+    __device__ void put(int32_t slot)
+    {
+        q.pos[slot] = pj;
+        q.prm[slot] = make_float2(rj.x, rj.y);
+        q.w[slot] = make_float4(vj.x, vj.y, vj.z,
+                                __uint_as_float(j | ((fbits(rj.w) & PF_STATIC) ? 0x80000000u : 0u)));
+    }
+    __device__ void pair(bool valid, int32_t src)
+    {
+        const float4 p = q.pos[src], v = q.w[src];
+        const float2 r = q.prm[src];
+        const uint32_t w = __float_as_uint(v.w);
+        const uint32_t flags = ((int32_t)w < 0 ? PF_STATIC : 0u) | (p.w != 0.0f ? PF_CHARGED : 0u);
+        adj_pair_term<SMODE, EMODE>(valid, pi, ri, fli, wi, p, make_float4(r.x, r.y, 0.0f, __uint_as_float(flags)),
+                                    make_float4(v.x, v.y, v.z, 0.0f), (int32_t)(w & 0x7fffffffu), a, cs, kf, hx, hy,
+                                    hz, dqi);
+    }
+};
 
 template <int SMODE, int EMODE>
 __global__ void __launch_bounds__(BLOCK) k_adj_pair_q(AdjPairArgs a)
 {
-    __shared__ float4 qpos[WAVES][ACHUNK], qprm[WAVES][ACHUNK], qw[WAVES][ACHUNK];
-    __shared__ uint8_t qidx[WAVES][CLUSTER][ACHUNK];
-    const int wv = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int32_t ci = __builtin_amdgcn_readfirstlane(blockIdx.x * WAVES + wv);
-    if (ci >= a.ncl)
-        return; // whole wave
-    const int32_t il = lane & 7, sl = lane >> 3;
-    const int32_t i = ci * CLUSTER + il;
-    const bool iv = i < a.n;
-    const float4 pi = iv ? a.pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 ri = iv ? a.jprm[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 wi = iv ? a.w[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint32_t fli = fbits(ri.w);
-    const float cs = (float)a.k.c_spring;
-    const float kf = (float)a.kf;
-    double hx = 0.0, hy = 0.0, hz = 0.0, dqi = 0.0;
-    const int32_t cnt = __builtin_amdgcn_readfirstlane(a.cln[ci]);
-    const uint32_t *L = a.cl + (size_t)ci * a.cap;
-    // 64 entries at a time in list order; the next stretch in flight
-    uint32_t w = lane < cnt ? L[lane] : 0u;
-    uint32_t j = w & CL_JMASK;
-    float4 pj = a.pos[j], rj = a.jprm[j], vj = a.w[j];
-    for (int32_t t0 = 0; t0 < cnt; t0 += ACHUNK)
+    extern __shared__ __align__(16) char lds[];
+    AdjLds *part = reinterpret_cast<AdjLds *>(lds); // one per wave
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int W = blockDim.x >> 6;
+    const int32_t ci = blockIdx.x;
+    AdjEval<SMODE, EMODE> ev(a, ci, part[w]);
+    queue_walk(a, ci, w, W, part[w].idx, ev);
+    double h[4] = {ev.hx, ev.hy, ev.hz, ev.dqi};
+    for (int c = 0; c < 4; ++c)
+        for (int off = 8; off < 64; off <<= 1)
+            h[c] += __shfl_xor(h[c], off, 64);
+    if (W > 1)
     {
-        qpos[wv][lane] = pj;
-        qprm[wv][lane] = rj;
-        qw[wv][lane] = make_float4(vj.x, vj.y, vj.z, __uint_as_float(j));
-        int32_t nq[CLUSTER];
-#pragma unroll
-        for (int k = 0; k < CLUSTER; ++k)
-        {
-            const bool on = (w >> (24 + k)) & 1u;
-            const uint64_t b = __ballot(on);
-            if (on)
-                qidx[wv][k][lanes_below(b)] = (uint8_t)lane;
-            nq[k] = __popcll(b);
-        }
-        const int32_t tn = t0 + ACHUNK + lane;
-        w = tn < cnt ? L[tn] : 0u;
-        j = w & CL_JMASK;
-        pj = a.pos[j];
-        rj = a.jprm[j];
-        vj = a.w[j];
-        wave_lds_sync();
-        int32_t mine = nq[0], most = nq[0];
-#pragma unroll
-        for (int k = 1; k < CLUSTER; ++k)
-        {
-            mine = il == k ? nq[k] : mine;
-            most = max(most, nq[k]);
-        }
-        for (int32_t e0 = 0; e0 < most; e0 += 8) // wave-uniform rounds
-        {
-            const int32_t e = e0 + sl;
-            const bool valid = e < mine;
-            const int32_t src = valid ? (int32_t)qidx[wv][il][e] : 0;
-            const float4 sw = qw[wv][src];
-            adj_pair_term<SMODE, EMODE>(valid, pi, ri, fli, wi, qpos[wv][src], qprm[wv][src],
-                                        make_float4(sw.x, sw.y, sw.z, 0.0f), (int32_t)__float_as_uint(sw.w), a, cs,
-                                        kf, hx, hy, hz, dqi);
-        }
-        wave_lds_sync();
+        if (lane < CLUSTER)
+            for (int c = 0; c < 4; ++c)
+                part[w].sum[lane][c] = h[c];
+        __syncthreads();
+        if (w != 0)
+            return;
+        for (int v = 1; v < W; ++v)
+            for (int c = 0; c < 4; ++c)
+                h[c] += part[v].sum[lane & 7][c];
     }
-    for (int off = 8; off < 64; off <<= 1)
+    const int32_t i = ci * CLUSTER + lane;
+    if (lane >= CLUSTER || i >= a.n)
+        return;
+    double4 o = make_double4(h[0], h[1], h[2], 0.0);
+    if (a.accumulate)
     {
-        hx += __shfl_xor(hx, off, 64);
-        hy += __shfl_xor(hy, off, 64);
-        hz += __shfl_xor(hz, off, 64);
-        dqi += __shfl_xor(dqi, off, 64);
+        const double4 b = a.hw[i];
+        o.x += b.x;
+        o.y += b.y;
+        o.z += b.z;
     }
-    if (sl == 0 && iv)
-    {
-        double4 h = make_double4(hx, hy, hz, 0.0);
-        if (a.accumulate)
-        {
-            const double4 o = a.hw[i];
-            h.x += o.x;
-            h.y += o.y;
-            h.z += o.z;
-        }
-        a.hw[i] = h;
-        // a static particle's dq is only ever added to atomically (by its
-        // dynamic partners); a plain read-modify-write here would race
-        if (EMODE > 0 && !(fli & PF_STATIC))
-            a.dq[i] += dqi;
-    }
+    a.hw[i] = o;
+    // a static particle's dq is only ever added to atomically (by its
+    // dynamic partners); a plain read-modify-write here would race
+    if (EMODE > 0 && !(ev.fli & PF_STATIC))
+        a.dq[i] += h[3];
 }
 
 template <int S> static void adj2(const AdjPairArgs &a, int32_t em, int32_t nb, hipStream_t s)
 {
-    if (a.queues)
+    if (a.plan)
     {
+        const int32_t W = pair_waves(a.ncl), lds = W * (int32_t)sizeof(AdjLds);
         if (em == 0)
-            k_adj_pair_q<S, 0><<<nb, BLOCK, 0, s>>>(a);
+            k_adj_pair_q<S, 0><<<a.ncl, 64 * W, lds, s>>>(a);
         else if (em == 1)
-            k_adj_pair_q<S, 1><<<nb, BLOCK, 0, s>>>(a);
+            k_adj_pair_q<S, 1><<<a.ncl, 64 * W, lds, s>>>(a);
         else
-            k_adj_pair_q<S, 2><<<nb, BLOCK, 0, s>>>(a);
+            k_adj_pair_q<S, 2><<<a.ncl, 64 * W, lds, s>>>(a);
         return;
     }
     if (em == 0)

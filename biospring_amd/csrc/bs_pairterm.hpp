@@ -244,15 +244,21 @@ constexpr int32_t QSTRETCH = 3;           // stretches of 64 words in the ring
 constexpr int32_t QRING = 64 * QSTRETCH;
 constexpr int32_t QLEN = 256;             // queue entries (a power of two >= QRING)
 
-// One wave's ring and queues in LDS.  j's parameters: all of jprm where the
+// One wave's queues in LDS.  Their stride keeps the 8 particles' entries in
+// different banks.
+struct QueueIdx
+{
+    uint8_t at[CLUSTER][QLEN + 16];
+};
+
+// One wave's ring of a pair walk.  j's parameters: all of jprm where the
 // hydrophobicity or the flags are read (WIDE: hydrophobic term, energies),
-// else the two steric factors.  The queues' stride keeps the 8 particles'
-// entries in different banks.
+// else the two steric factors.
 template <bool WIDE> struct QueueLds
 {
     float4 pos[QRING];
     float4 prm[QRING];
-    uint8_t idx[CLUSTER][QLEN + 16];
+    QueueIdx idx;
     __device__ void put(int s, float4 r) { prm[s] = r; }
     __device__ float4 get(int s) const { return prm[s]; }
 };
@@ -260,7 +266,7 @@ template <> struct QueueLds<false>
 {
     float4 pos[QRING];
     float2 prm[QRING];
-    uint8_t idx[CLUSTER][QLEN + 16];
+    QueueIdx idx;
     __device__ void put(int s, float4 r) { prm[s] = make_float2(r.x, r.y); }
     __device__ float4 get(int s) const
     {
@@ -382,17 +388,14 @@ struct PairSums
     }
 };
 
-template <int SMODE, int EMODE, int HYDRO, bool ENERGY>
-__device__ inline void queue_walk(const PairArgs &a, int32_t ci, int32_t w, int32_t W, QueueLds<ENERGY || HYDRO> &q,
-                                  PairSums &s)
+// The walk of wave w of W over cluster ci's list.  ev.fetch(j) loads a word's
+// data (one j per lane), ev.put(slot) stores it in the ring, ev.pair(valid,
+// slot) evaluates one pair of the lane's particle.
+template <class Args, class Eval>
+__device__ inline void queue_walk(const Args &a, int32_t ci, int32_t w, int32_t W, QueueIdx &idx, Eval &ev)
 {
     const int lane = threadIdx.x & 63;
     const int32_t il = lane & 7, sl = lane >> 3;
-    const int32_t i = ci * CLUSTER + il;
-    const bool iv = i < a.n;
-    const float4 pi = iv ? a.pos[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4 ri = iv ? a.jprm[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    const PairI c = pair_i<SMODE, EMODE>(pi, ri, a);
     const int32_t cnt = __builtin_amdgcn_readfirstlane(a.cln[ci]);
     const uint32_t *L = a.cl + (size_t)ci * a.cap;
     // constant during the kernel: read with scalar loads
@@ -400,8 +403,7 @@ __device__ inline void queue_walk(const PairArgs &a, int32_t ci, int32_t w, int3
     PlanPtr plan = (PlanPtr)(a.plan + ((size_t)ci * a.nst + w) * QPLAN_BYTES);
     // the first stretch in flight
     int32_t t = 64 * w;
-    uint32_t j = t + lane < cnt ? L[t + lane] & CL_JMASK : 0u;
-    float4 pj = partner(a.pos, j), rj = partner(a.jprm, j);
+    ev.fetch(t + lane < cnt ? L[t + lane] & CL_JMASK : 0u);
     // the stretch's plan (scalar registers), and entries queued per particle
     uint64_t sees[CLUSTER], counts = 0;
     int32_t rounds = 0;
@@ -421,16 +423,15 @@ __device__ inline void queue_walk(const PairArgs &a, int32_t ci, int32_t w, int3
     int32_t slot = 0;
     while (t < cnt)
     {
-        q.pos[slot + lane] = pj;
-        q.put(slot + lane, rj);
+        ev.put(slot + lane);
 #pragma unroll
         for (int k = 0; k < CLUSTER; ++k)
         {
             const uint64_t b = sees[k];
             if (__builtin_amdgcn_inverse_ballot_w64(b))
-                q.idx[k][__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
-                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)b, tail[k])) &
-                         (QLEN - 1)] = (uint8_t)(slot + lane);
+                idx.at[k][__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)b, tail[k])) &
+                          (QLEN - 1)] = (uint8_t)(slot + lane);
             tail[k] += (uint32_t)__popcll(b);
         }
         counts = plan->counts;
@@ -442,24 +443,57 @@ __device__ inline void queue_walk(const PairArgs &a, int32_t ci, int32_t w, int3
         if (t < cnt)
         {
             read_plan();
-            j = t + lane < cnt ? L[t + lane] & CL_JMASK : 0u;
-            pj = partner(a.pos, j);
-            rj = partner(a.jprm, j);
+            ev.fetch(t + lane < cnt ? L[t + lane] & CL_JMASK : 0u);
         }
         wave_lds_sync();
         int32_t e = head + sl;
         for (int32_t r = 0; r < rounds; ++r, e += 8)
         {
             const bool valid = e < mine;
-            const int32_t src = valid ? (int32_t)q.idx[il][e & (QLEN - 1)] : 0;
-            interact<SMODE, EMODE, HYDRO, ENERGY>(valid, pi, ri, q.pos[src], q.get(src), a, c, s.fx, s.fy, s.fz, s.es,
-                                                  s.ee, s.eh);
+            ev.pair(valid, valid ? (int32_t)idx.at[il][e & (QLEN - 1)] : 0);
         }
         head = min(head + 8 * rounds, mine);
         wave_lds_sync();
         slot = slot == QRING - 64 ? 0 : slot + 64;
     }
 }
+
+// The pair terms as the walk evaluates them.
+template <int SMODE, int EMODE, int HYDRO, bool ENERGY> struct PairEval
+{
+    const PairArgs &a;
+    QueueLds<ENERGY || HYDRO> &q;
+    float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), ri = make_float4(0.f, 0.f, 0.f, 0.f);
+    PairI c;
+    float4 pj, rj;
+    PairSums s;
+
+    __device__ PairEval(const PairArgs &args, int32_t ci, QueueLds<ENERGY || HYDRO> &lds) : a(args), q(lds)
+    {
+        const int32_t i = ci * CLUSTER + (int32_t)(threadIdx.x & 7u);
+        if (i < a.n)
+        {
+            pi = a.pos[i];
+            ri = a.jprm[i];
+        }
+        c = pair_i<SMODE, EMODE>(pi, ri, a);
+    }
+    __device__ void fetch(uint32_t j)
+    {
+        pj = partner(a.pos, j);
+        rj = partner(a.jprm, j);
+    }
+    __device__ void put(int32_t slot)
+    {
+        q.pos[slot] = pj;
+        q.put(slot, rj);
+    }
+    __device__ void pair(bool valid, int32_t src)
+    {
+        interact<SMODE, EMODE, HYDRO, ENERGY>(valid, pi, ri, q.pos[src], q.get(src), a, c, s.fx, s.fy, s.fz, s.es,
+                                              s.ee, s.eh);
+    }
+};
 
 } // namespace
 

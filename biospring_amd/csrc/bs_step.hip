@@ -95,11 +95,11 @@ __global__ void __launch_bounds__(BLOCK) k_step(PairArgs p, SpringArgs a)
     const int rows = CLUSTER / W;
     spring_walk<COMP, ENERGY>(a, ci * CLUSTER + w * rows, rows, part[w].spring);
     {
-        PairSums s;
-        queue_walk<SMODE, EMODE, HYDRO, ENERGY>(p, ci, w, W, part[w].q, s);
-        s.reduce<ENERGY>();
+        PairEval<SMODE, EMODE, HYDRO, ENERGY> ev(p, ci, part[w].q);
+        queue_walk(p, ci, w, W, part[w].q.idx, ev);
+        ev.s.template reduce<ENERGY>();
         if (lane < CLUSTER)
-            s.store<ENERGY>(part[w].pair[lane]);
+            ev.s.template store<ENERGY>(part[w].pair[lane]);
     }
     __syncthreads();
     const int t = threadIdx.x;
