@@ -35,7 +35,8 @@ struct List
     uint32_t imask = 0, jmask = 0;
     int32_t dims[3] = {1, 1, 1};
     int32_t ncells = 1;
-    int32_t *bstart = nullptr, *bidx = nullptr; // a small system's cells (k_bin): [ncells + 1], [n]
+    int32_t *bstart = nullptr; // a small system's cells (k_bin): [ncells + 1]
+    float4 *bxs = nullptr;     // and their member words: [n]
     int32_t cap = 0;          // entries per i-cluster
     uint32_t *cl = nullptr;   // [ncl * cap] j | mask << 24, in search order
     int32_t *cln = nullptr;   // [ncl]
@@ -177,6 +178,7 @@ struct bs_handle
     uint32_t *ex_w = nullptr;                         // j << 8 | bonded mask
     int32_t *cell_of = nullptr, *counts = nullptr, *cstart = nullptr, *ctmp = nullptr,
             *cidx = nullptr;
+    float4 *cxs = nullptr; // member words of the engine's cells, in cell order
     int32_t cell_cap = 0;
     double *box_part = nullptr, *box = nullptr;
     int32_t box_blocks = 0;
@@ -339,7 +341,7 @@ void free_device(bs_handle *h)
     }
     f(h->vel); f(h->fnb); f(h->jprm); f(h->iprm); f(h->xref); f(h->fext); f(h->fout);
     f(h->sp_ptr); f(h->sp_e); f(h->perm_d); f(h->sp_k);
-    f(h->cell_of); f(h->counts); f(h->cstart); f(h->ctmp); f(h->cidx);
+    f(h->cell_of); f(h->counts); f(h->cstart); f(h->ctmp); f(h->cidx); f(h->cxs);
     f(h->box_part); f(h->box); f(h->energies_d); f(h->status); f(h->counters);
     f(h->epp); f(h->ese); f(h->seg_start); f(h->sys_seg); f(h->seg_part); f(h->sys_E); f(h->shift);
     h->epp = h->ese = nullptr;
@@ -369,7 +371,7 @@ void free_device(bs_handle *h)
         f(l.cln);
         f(l.plan);
         f(l.bstart);
-        f(l.bidx);
+        f(l.bxs);
         f(l.rows);
         f(l.rlen);
     }
@@ -380,6 +382,7 @@ void free_device(bs_handle *h)
     h->sp_e = nullptr;
     h->sp_k = nullptr;
     h->cell_of = h->counts = h->cstart = h->ctmp = h->cidx = nullptr;
+    h->cxs = nullptr;
     h->box_part = h->box = h->energies_d = nullptr;
     h->status = h->counters = nullptr;
     h->cell_cap = 0;
@@ -392,7 +395,7 @@ void free_device(bs_handle *h)
 int check_device(bs_handle *h)
 {
     const void *need[] = {h->pos[0], h->pos[1], h->vel, h->fnb, h->jprm, h->iprm, h->xref, h->fext, h->fout,
-                          h->sp_ptr, h->sp_e, h->sp_k, h->perm_d, h->cell_of, h->ctmp, h->cidx,
+                          h->sp_ptr, h->sp_e, h->sp_k, h->perm_d, h->cell_of, h->ctmp, h->cidx, h->cxs,
                           h->counts, h->cstart, h->box, h->box_part, h->epp, h->ese, h->seg_start,
                           h->sys_seg, h->seg_part, h->sys_E, h->energies_d, h->status, h->counters, h->ex_ptr,
                           h->ex_w};
@@ -702,8 +705,8 @@ int ensure_cells(bs_handle *h, int32_t ncells)
 
 const int32_t *gate_of(bs_handle *h, bool gated) { return gated ? h->status : nullptr; }
 
-// The build arguments of list l from the cells at start, idx.
-ListArgs list_args(const bs_handle *h, const List &l, const int32_t *start, const int32_t *idx, const int32_t *gate,
+// The build arguments of list l from the cells at start, xs.
+ListArgs list_args(const bs_handle *h, const List &l, const int32_t *start, const float4 *xs, const int32_t *gate,
                    int32_t cap_override)
 {
     ListArgs a{};
@@ -711,7 +714,7 @@ ListArgs list_args(const bs_handle *h, const List &l, const int32_t *start, cons
     a.shift = h->shift;
     a.jprm = h->jprm;
     a.cell_start = start;
-    a.cell_idx = idx;
+    a.cell_xs = xs;
     a.box = h->box;
     a.ex_ptr = h->ex_ptr;
     a.ex_w = h->ex_w;
@@ -755,15 +758,15 @@ void build_list(bs_handle *h, List &l, bool gated, int32_t cap_override)
                     0.5f * l.radius, 0, h->cell_of, h->counts, g, s);
     launch_scan(h->counts, h->cstart, l.ncells, g, s);
     launch_scatter(h->cell_of, n, h->cstart, h->counts, 1, h->ctmp, g, s);
-    launch_cell_sort(h->cell_of, n, h->cstart, h->ctmp, nullptr, h->cidx, g, s);
-    const ListArgs a = list_args(h, l, h->cstart, h->cidx, g, cap_override);
+    launch_cell_members(h->cell_of, n, h->cstart, h->ctmp, h->pos[h->cur], h->shift, h->cxs, 0, g, s);
+    const ListArgs a = list_args(h, l, h->cstart, h->cxs, g, cap_override);
     launch_list_build(&a, 1, s);
     if (cap_override < 0)
         expand_rows(h, l, g);
 }
 
 // Whether one workgroup bins this system (setup gave its lists their cells).
-bool small_bins(const bs_handle *h) { return !h->lists.empty() && h->lists.front().bidx; }
+bool small_bins(const bs_handle *h) { return !h->lists.empty() && h->lists.front().bxs; }
 
 // The gate kernel: with lists, it also writes the box partials of the
 // current positions for the chain's cell binning, or does the whole binning
@@ -795,7 +798,7 @@ void launch_gate(bs_handle *h, int32_t interval, int32_t advance)
             a.list[li].edge = 0.5f * l.radius;
             a.list[li].mask = l.jmask;
             a.list[li].start = l.bstart;
-            a.list[li].idx = l.bidx;
+            a.list[li].xs = l.bxs;
         }
         launch_bin(a, h->stream);
         return;
@@ -816,7 +819,7 @@ void rebuild_chain(bs_handle *h, bool prepped = false)
         ListArgs a[MAX_LISTS];
         int32_t nl = 0;
         for (auto &l : h->lists)
-            a[nl++] = list_args(h, l, l.bstart, l.bidx, h->status, -1);
+            a[nl++] = list_args(h, l, l.bstart, l.bxs, h->status, -1);
         launch_list_build(a, nl, h->stream);
         for (auto &l : h->lists)
             expand_rows(h, l, h->status);
@@ -1955,6 +1958,7 @@ int do_setup(bs_handle *h)
     ALLOC(h->cell_of, int32_t, n);
     ALLOC(h->ctmp, int32_t, n);
     ALLOC(h->cidx, int32_t, n);
+    ALLOC(h->cxs, float4, n);
     ALLOC(h->status, int32_t, 8);
     ALLOC(h->counters, int32_t, 4);
     ALLOC(h->energies_d, double, BS_NUM_ENERGIES);
@@ -2263,7 +2267,7 @@ int do_setup(bs_handle *h)
         if (n <= BIN_MAX)
         {
             ALLOC(l.bstart, int32_t, l.ncells + 1);
-            ALLOC(l.bidx, int32_t, n);
+            ALLOC(l.bxs, float4, n);
         }
         launch_fill_i32(h->status + 3, 0, 1, nullptr, h->stream);
         build_list(h, l, false, 0);
@@ -3474,7 +3478,7 @@ static int springs_from_cutoff(bs_handle *h, double cutoff, float stiffness, con
         HIPCHK(h, e);
         int32_t *tmp = S.get<int32_t>((size_t)n, e);
         HIPCHK(h, e);
-        int32_t *cidx = S.get<int32_t>((size_t)n, e);
+        float4 *xs = S.get<float4>((size_t)n, e);
         HIPCHK(h, e);
         int32_t *rcnt = S.get<int32_t>((size_t)n, e);
         HIPCHK(h, e);
@@ -3484,12 +3488,12 @@ static int springs_from_cutoff(bs_handle *h, double cutoff, float stiffness, con
         launch_scan(counts, cstart, (int32_t)ncells, nullptr, st);
         launch_fill_i32(cursor, 0, ncells, nullptr, st);
         launch_scatter(cell_of, (int32_t)n, cstart, cursor, 0, tmp, nullptr, st);
-        launch_cell_sort(cell_of, (int32_t)n, cstart, tmp, nullptr, cidx, nullptr, st);
+        launch_cell_members(cell_of, (int32_t)n, cstart, tmp, pos, nullptr, xs, 1, nullptr, st);
         TopoArgs a{};
         a.pos = pos;
         a.box = box;
         a.cstart = cstart;
-        a.cidx = cidx;
+        a.xs = xs;
         a.counts = rcnt;
         a.n = (int32_t)n;
         for (int q = 0; q < 3; ++q)

@@ -277,7 +277,7 @@ struct TopoArgs
     const float4 *pos;        // original order; .w = static flag bits
     const double *box;        // [6]
     const int32_t *cstart;    // [ncells + 1]
-    const int32_t *cidx;      // members sorted by index within each cell
+    const float4 *xs;         // member words sorted by index within each cell; bit 31: static
     const int32_t *offs;      // nullable: fill pass, row starts [n + 1]
     int32_t *counts;          // count pass: [n]
     int32_t *jout;            // fill pass: [springs]
@@ -299,7 +299,7 @@ struct ListArgs
     const float4 *shift;       // nullable: per-particle offset of its system for binning
     const float4 *jprm;
     const int32_t *cell_start; // [ncells + 1]
-    const int32_t *cell_idx;   // sorted members
+    const float4 *cell_xs;     // member words in cell order (k_cell_sort), those with j_mask only
     const double *box;         // [6] current box (device)
     const int32_t *ex_ptr;     // [ncl + 1] static exclusions per i-cluster
     const uint32_t *ex_w;      // j << 8 | bonded mask, sorted by j
@@ -338,7 +338,8 @@ struct BinArgs
         int32_t dims[3];
         float edge;
         uint32_t mask;
-        int32_t *start, *idx; // [cells + 1], [n]
+        int32_t *start; // [cells + 1]
+        float4 *xs;     // [n] member words in cell order
     } list[MAX_LISTS];
 };
 
@@ -360,6 +361,11 @@ void launch_scatter(const int32_t *cell_of, int32_t n, const int32_t *start, int
                     int32_t *tmp_idx, const int32_t *gate, hipStream_t s);
 void launch_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *start, const int32_t *tmp_idx,
                       const int32_t *key, int32_t *out_idx, const int32_t *gate, hipStream_t s);
+// The members' words in cell order instead: binning position and index (bit 31
+// with flagged: pos.w is not 0).
+void launch_cell_members(const int32_t *cell_of, int32_t n, const int32_t *start, const int32_t *tmp_idx,
+                         const float4 *pos, const float4 *shift, float4 *xs, int32_t flagged, const int32_t *gate,
+                         hipStream_t s);
 void launch_list_build(const ListArgs *a, int32_t nlists, hipStream_t s);
 // A small system's gate (as launch_prestep) and, when it is set, the reference
 // positions, the box and every list's cells (n <= BIN_MAX, at most BIN_CELLS

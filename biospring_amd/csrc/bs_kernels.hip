@@ -258,9 +258,30 @@ __global__ void k_scatter(const int32_t *cell_of, int32_t n, const int32_t *star
     tmp[start[c] + slot] = i;
 }
 
-// Places each member at its rank by key within its cell (keys are distinct).
+// A binned particle as the searches read it, in cell order: its binning
+// position (with its system's offset) and its index, so that a candidate is
+// one coalesced load.
+__device__ inline float4 member_word(const float4 *pos, const float4 *shift, int32_t i, bool flagged)
+{
+    float4 p = pos[i];
+    const uint32_t flag = flagged && fbits(p.w) != 0u ? 0x80000000u : 0u;
+    if (shift)
+    {
+        const float4 o = shift[i];
+        p.x += o.x;
+        p.y += o.y;
+        p.z += o.z;
+    }
+    p.w = __uint_as_float((uint32_t)i | flag);
+    return p;
+}
+
+// Places each member at its rank by key within its cell (keys are distinct):
+// its index in out, or (xs) its member word; flagged: bit 31 of the index for
+// a nonzero pos.w.
 __global__ void k_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *start, const int32_t *tmp,
-                            const int32_t *key, int32_t *out, const int32_t *gate)
+                            const int32_t *key, int32_t *out, const float4 *pos, const float4 *shift, float4 *xs,
+                            int32_t flagged, const int32_t *gate)
 {
     if (gated_off(gate))
         return;
@@ -278,7 +299,10 @@ __global__ void k_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *st
         const int32_t m = tmp[t];
         rank += (key ? key[m] : m) < ki;
     }
-    out[b + rank] = i;
+    if (xs)
+        xs[b + rank] = member_word(pos, shift, i, flagged != 0);
+    else
+        out[b + rank] = i;
 }
 
 // ---------------------------------------------------------------------------
@@ -1070,11 +1094,11 @@ __global__ __launch_bounds__(64 * TOPO_WAVES) void k_topo_rows(TopoArgs a)
 #pragma unroll
             for (int q = 7; q >= 0; --q)
                 m = t < re[q] ? rs[q] + t : m;
-            j = a.cidx[m];
+            const float4 pj = a.xs[m];
+            j = (int32_t)(fbits(pj.w) & 0x7fffffffu);
             if (j > i && !(a.group && a.group[j] == gi)) // same topology: skipped when merging
             {
-                const float4 pj = a.pos[j];
-                if (!(si && fbits(pj.w) != 0u))
+                if (!(si && (fbits(pj.w) >> 31) != 0u))
                 {
                     r2 = topo_r2(pi, pj);
                     // SpringAlreadyExistsException: the loaded spring stays
@@ -1351,7 +1375,7 @@ __global__ void __launch_bounds__(BIN_BLOCK) k_bin(BinArgs a)
                 int32_t rank = 0;
                 for (int32_t m = b; m < end; ++m)
                     rank += (int32_t)member[m] < i ? 1 : 0;
-                L.idx[b + rank] = i;
+                L.xs[b + rank] = member_word(a.pos, a.shift, i, false);
             }
         __syncthreads();
     }
@@ -1695,7 +1719,15 @@ void launch_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *start, c
                       const int32_t *key, int32_t *out, const int32_t *gate, hipStream_t s)
 {
     if (n > 0)
-        k_cell_sort<<<nblk(n), BLOCK, 0, s>>>(cell_of, n, start, tmp, key, out, gate);
+        k_cell_sort<<<nblk(n), BLOCK, 0, s>>>(cell_of, n, start, tmp, key, out, nullptr, nullptr, nullptr, 0, gate);
+}
+
+void launch_cell_members(const int32_t *cell_of, int32_t n, const int32_t *start, const int32_t *tmp,
+                         const float4 *pos, const float4 *shift, float4 *xs, int32_t flagged, const int32_t *gate,
+                         hipStream_t s)
+{
+    if (n > 0)
+        k_cell_sort<<<nblk(n), BLOCK, 0, s>>>(cell_of, n, start, tmp, nullptr, nullptr, pos, shift, xs, flagged, gate);
 }
 
 template <int G> static void spring_g(const SpringArgs &a, int32_t nb, hipStream_t s)

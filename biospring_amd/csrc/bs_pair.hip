@@ -64,24 +64,11 @@ __device__ inline float lane_f(float x, int k) { return __int_as_float(__builtin
 // come from the cells covering the cluster's bounding box grown by the list
 // radius, so the search is complete for any cluster shape.
 // ---------------------------------------------------------------------------
-struct ListSet
+__device__ inline void cluster_list(const ListArgs &a, int32_t ci, uint32_t *tab)
 {
-    ListArgs list[MAX_LISTS];
-};
-
-__global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
-{
-    const ListArgs &a = set.list[blockIdx.y];
-    if (gated_off(a.gate))
-        return;
-    __shared__ uint32_t ex_tab[WAVES][EX_SLOTS];
     const int lane = threadIdx.x & 63;
-    const int32_t ci = blockIdx.x * WAVES + (threadIdx.x >> 6);
-    if (ci >= a.ncl)
-        return; // whole wave
     // exclusions of this cluster into the wave's hash table (small sets);
     // larger sets are searched in global memory
-    uint32_t *tab = ex_tab[threadIdx.x >> 6];
     bool ex_lds = false;
     if (a.exclude_bonded)
     {
@@ -187,9 +174,8 @@ __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
         // The candidates form a stream, generated in row order (a row's
         // cells cx0..cx1 are contiguous in the cell array), cut into batches
         // of 64 that run across row ends, so that short rows do not leave
-        // lanes idle.  A three-stage pipeline runs over the batches: while
-        // batch b is tested, batch b+1's positions and batch b+2's particle
-        // indices are in flight, so a batch never waits for its own loads.
+        // lanes idle.  While batch b is tested, batch b+1's member words
+        // (positions and indices, contiguous in a run) are in flight.
         // Row setup is lane-parallel: lane l takes row rbase + l of the
         // (cy fastest, then cz) order, computes its x range and member run,
         // and a wave prefix sum places the runs in the stream, 64 rows per
@@ -262,42 +248,25 @@ __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
             spos = lim;
             return true;
         };
-        // Index loads are clamped into the cell array (n entries); a lane
-        // past its batch's end gathers particle 0 and tests nothing.
-        int32_t t0, t1, t2;
+        // Loads are clamped into the cell array (n entries); a lane past its
+        // batch's end tests nothing.
+        int32_t t0, t1;
         bool h0 = next_batch(t0);
-        bool h1 = next_batch(t1);
         const int32_t last = a.n > 0 ? a.n - 1 : 0;
-        int32_t j0 = a.cell_idx[min(max(t0, 0), last)];
-        int32_t j1 = a.cell_idx[min(max(t1, 0), last)];
-        j0 = t0 >= 0 ? j0 : 0;
-        float4 p0 = a.pos[j0];
-        float4 o0 = a.shift ? a.shift[j0] : make_float4(0.f, 0.f, 0.f, 0.f);
-        uint32_t f0 = fbits(a.jprm[j0].w);
+        float4 p0 = a.cell_xs[min(max(t0, 0), last)];
         while (h0) // wave-uniform
         {
-            const bool h2 = next_batch(t2);
-            // batch b+1's positions and b+2's indices in flight
-            j1 = t1 >= 0 ? j1 : 0;
-            const float4 p1 = a.pos[j1];
-            const float4 o1 = a.shift ? a.shift[j1] : make_float4(0.f, 0.f, 0.f, 0.f);
-            const uint32_t f1 = fbits(a.jprm[j1].w);
-            const int32_t j2 = a.cell_idx[min(max(t2, 0), last)];
+            const bool h1 = next_batch(t1);
+            const float4 p1 = a.cell_xs[min(max(t1, 0), last)]; // batch b+1 in flight
             // batch b
             uint32_t m = 0u;
-            const int32_t j = j0;
+            const int32_t j = (int32_t)fbits(p0.w);
             if (t0 >= 0)
             {
-                float4 pj = p0;
-                bool same_sys = true;
-                if (a.shift)
-                { // independent systems never pair, however far they move from their setup places
-                    pj.x += o0.x;
-                    pj.y += o0.y;
-                    pj.z += o0.z;
-                    same_sys = fbits(o0.w) == tag0;
-                }
-                if (same_sys && (a.j_mask == 0u || (f0 & a.j_mask)))
+                const float4 pj = p0;
+                // independent systems never pair, however far they move from their setup places
+                const bool same_sys = !a.shift || fbits(a.shift[j].w) == tag0;
+                if (same_sys)
                 {
 #pragma unroll
                     for (int k = 0; k < CLUSTER; ++k)
@@ -326,13 +295,7 @@ __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
             }
             t0 = t1;
             h0 = h1;
-            t1 = t2;
-            h1 = h2;
-            j0 = j1;
-            j1 = j2;
             p0 = p1;
-            o0 = o1;
-            f0 = f1;
         }
     }
     // zero words up to the next multiple of 16, read unconditionally by the
@@ -359,6 +322,29 @@ __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
         if (count > 0)
             atomicMax(&a.status[3], count);
     }
+}
+
+struct ListSet
+{
+    ListArgs list[MAX_LISTS];
+};
+
+// Blocks of one wave (a slot is free as soon as its cluster is done; clusters'
+// candidates differ by half) where the build is most of the launch, of four
+// where a gated-off launch is: at 31,250 clusters 67 against 77 us a step, at
+// two lists of 12,000 with few rebuilds 4.1 against 2.7 us a launch.
+constexpr int32_t list_waves(int32_t ncl) { return ncl > 16384 ? 1 : 4; }
+
+__global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
+{
+    const ListArgs &a = set.list[blockIdx.y];
+    if (gated_off(a.gate))
+        return;
+    extern __shared__ uint32_t ex_tab[]; // EX_SLOTS per wave
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int32_t ci = blockIdx.x * (int32_t)(blockDim.x >> 6) + wv;
+    if (ci < a.ncl) // wave-uniform
+        cluster_list(a, ci, ex_tab + wv * EX_SLOTS);
 }
 
 // Pair forces of one i-cluster per wave.  A block is 16 list words, two per
@@ -730,7 +716,10 @@ void launch_list_build(const ListArgs *a, int32_t nlists, hipStream_t s)
     for (int32_t l = 0; l < nlists; ++l)
         set.list[l] = a[l];
     if (nlists > 0 && a[0].ncl > 0)
-        k_cluster_list<<<dim3(cluster_blocks(a[0].ncl), nlists), BLOCK, 0, s>>>(set);
+    {
+        const int32_t W = list_waves(a[0].ncl);
+        k_cluster_list<<<dim3((a[0].ncl + W - 1) / W, nlists), 64 * W, W * EX_SLOTS * sizeof(uint32_t), s>>>(set);
+    }
 }
 
 // Pair forces in the queue layout: a block of W waves per cluster
@@ -987,8 +976,8 @@ void launch_pair(const PairArgs &a, int32_t elec_mode, int32_t hydro, int32_t nb
 // ring entry also holds j's adjoint weight; its fourth word is the index j,
 // with bit 31 for a static partner (whose dq takes an atomic).  jprm's flags
 // are not needed beside it: a charge is 0 where the flag is clear.
-// At 40,000 beads 75 -> 52 us a launch, at 2,000 (one wave per cluster left
-// the chip idle) 33 -> 12 us.
+// At 40,000 beads 75 -> 57 us a launch, at 2,000 (one wave per cluster left
+// the chip idle) 33 -> 10 us.
 // ---------------------------------------------------------------------------
 struct AdjLds
 {

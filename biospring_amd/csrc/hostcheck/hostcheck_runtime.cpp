@@ -462,13 +462,41 @@ void launch_cell_sort(const int32_t *cell_of, int32_t n, const int32_t *start, c
 
 // Cluster list build on the CPU with the kernel's semantics (search range =
 // cells covering the cluster bounding box grown by the radius).
+void launch_cell_members(const int32_t *cell_of, int32_t n, const int32_t *start, const int32_t *tmp,
+                         const float4 *pos, const float4 *shift, float4 *xs, int32_t flagged, const int32_t *gate,
+                         hipStream_t s)
+{
+    need(xs, sizeof(float4) * n, "cell_members: xs");
+    if (gated_off(gate))
+        return;
+    std::vector<std::pair<int32_t, int32_t>> m; // (cell, particle)
+    for (int32_t i = 0; i < n; ++i)
+        if (cell_of[i] >= 0)
+            m.push_back({cell_of[i], i});
+    std::sort(m.begin(), m.end());
+    std::vector<int32_t> in(tmp, tmp + m.size());
+    std::sort(in.begin(), in.end());
+    for (size_t t = 0; t < m.size(); ++t)
+    {
+        const int32_t i = m[t].second;
+        if (!std::binary_search(in.begin(), in.end(), i) || (int32_t)t < start[m[t].first] ||
+            (int32_t)t >= start[m[t].first + 1])
+            hc_fail("cell_members: members and starts differ");
+        float4 p = shifted(pos, shift, i);
+        uint32_t w = (uint32_t)i | (flagged && fbits(pos[i].w) != 0u ? 0x80000000u : 0u);
+        std::memcpy(&p.w, &w, 4);
+        xs[t] = p;
+    }
+    (void)s;
+}
+
 static void list_build_one(const ListArgs &a)
 {
     const int64_t nc = (int64_t)a.dims[0] * a.dims[1] * a.dims[2];
     need(a.pos, sizeof(float4) * a.n, "list: pos");
     need(a.jprm, sizeof(float4) * a.n, "list: jprm");
     need(a.cell_start, sizeof(int32_t) * (nc + 1), "list: cell_start");
-    need(a.cell_idx, sizeof(int32_t) * a.n, "list: cell_idx");
+    need(a.cell_xs, sizeof(float4) * a.n, "list: cell_xs");
     need(a.box, sizeof(double) * 6, "list: box");
     need(a.cln, sizeof(int32_t) * a.ncl, "list: cln");
     need(a.status, sizeof(int32_t) * 4, "list: status");
@@ -545,7 +573,7 @@ static void list_build_one(const ListArgs &a)
                         hc_fail("list: cell row out of range");
                     for (int32_t t = a.cell_start[row + clo[0]]; t < a.cell_start[row + chi[0] + 1]; ++t)
                     {
-                        const int32_t j = a.cell_idx[t];
+                        const int32_t j = (int32_t)fbits(a.cell_xs[t].w);
                         if (j < 0 || j >= a.n)
                             hc_fail("list: member out of range");
                         if (a.j_mask && !(fbits(a.jprm[j].w) & a.j_mask))
@@ -1128,7 +1156,7 @@ void launch_topo_springs(const TopoArgs &a, hipStream_t)
     need(a.box, sizeof(double) * 6, "topo: box");
     const int64_t ncells = (int64_t)a.dims[0] * a.dims[1] * a.dims[2];
     need(a.cstart, sizeof(int32_t) * (ncells + 1), "topo: cstart");
-    need(a.cidx, sizeof(int32_t) * n, "topo: cidx");
+    need(a.xs, sizeof(float4) * n, "topo: xs");
     if (a.group)
         need(a.group, sizeof(int32_t) * n, "topo: group");
     if (!(std::sqrt(a.r2max) >= a.rc && std::sqrt(std::nextafter(a.r2max, 0.0)) < a.rc))
@@ -1153,7 +1181,7 @@ void launch_topo_springs(const TopoArgs &a, hipStream_t)
                     const int32_t cell = x + y * a.dims[0] + z * a.dims[0] * a.dims[1];
                     for (int32_t t = a.cstart[cell]; t < a.cstart[cell + 1]; ++t)
                     {
-                        const int32_t j = a.cidx[t];
+                        const int32_t j = (int32_t)(fbits(a.xs[t].w) & 0x7fffffffu);
                         if (j < 0 || j >= n)
                             hc_fail("topo: member index out of range");
                         if (j <= i)
@@ -1410,7 +1438,7 @@ void launch_bin(const BinArgs &a, hipStream_t s)
         if (nc > BIN_CELLS)
             hc_fail("bin: too many cells");
         need(L.start, sizeof(int32_t) * (nc + 1), "bin: start");
-        need(L.idx, sizeof(int32_t) * a.n, "bin: idx");
+        need(L.xs, sizeof(float4) * a.n, "bin: xs");
         std::vector<std::vector<int32_t>> cells((size_t)nc);
         for (int32_t i = 0; i < a.n; ++i)
         {
@@ -1428,7 +1456,11 @@ void launch_bin(const BinArgs &a, hipStream_t s)
         {
             L.start[c] = at;
             for (const int32_t i : cells[(size_t)c])
-                L.idx[at++] = i;
+            {
+                float4 p = shifted(a.pos, a.shift, i);
+                std::memcpy(&p.w, &i, 4);
+                L.xs[at++] = p;
+            }
         }
         L.start[nc] = at;
     }
