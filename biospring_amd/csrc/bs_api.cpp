@@ -2095,7 +2095,7 @@ int do_setup(bs_handle *h)
         HIPCHK(h, hipMemcpyAsync(&dv, diff, sizeof dv, hipMemcpyDeviceToHost, st));
         HIPCHK(h, hipMemcpyAsync(&h->k_uni, h->dsk, sizeof(float), hipMemcpyDeviceToHost, st));
         HIPCHK(h, hipStreamSynchronize(st));
-        h->k_uniform = dv == 0;
+        h->k_uniform = dv == 0 && std::isfinite(h->k_uni); // a null edge's k ext is then 0
     }
     HIPCHK(h, hipStreamSynchronize(st)); // the scratch is freed on return
     rc = upload_positions(h);

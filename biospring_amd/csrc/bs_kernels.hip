@@ -1222,9 +1222,11 @@ __global__ void __launch_bounds__(BLOCK) k_prestep(int32_t *status, int32_t *cou
 // A small system's whole binning in one workgroup: the gate, then (when set)
 // the reference positions, the box and, for each list, cell counts, starts and
 // the members in order.  A gated-off step costs one launch instead of one for
-// the gate and four for each list (1.4 us and a gap of 1 us each), a rebuild
-// about 10 us a list at 9,000 beads, as the separate kernels.  Counts and
-// starts are 16-bit halves of LDS words (n <= BIN_MAX).
+// the gate and four for each list (1.4 us and a gap of 1 us each): with the
+// lists in one launch too, a step of 3,001 beads and two lists takes 16 us
+// instead of 31.  A rebuild is one workgroup's work, which bounds the size:
+// at 9,001 beads, three lists and a rebuild every 10 steps a step still takes
+// 78 us instead of 109.  Counts and starts are 16-bit halves of LDS words.
 constexpr int32_t BIN_BLOCK = 1024;
 constexpr int32_t BIN_EACH = BIN_MAX / BIN_BLOCK; // particles per lane
 
@@ -1450,7 +1452,7 @@ constexpr int32_t EDGE_LDS = 64 * EDGE_KEYS; // longer rows rank from global mem
 // order, then the null edges.  Rows up to EDGE_LDS keep their keys in
 // registers and compare all of them with each partner read from LDS: 3.4
 // reads of four partners per key instead of one 64-bit key per pair (1.81 ->
-// 0.62 ms at 100,000 rows of 182).
+// 0.32 ms at 100,000 rows of 182).
 __global__ void __launch_bounds__(BLOCK) k_edge_sort(const int32_t *ptr, const int32_t *cnt, int32_t n,
                                                      const uint2 *key, const float4 *jprm, const float *sl,
                                                      const float *sk, uint2 *rows, float *rk)
@@ -1529,7 +1531,7 @@ constexpr int32_t EX_STAGE = 2048; // partners of a cluster's rows held in LDS
 // One wave per i-cluster: the words j << 8 | 1 << k of its rows k = 0..7
 // merged in j order (stable in k) from merged[EDGE_PAD ptr[8c]] on, then the
 // number of distinct j.  The binary searches run on a copy of the rows in LDS
-// when they fit (0.96 -> 0.45 ms at 100,000 rows of 182).
+// when they fit (0.96 -> 0.55 ms at 100,000 rows of 182).
 __global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n,
                                                     int32_t ncl, uint32_t *merged, int32_t *ucount)
 {

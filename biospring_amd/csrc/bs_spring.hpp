@@ -126,7 +126,7 @@ template <bool COMP> struct RowSum
     // reciprocal square root and one Newton step (1e-14 relative), so that
     // the extension keeps its accuracy near rest; its seed's argument is kept
     // at or above the smallest normal float (a coincident pair: length 0,
-    // finite factor, no force).
+    // finite factor, no force; closer than 1e-19 A: finite, inexact).
     __device__ void edge(float4 pj, const float4 *plo, uint32_t j, float k, float l0, bool energy, float scale)
     {
         double dx = (double)pj.x - px, dy = (double)pj.y - py, dz = (double)pj.z - pz;

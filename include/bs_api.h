@@ -132,10 +132,10 @@ typedef struct bs_params {
     int32_t graph_steps;
 
     /* Engine option: layout the pair kernels read.  BS_PAIR_QUEUES (the
-       default): the cluster lists read in chunks of at most 128 entries,
-       each entry's j data loaded once into LDS and queued for the
-       particles that see it, so that lanes evaluate listed pairs at the
-       cluster layout's load count.  BS_PAIR_CLUSTERS: the cluster lists in
+       default): the cluster lists read 64 entries at a time, each entry's
+       j data loaded once into an LDS ring and queued for the particles
+       that see it, at places the list build planned, so that lanes
+       evaluate listed pairs at the cluster layout's load count.  BS_PAIR_CLUSTERS: the cluster lists in
        search order, 8 particles x 8 entries per wave, one load of j's data
        serving 8 lanes; lanes of entries a particle does not see stay idle.
        BS_PAIR_ROWS: the cluster lists expanded at each rebuild into one list
