@@ -332,8 +332,11 @@ struct ListSet
 // Blocks of one wave (a slot is free as soon as its cluster is done; clusters'
 // candidates differ by half) where the build is most of the launch, of four
 // where a gated-off launch is: at 31,250 clusters 67 against 77 us a step, at
-// two lists of 12,000 with few rebuilds 4.1 against 2.7 us a launch.
-constexpr int32_t list_waves(int32_t ncl) { return ncl > 16384 ? 1 : 4; }
+// two lists of 12,000 with few rebuilds 4.1 against 2.7 us a launch.  A
+// gated-off launch costs 0.16 ns a block, so above 65,536 clusters (10 us)
+// blocks are of four again: 2.1 M sparse beads, 262,000 clusters, 1.24 ms a
+// step with single waves, 1.18 with four.
+constexpr int32_t list_waves(int32_t ncl) { return ncl > 16384 && ncl <= 65536 ? 1 : 4; }
 
 __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
 {
