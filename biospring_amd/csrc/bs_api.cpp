@@ -419,7 +419,7 @@ int check_device(bs_handle *h)
     for (const auto &l : h->lists)
         if (!l.cl || !l.cln || l.cap <= 0 || l.ncells > h->cell_cap ||
             (h->p.pair_layout == BS_PAIR_ROWS && (!l.rows || !l.rlen || l.rcap < l.cap)) ||
-            (h->p.pair_layout == BS_PAIR_QUEUES && (!l.plan || l.nst * 64 < l.cap)))
+            (h->p.pair_layout == BS_PAIR_QUEUES ? !l.plan || l.nst * 64 < l.cap : l.plan != nullptr))
             return fail(h, BS_ERR_STATE, "internal: neighbour list buffers missing");
     return BS_OK;
 }
@@ -1232,6 +1232,40 @@ void launch_forces(bs_handle *h, bool energy)
             prof_span(h, BS_PROF_PAIR, e1, e2);
         prof_span(h, BS_PROF_SPRING, e2, prof_mark(h));
     }
+}
+
+// Moves a handle that is set up between the cluster and the queue layout: the
+// queue layout's lists have plans, which the kernels follow wherever they are
+// given, the cluster layout's have none.  The lists are rebuilt at the next
+// use.  On an error h keeps the layout it had.
+int set_pair_layout(bs_handle *h, int32_t layout)
+{
+    std::vector<char *> plans;
+    hipError_t e = hipSuccess;
+    if (layout == BS_PAIR_QUEUES)
+        for (const auto &l : h->lists)
+        {
+            plans.push_back(dalloc<char>((size_t)h->ncl * ((l.cap + 63) / 64) * QPLAN_BYTES, e));
+            if (e != hipSuccess)
+                break;
+        }
+    if (e != hipSuccess)
+    {
+        for (char *q : plans)
+            (void)hipFree(q);
+        HIPCHK(h, e);
+    }
+    for (size_t li = 0; li < h->lists.size(); ++li)
+    {
+        List &l = h->lists[li];
+        if (l.plan)
+            (void)hipFree(l.plan);
+        l.plan = plans.empty() ? nullptr : plans[li];
+        l.nst = l.plan ? (l.cap + 63) / 64 : 0;
+    }
+    h->p.pair_layout = layout;
+    launch_fill_i32(h->status + 7, 1, 1, nullptr, h->stream);
+    return BS_OK;
 }
 
 // One step: rebuild gate, (gated) list rebuild, forces and integration.
@@ -3750,10 +3784,11 @@ int bs_autotune(bs_handle *h, int32_t steps, int32_t *group_out, int32_t *graph_
     if (h->p.graph_steps != bgr || h->p.pair_layout != blay)
         drop_graph(h);
     h->p.graph_steps = bgr;
-    if (h->p.pair_layout != BS_PAIR_ROWS && h->p.pair_layout != blay)
-    { // row buffers are sized at setup; the other two read lists in their own order
-        h->p.pair_layout = blay;
-        launch_fill_i32(h->status + 7, 1, 1, nullptr, h->stream);
+    if (h->p.pair_layout != BS_PAIR_ROWS && h->p.pair_layout != blay) // row buffers are sized at setup
+    {
+        rc = set_pair_layout(h, blay);
+        if (rc)
+            return rc;
     }
     if (group_out)
         *group_out = bg;

@@ -201,9 +201,17 @@ hipError_t hipEventCreate(hipEvent_t *e)
     return hipSuccess;
 }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+// Event times: those of hc_event_times in order, then 0.
+static std::vector<float> g_event_ms;
+static size_t g_event_next = 0;
+extern "C" void hc_event_times(const float *ms, int32_t n)
+{
+    g_event_ms.assign(ms, ms + n);
+    g_event_next = 0;
+}
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
 {
-    *ms = 0.0f;
+    *ms = g_event_next < g_event_ms.size() ? g_event_ms[g_event_next++] : 0.0f;
     return hipSuccess;
 }
 hipError_t hipEventDestroy(hipEvent_t e)
@@ -224,6 +232,19 @@ extern "C" int64_t hc_malloc_calls()
 {
     std::lock_guard<std::mutex> lk(mu());
     return g_malloc_calls;
+}
+
+// Launches since the last call, by what they read: [0] pair and adjoint pair
+// kernels on lists alone, [1] the same with plans (queue layout), [2] step
+// kernels, [3] list builds that write plans.
+static int64_t g_launches[4] = {0, 0, 0, 0};
+extern "C" void hc_take_launches(int64_t *out4)
+{
+    for (int k = 0; k < 4; ++k)
+    {
+        out4[k] = g_launches[k];
+        g_launches[k] = 0;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -616,7 +637,10 @@ void launch_list_build(const ListArgs *a, int32_t nlists, hipStream_t)
     if (nlists > MAX_LISTS)
         hc_fail("list: too many lists");
     for (int32_t l = 0; l < nlists; ++l)
+    {
+        g_launches[3] += a[l].plan && !gated_off(a[l].gate) ? 1 : 0;
         list_build_one(a[l]);
+    }
 }
 
 void launch_rows(const uint32_t *cl, const int32_t *cln, int32_t ncl, int32_t cap, uint32_t *rows, int32_t *rlen,
@@ -646,7 +670,7 @@ void launch_rows(const uint32_t *cl, const int32_t *cln, int32_t ncl, int32_t ca
         }
 }
 
-void launch_pair(const PairArgs &a, int32_t, int32_t, int32_t nb, hipStream_t)
+static void pair_work(const PairArgs &a, int32_t nb)
 {
     if (a.rows)
     {
@@ -702,6 +726,12 @@ void launch_pair(const PairArgs &a, int32_t, int32_t, int32_t nb, hipStream_t)
         }
 }
 
+void launch_pair(const PairArgs &a, int32_t, int32_t, int32_t nb, hipStream_t)
+{
+    ++g_launches[a.plan ? 1 : 0];
+    pair_work(a, nb);
+}
+
 // The force rows as EdgeRow reads them: partners in range, the last edge of
 // every row a null edge.
 static void check_rows(const int32_t *ptr, const uint2 *rows, const float *rk, int32_t n, const char *who)
@@ -721,11 +751,12 @@ static void check_rows(const int32_t *ptr, const uint2 *rows, const float *rk, i
     }
 }
 
-void launch_step_kernel(const PairArgs &p, const SpringArgs &a, int32_t em, int32_t h, hipStream_t s)
+void launch_step_kernel(const PairArgs &p, const SpringArgs &a, int32_t, int32_t, hipStream_t s)
 {
     if (!p.plan || !a.integrate || a.probe.state)
         hc_fail("step kernel: queue layout, integration and no probe only");
-    launch_pair(p, em, h, (p.ncl + BLOCK / 64 - 1) / (BLOCK / 64), s);
+    ++g_launches[2];
+    pair_work(p, (p.ncl + BLOCK / 64 - 1) / (BLOCK / 64));
     launch_spring(a, 16, (int32_t)(((int64_t)a.n * 16 + BLOCK - 1) / BLOCK), s);
 }
 
@@ -797,6 +828,9 @@ void launch_spring(const SpringArgs &a, int32_t group, int32_t nb, hipStream_t)
 // be checked.
 void launch_adj_pair(const AdjPairArgs &a, int32_t, int32_t, int32_t nb, hipStream_t)
 {
+    ++g_launches[a.plan ? 1 : 0];
+    if (a.plan)
+        need(a.plan, (size_t)a.ncl * a.nst * QPLAN_BYTES, "adj_pair: plan");
     need(a.pos, sizeof(float4) * a.n, "adj_pair: pos");
     need(a.jprm, sizeof(float4) * a.n, "adj_pair: jprm");
     need(a.cln, sizeof(int32_t) * a.ncl, "adj_pair: cln");

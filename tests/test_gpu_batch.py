@@ -6,7 +6,7 @@ import sys
 import numpy as np
 import pytest
 
-from biospring_amd import workloads
+from biospring_amd import _abi, workloads
 from biospring_amd.network import SpringNetwork
 from oracle import pyoracle as po
 from tests.parity import ENERGY_RTOL, FORCE_RTOL, energy_error, force_errors
@@ -90,6 +90,38 @@ def test_autotune_picks_a_valid_configuration():
     xa, _ = a.getState()
     xb, _ = b.getState()
     assert np.abs(xa - xb).max() <= 1e-4
+
+
+@pytest.mark.parametrize("layout", [_abi.PAIR_CLUSTERS, _abi.PAIR_QUEUES])
+def test_autotuned_handle_runs_from_either_layout(layout):
+    """A handle set up in one pair layout runs, gives forces and gradients in
+    the layout that autotune chose, as one set up in that layout does.  The
+    same kernels on the same lists; a tuned lane count sums a row's springs in
+    another order, in FP64, rounded once to FP32: 6e-8 a step of the largest
+    velocity change, 25 steps."""
+    s = workloads.generate(1, seed=8, n=6001)
+    p = s.params.copy()
+    p.pair_layout = layout
+    a = SpringNetwork.from_system(s, params=p)
+    a.setup()
+    p = s.params.copy()
+    _, p.graph_steps, p.pair_layout = a.autotune(10)
+    _log(f"autotune: layout {layout} -> {p.pair_layout}")
+    b = SpringNetwork.from_system(s, params=p)
+    a.setState(*b.getState())
+    for net in (a, b):
+        net.run(25)
+    (xa, va), (xb, vb) = a.getState(), b.getState()
+    assert np.abs(va - vb).max() <= 25 * 6e-8 * np.abs(vb).max()
+    assert np.abs(xa - xb).max() <= 25 * 6e-8 * np.abs(xb).max()
+    a.setState(xb, vb)
+    b.setState(xb, vb)
+    fa, ea = a.computeForces()
+    fb, eb = b.computeForces()
+    assert np.abs(fa - fb).max() <= 2 * 6e-8 * np.abs(fb).max() and np.allclose(ea, eb, rtol=1e-9)
+    ga, gb = a.adjoint(5, s.x, 0), b.adjoint(5, s.x, 0)
+    for u, v in zip(ga[1:], gb[1:]):
+        assert np.abs(u - v).max() <= 1e-6 * np.abs(v).max()
 
 
 def test_systems_never_pair_after_moving_onto_each_other():

@@ -406,3 +406,56 @@ def test_overflow_lengthens_lists_and_resumes(hostcheck_lib):
         print("ok", cap0, cnt["list_cap"])
         ''', hostcheck_lib)
     assert "ok" in out
+
+
+def test_autotune_layout_switch(hostcheck_lib):
+    """The pair layout that autotune settles on is the one that runs, with its
+    buffers in place, in both directions: a clock makes either layout the
+    faster, then steps (past an overflow too), forces and a gradient are
+    asked for.  Only the queue layout builds plans and launches the step
+    kernel."""
+    out = _run('''
+        s = workloads.generate(1, seed=3, n=3000)
+        base = L.hc_live_allocations()
+        C, Q = _abi.PAIR_CLUSTERS, _abi.PAIR_QUEUES
+        L.hc_event_times.argtypes = [ctypes.POINTER(ctypes.c_float), ctypes.c_int32]
+        def launches():
+            v = (ctypes.c_int64 * 4)()
+            L.hc_take_launches(v)
+            return dict(zip(("plain", "planned", "step", "plans"), v))
+        def calls(net, layout):
+            launches()
+            net.run(3)
+            a = launches()
+            net.setState(*net.getState())    # the lists are built anew
+            net.computeForces()
+            net.adjoint(4, s.x, 2)
+            b = launches()
+            if layout == Q:
+                assert a["step"] == 3 and a["plain"] == 0, a
+                assert b["step"] and b["planned"] and b["plans"] and not b["plain"], b
+            else:
+                assert a["plain"] >= 3 and not (a["step"] or a["planned"] or a["plans"]), a
+                assert b["plain"] and not (b["step"] or b["planned"] or b["plans"]), b
+        for start, wins in ((C, Q), (Q, C), (C, C), (Q, Q)):
+            for cutoffs in ((12.0, 12.0), (6.0, 9.0)):  # one list, two lists
+                p = s.params.copy()
+                p.pair_layout, p.spring_enable = start, 1
+                p.steric_cutoff, p.electrostatic_cutoff = cutoffs
+                net = SpringNetwork.from_system(s, params=p, library=L)
+                net.setup()
+                ms = (ctypes.c_float * 2)(*((1.0, 2.0) if wins == C else (2.0, 1.0)))
+                L.hc_event_times(ms, 2)
+                assert net.autotune(2)[2] == wins
+                calls(net, wins)
+                x = s.x.reshape(-1, 3).astype(np.float64)
+                c = x.mean(axis=0)
+                cap = net.counters()["list_cap"]
+                net.setState(((x - c) * 0.6 + c).astype(np.float32), np.zeros((s.n, 3), np.float32))
+                net.run(3)                       # overflows: the lists grow
+                assert net.counters()["list_cap"] > cap
+                calls(net, wins)
+                net.close()
+        print("switched, leak", L.hc_live_allocations() - base)
+        ''', hostcheck_lib)
+    assert "switched, leak 0" in out, out
