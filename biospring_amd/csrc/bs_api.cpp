@@ -1451,91 +1451,43 @@ void springs_host_changed(bs_handle *h)
     h->sp_dev = false;
 }
 
-// The CSR edge on which the adjoint sweep accumulates each spring's
-// gradients: the edge of the dynamic row that owns it (a static partner, or
-// else the larger index is the partner; the rule of k_adj_spring), -1 when
-// both ends are static.  Built once per setup.
+// The slot in which the adjoint sweep accumulates each spring's gradients:
+// that of its edge in the dynamic row that owns it (a static partner, or else
+// the larger index is the partner; the rule of k_adj_spring), -1 when both
+// ends are static.  Built once per setup, from the rows and the table on the
+// device.
 int build_spring_owners(bs_handle *h)
 {
-    const int64_t n = h->n, m = h->nsp, E = h->nunits * EDGE_PAD;
+    const int64_t n = h->n, m = h->nsp;
     if (h->nslots >= 0 || m == 0)
         return BS_OK;
-    const int hrc = springs_host(h);
-    if (hrc)
-        return hrc;
-    std::vector<int32_t> hu((size_t)n + 1);
-    std::vector<uint2> he((size_t)std::max<int64_t>(E, 1));
-    HIPCHK(h, hipMemcpy(hu.data(), h->sp_ptr, sizeof(int32_t) * (n + 1), hipMemcpyDeviceToHost));
-    if (E > 0)
-        HIPCHK(h, hipMemcpy(he.data(), h->sp_e, sizeof(uint2) * E, hipMemcpyDeviceToHost));
-    // partners of row i's edges: hj[hp[i]] to hj[hp[i + 1]], without the null
-    // edges (partner i) that end a row
-    std::vector<int32_t> hp((size_t)n + 1, 0), hj, own((size_t)m, -1);
-    hj.reserve((size_t)std::max<int64_t>(h->nedges, 1));
-    for (int64_t i = 0; i < n; ++i)
-    {
-        for (int64_t t = (int64_t)hu[(size_t)i] * EDGE_PAD;
-             t < (int64_t)hu[(size_t)i + 1] * EDGE_PAD && he[(size_t)t].x != (uint32_t)i; ++t)
-            hj.push_back((int32_t)he[(size_t)t].x);
-        hp[(size_t)i + 1] = (int32_t)hj.size();
-    }
-    // a slot per owned edge: in a moving row, the edges to static partners
-    // and to partners of higher index, numbered in edge order
-    std::vector<int32_t> ord(std::max<size_t>(hj.size(), 1), -1), sp((size_t)n + 1, 0);
-    for (int64_t i = 0; i < n; ++i)
-    {
-        int32_t c = sp[(size_t)i];
-        if (!(h->flags[(size_t)h->perm[(size_t)i]] & BS_FLAG_STATIC))
-            for (int32_t t = hp[(size_t)i]; t < hp[(size_t)i + 1]; ++t)
-                if (hj[(size_t)t] < 0 || hj[(size_t)t] > (int32_t)i)
-                    ord[(size_t)t] = c++;
-        sp[(size_t)i + 1] = c;
-    }
-    const int64_t ns = sp[(size_t)n];
-    // each spring with a moving end finds its edge in the owning row (the
-    // table holds no repeated pair: every way in drops repeats)
-#pragma omp parallel for schedule(static, 4096)
-    for (int64_t s = 0; s < m; ++s)
-    {
-        int32_t a = h->iperm[h->s1[(size_t)s]], b = h->iperm[h->s2[(size_t)s]];
-        const bool sa = (h->flags[h->s1[(size_t)s]] & BS_FLAG_STATIC) != 0;
-        const bool sb = (h->flags[h->s2[(size_t)s]] & BS_FLAG_STATIC) != 0;
-        if ((sa && sb) || a == b)
-            continue;
-        if (sa || (!sb && b < a))
-            std::swap(a, b); // row a owns the edge to b
-        int32_t lo = hp[(size_t)a], hi = hp[(size_t)a + 1];
-        while (lo < hi)
-        {
-            const int32_t mid = (lo + hi) >> 1;
-            if ((hj[(size_t)mid] & 0x7fffffff) < b)
-                lo = mid + 1;
-            else
-                hi = mid;
-        }
-        if (lo < hp[(size_t)a + 1] && (hj[(size_t)lo] & 0x7fffffff) == b)
-            own[(size_t)s] = lo;
-    }
-    std::vector<int32_t> so((size_t)m, -1);
-    std::vector<char> used((size_t)std::max<int64_t>(ns, 1), 0);
-    for (int64_t s = 0; s < m; ++s)
-    {
-        const int32_t e = own[(size_t)s];
-        if (e < 0)
-            continue;
-        const int32_t r = ord[(size_t)e];
-        if (r < 0 || used[(size_t)r])
-            return fail(h, BS_ERR_STATE, "internal: spring %lld has no free slot", (long long)s);
-        used[(size_t)r] = 1;
-        so[(size_t)s] = r;
-    }
     hipError_t e = hipSuccess;
-    h->slot_ptr = dalloc<int32_t>((size_t)n + 1, e);
+    Scratch S;
+    int32_t *iperm = S.get<int32_t>((size_t)n, e);
     HIPCHK(h, e);
-    h->slot_of = dalloc<int32_t>((size_t)m, e);
+    int32_t *owned = S.get<int32_t>((size_t)n, e);
     HIPCHK(h, e);
-    HIPCHK(h, hipMemcpy(h->slot_ptr, sp.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->slot_of, so.data(), sizeof(int32_t) * m, hipMemcpyHostToDevice));
+    int32_t *len = S.get<int32_t>((size_t)n, e);
+    HIPCHK(h, e);
+    if (!h->slot_ptr)
+    {
+        h->slot_ptr = dalloc<int32_t>((size_t)n + 1, e);
+        HIPCHK(h, e);
+    }
+    if (!h->slot_of)
+    {
+        h->slot_of = dalloc<int32_t>((size_t)m, e);
+        HIPCHK(h, e);
+    }
+    hipStream_t st = h->stream;
+    int32_t ns = 0;
+    HIPCHK(h, hipMemcpyAsync(iperm, h->iperm.data(), sizeof(int32_t) * n, hipMemcpyHostToDevice, st));
+    launch_slot_rows(h->sp_ptr, h->sp_e, h->jprm, (int32_t)n, owned, len, st);
+    launch_scan(owned, h->slot_ptr, (int32_t)n, nullptr, st);
+    launch_slot_find(h->dsa, h->dsb, m, iperm, h->jprm, h->sp_ptr, h->sp_e, len, h->slot_ptr, (int32_t)n, h->slot_of,
+                     st);
+    HIPCHK(h, hipMemcpyAsync(&ns, h->slot_ptr + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    HIPCHK(h, hipStreamSynchronize(st)); // also: the scratch is freed on return
     h->nslots = ns;
     return BS_OK;
 }

@@ -423,6 +423,15 @@ void launch_unperm_f64(const double *in, const int32_t *perm, int32_t n, double 
 // owning CSR edge) dk[r] += dke[r] in FP64 and the FP32 sum is cleared;
 // likewise dl0.
 void launch_spring_grads(float *dke, float *dle, int64_t nslots, double *dk, double *dl0, hipStream_t s);
+// Gradient slots: one per edge that its row owns (a moving row's edges to
+// static partners and to partners of higher index), numbered in edge order.
+// The owned and the real (not null) edges of each row; then, with the rows'
+// first slots in slot_ptr, every spring's slot, -1 when both ends are static.
+void launch_slot_rows(const int32_t *ptr, const uint2 *rows, const float4 *jprm, int32_t n, int32_t *owned,
+                      int32_t *len, hipStream_t s);
+void launch_slot_find(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const float4 *jprm,
+                      const int32_t *ptr, const uint2 *rows, const int32_t *len, const int32_t *slot_ptr, int32_t n,
+                      int32_t *slot_of, hipStream_t s);
 // Per spring from per slot: out[s] = slot_of[s] >= 0 ? v[slot_of[s]] : 0.
 void launch_spring_out(const int32_t *slot_of, int64_t m, const double *dk, const double *dl0, double *outk,
                        double *outl, hipStream_t s);

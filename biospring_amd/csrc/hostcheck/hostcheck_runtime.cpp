@@ -900,6 +900,64 @@ void launch_adj_spring(const AdjSpringArgs &a, int32_t group, int32_t nb, hipStr
     }
 }
 
+void launch_slot_rows(const int32_t *ptr, const uint2 *rows, const float4 *jprm, int32_t n, int32_t *owned,
+                      int32_t *len, hipStream_t)
+{
+    need(ptr, sizeof(int32_t) * ((size_t)n + 1), "slot_rows: ptr");
+    need(jprm, sizeof(float4) * (size_t)n, "slot_rows: jprm");
+    need(owned, sizeof(int32_t) * (size_t)n, "slot_rows: owned");
+    need(len, sizeof(int32_t) * (size_t)n, "slot_rows: len");
+    check_rows(ptr, rows, nullptr, n, "slot_rows");
+    for (int32_t i = 0; i < n; ++i)
+    {
+        const bool dyn = !(fbits(jprm[i].w) & PF_STATIC);
+        owned[i] = len[i] = 0;
+        for (size_t e = (size_t)ptr[i] * EDGE_PAD; e < (size_t)ptr[i + 1] * EDGE_PAD; ++e)
+        {
+            const int32_t j = (int32_t)rows[e].x;
+            len[i] += j != i;
+            owned[i] += dyn && j != i && (j < 0 || j > i);
+        }
+    }
+}
+
+// Every slot is taken once, by the spring whose edge it counts.
+void launch_slot_find(const uint32_t *sa, const uint32_t *sb, int64_t m, const int32_t *iperm, const float4 *jprm,
+                      const int32_t *ptr, const uint2 *rows, const int32_t *len, const int32_t *slot_ptr, int32_t n,
+                      int32_t *slot_of, hipStream_t)
+{
+    need(sa, sizeof(uint32_t) * (size_t)m, "slot_find: sa");
+    need(sb, sizeof(uint32_t) * (size_t)m, "slot_find: sb");
+    need(iperm, sizeof(int32_t) * (size_t)n, "slot_find: iperm");
+    need(jprm, sizeof(float4) * (size_t)n, "slot_find: jprm");
+    need(len, sizeof(int32_t) * (size_t)n, "slot_find: len");
+    need(slot_ptr, sizeof(int32_t) * ((size_t)n + 1), "slot_find: slot_ptr");
+    need(slot_of, sizeof(int32_t) * (size_t)m, "slot_find: slot_of");
+    check_rows(ptr, rows, nullptr, n, "slot_find");
+    std::vector<char> used((size_t)slot_ptr[n], 0);
+    for (int64_t s = 0; s < m; ++s)
+    {
+        int32_t a = iperm[sa[s]], b = iperm[sb[s]];
+        const bool fa = fbits(jprm[a].w) & PF_STATIC, fb = fbits(jprm[b].w) & PF_STATIC;
+        slot_of[s] = -1;
+        if (fa && fb)
+            continue;
+        if (fa || (!fb && b < a))
+            std::swap(a, b);
+        int32_t slot = slot_ptr[a];
+        for (int32_t t = 0; t < len[a]; ++t)
+        {
+            const int32_t j = (int32_t)rows[(size_t)ptr[a] * EDGE_PAD + t].x;
+            if ((j & 0x7fffffff) == b)
+                slot_of[s] = slot;
+            slot += j < 0 || j > a;
+        }
+        if (slot != slot_ptr[a + 1] || slot_of[s] < 0 || used[(size_t)slot_of[s]])
+            hc_fail("slot_find: a spring without a slot of its own");
+        used[(size_t)slot_of[s]] = 1;
+    }
+}
+
 void launch_spring_grads(float *dke, float *dle, int64_t ns, double *dk, double *dl0, hipStream_t)
 {
     need(dke, sizeof(float) * ns, "spring_grads: dke");

@@ -225,3 +225,40 @@ def test_torch_wrapper_refuses_a_replaced_record():
     q = torch.tensor(s.charge.astype(np.float64), requires_grad=True)
     with pytest.raises(ValueError):
         final_positions(net, s, q=q, nsteps=2)
+
+
+@pytest.mark.parametrize("spokes", [1, 7, 8, 63, 64, 65, 300, 700])
+def test_every_spring_gets_its_own_gradient(spokes):
+    """One step of hubs and spokes, some of them fixed, springs given in a
+    shuffled order and direction: each spring's gradients are a closed form of
+    its own ends.  They are summed once, in FP32 (6e-8); x_1 is the engine's."""
+    rng = np.random.default_rng(spokes)
+    n = 3 * (spokes + 1)
+    x = (rng.normal(size=(n, 3)) * 8.0).astype(np.float32)
+    a = np.repeat(np.arange(3), spokes)
+    b = 3 + np.arange(3 * spokes)
+    ring = np.stack([b, np.roll(b, 1)], 1) if spokes > 1 else np.zeros((0, 2), int)
+    ends = np.concatenate([np.stack([a, b], 1), ring, [[0, 1], [1, 2], [0, 2]]])
+    ends = ends[rng.permutation(len(ends))]
+    flip = rng.random(len(ends)) < 0.5
+    ends[flip] = ends[flip][:, ::-1]
+    ends = rng.permutation(n)[ends]  # hubs anywhere in the index range
+    fixed = (rng.random(n) < 0.3).astype(np.uint8)
+    l0 = rng.uniform(1.0, 6.0, len(ends)).astype(np.float32)
+    k = rng.uniform(0.1, 1.0, len(ends)).astype(np.float32)
+    p = _abi.default_params()
+    p.spring_enable, p.viscosity_enable, p.timestep = 1, 0, 1.0
+    net = SpringNetwork(p)
+    net.setParticles(x, flags=fixed * np.uint8(_abi.FLAG_STATIC))
+    net.setSprings(ends[:, 0].astype(np.uint32), ends[:, 1].astype(np.uint32), l0, k)
+    y = (x + rng.normal(size=x.shape)).astype(np.float32)
+    _, dk, dl, _ = net.adjoint(1, y, 0)
+    x1, _ = net.getState()
+    moves = (1 - fixed)[:, None]
+    g = 2.0 / n * (x1.astype(np.float64) - y) * moves
+    d = x[ends[:, 1]].astype(np.float64) - x[ends[:, 0]]
+    r = np.linalg.norm(d, axis=1)
+    c = 1.0e3 / 6.02214169e23 * 1.0e10 * (1.0e10 / 1.66054e-27 * 1e-30)
+    along = ((g[ends[:, 0]] - g[ends[:, 1]]) * d).sum(1) / r * c  # dL per unit of the pull on the first end
+    for got, want in ((dk, along * (r - l0)), (dl, -along * k.astype(np.float64))):
+        assert np.abs(got - want).max() <= 4e-7 * np.abs(want).max()
