@@ -158,7 +158,8 @@ def pmc_summary(fetch_dir, fetch_copy_dir, write_dir, write_copy_dir):
     sw = COPY_BYTES / (cw * 1024.0)
     fm = _counter_means(fetch_dir, "FETCH_SIZE")
     wm = _counter_means(write_dir, "WRITE_SIZE")
-    for name, keys in (("pair", ("k_pair_q<1, 2, 0, false>", "k_pair<1, 2, 0, false>")),
+    for name, keys in (("step", ("k_step<1, 2, 0, false, false>",)),
+                       ("pair", ("k_pair_q<1, 2, 0, false>", "k_pair<1, 2, 0, false>")),
                        ("spring_integrate", ("k_spring<16, true, false",)), ("cluster_list", ("k_cluster_list",))):
         f = next((v for v in (pick(fm, k) for k in keys) if v is not None), None)
         w = next((v for v in (pick(wm, k) for k in keys) if v is not None), None)
@@ -185,7 +186,8 @@ def pmc_valu_summary(valu_dir, command):
     launch = 64 lanes x (ADD + MUL + 2 FMA + TRANS) wave instructions."""
     out = {"command": command, "flop_rule": "64 lanes x (ADD + MUL + 2 FMA + TRANS) wave instructions, per type"}
     means = {c: _counter_means(valu_dir, c) for c in VALU_COUNTERS}
-    for name, keys in (("pair", ("k_pair_q<1, 2, 0, false>", "k_pair<1, 2, 0, false>")),
+    for name, keys in (("step", ("k_step<1, 2, 0, false, false>",)),
+                       ("pair", ("k_pair_q<1, 2, 0, false>", "k_pair<1, 2, 0, false>")),
                        ("spring_integrate", ("k_spring<16, true, false",))):
         row = {}
         for c in VALU_COUNTERS:
@@ -309,26 +311,40 @@ def main():
     k_uniform = bool(s.m > 0 and np.all(s.k.view(np.uint32) == s.k.view(np.uint32)[0]))
     b_alg = 4 * (n + 1) + (8 if k_uniform else 12) * edges + 64 * n
     f_alg = PAIR_FLOP * pairs_unique
-    spring_gbs = b_alg / (spring_ms * 1e-3) / 1e9
-    pair_tflops = f_alg / (pair_ms * 1e-3) / 1e12
-    kernels = {
-        "spring_integrate": {"avg_ms": spring_ms, "bound": "hbm", "achieved": spring_gbs, "peak": HBM_PEAK_GBS,
-                             "unit": "GB/s", "frac": spring_gbs / HBM_PEAK_GBS, "alg_bytes": b_alg,
-                             "uniform_stiffness": k_uniform},
-        "pair": {"avg_ms": pair_ms, "bound": "valu", "achieved": pair_tflops, "peak": FP32_PEAK_TFLOPS,
-                 "unit": "TFLOP/s", "frac": pair_tflops / FP32_PEAK_TFLOPS, "alg_flops": f_alg,
-                 "note": "compute-bound FP32/FP64 vector ALU work priced against the FP32 peak"},
-        "rebuild_chain_avg_ms_per_step": rebuild_ms,
-    }
-    dom = "pair" if pair_ms >= spring_ms else "spring_integrate"
+
+    def hbm(ms):
+        g = b_alg / (ms * 1e-3) / 1e9
+        return {"avg_ms": ms, "bound": "hbm", "achieved": g, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": g / HBM_PEAK_GBS, "alg_bytes": b_alg, "uniform_stiffness": k_uniform}
+
+    def valu(ms):
+        f = f_alg / (ms * 1e-3) / 1e12
+        return {"avg_ms": ms, "bound": "valu", "achieved": f, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
+                "frac": f / FP32_PEAK_TFLOPS, "alg_flops": f_alg,
+                "note": "compute-bound FP32/FP64 vector ALU work priced against the FP32 peak"}
+
+    layout = int(s.params.pair_layout) if tuned is None else tuned[2]
+    if layout == _abi.PAIR_QUEUES:
+        # one kernel takes the (last) list's pairs, the springs and the
+        # integrator; the pairs' operations and the springs' bytes are both its
+        step_ms = pair_ms + spring_ms
+        kernels = {"step": valu(step_ms)}
+        mem = hbm(step_ms)
+        kernels["step"].update({"alg_bytes": b_alg, "uniform_stiffness": k_uniform, "hbm_gbs": mem["achieved"],
+                                "hbm_frac": mem["frac"], "earlier_lists_pair_ms": pair_ms})
+        dom = "step"
+    else:
+        kernels = {"spring_integrate": hbm(spring_ms), "pair": valu(pair_ms)}
+        dom = "pair" if pair_ms >= spring_ms else "spring_integrate"
+    kernels["rebuild_chain_avg_ms_per_step"] = rebuild_ms
     traffic = None
     tfile = os.path.join(ROOT, "profiles", "pmc_traffic.json")
     if os.path.exists(tfile) and args.workload == 1 and n == 250000:
         # HBM bytes per launch from the committed FETCH_SIZE / WRITE_SIZE runs
         with open(tfile) as fh:
             tt = json.load(fh)
-        for name in ("pair", "spring_integrate"):
-            if name in tt:
+        for name in ("step", "pair", "spring_integrate"):
+            if name in tt and name in kernels:
                 kernels[name]["traffic_bytes"] = tt[name]["bytes"]
         traffic = tt.get(dom, {}).get("bytes")
     vfile = os.path.join(ROOT, "profiles", "pmc_valu.json")
@@ -337,8 +353,8 @@ def main():
         # over this run's average launch time
         with open(vfile) as fh:
             vv = json.load(fh)
-        for name in ("pair", "spring_integrate"):
-            if name in vv:
+        for name in ("step", "pair", "spring_integrate"):
+            if name in vv and name in kernels:
                 ms = kernels[name]["avg_ms"]
                 e32, e64 = vv[name]["executed_fp32_flop"], vv[name]["executed_fp64_flop"]
                 kernels[name]["executed_valu"] = {"fp32_tflops": e32 / (ms * 1e-3) / 1e12,
@@ -357,7 +373,7 @@ def main():
                    "systems": 1 if off is None else len(off) - 1,
                    "graph_steps": int(s.params.graph_steps) if tuned is None else tuned[1],
                    "spring_lanes": None if tuned is None else tuned[0],
-                   "pair_layout": int(s.params.pair_layout) if tuned is None else tuned[2], "springs": s.m, "directed_edges": edges, "unique_pairs": pairs_unique,
+                   "pair_layout": layout, "springs": s.m, "directed_edges": edges, "unique_pairs": pairs_unique,
                    "seed": args.seed, "digest": s.digest(),
                    "rebuilds_in_timed_region": cnt1["rebuilds"] - cnt0["rebuilds"],
                    "list_capacity": cnt1["list_cap"]},
@@ -661,8 +677,8 @@ def adjoint_leg(seed=1, n=0, T=200, K=20, warmup=5, fp64=True, cpu=True, check_n
     }
     for k in kernels.values():
         k["frac"] = k["achieved"] / k["peak"]
-    kernels["forward_pair_avg_ms"] = prof["pair"]["ms"] / max(prof["pair"]["launches"], 1)
-    kernels["forward_spring_avg_ms"] = prof["spring"]["ms"] / max(prof["spring"]["launches"], 1)
+    # pairs, springs and integrator (one kernel in the queue layout)
+    kernels["forward_step_avg_ms"] = sum(prof[c]["ms"] for c in ("pair", "spring")) / max(prof["spring"]["launches"], 1)
     kernels["rebuild_avg_ms"] = prof["rebuild"]["ms"] / max(prof["rebuild"]["launches"], 1)
     dom = "adj_pair" if ap_ms >= as_ms else "adj_spring"
     d = kernels[dom]

@@ -1206,29 +1206,26 @@ int regrow_lists(bs_handle *h)
 
 // A step's forces and integration, lists in place: the pair forces, springs,
 // rigid bodies and probe.  In the queue layout the last list's pairs, the
-// springs and the integrator are one kernel; the probe's block sums and a
-// profiled call's timing of the two parts need them apart.
+// springs and the integrator are one kernel; the probe's block sums need them
+// apart.  Event timing changes nothing that is launched.
 void launch_forces(bs_handle *h, bool energy)
 {
     const size_t nl = h->lists.size();
-    if (nl > 0 && h->p.pair_layout == BS_PAIR_QUEUES && !h->p.probe_enable && !h->prof)
-    {
-        const List &l = h->lists[nl - 1];
-        launch_pairs(h, energy, nl - 1);
-        launch_step_kernel(pair_args(h, nl - 1, energy), spring_args(h, true, energy), elec_mode(h, l),
-                           (l.terms & TERM_HYDRO) ? 1 : 0, h->stream);
-        launch_bodies(h);
-        return;
-    }
+    const bool fused = nl > 0 && h->p.pair_layout == BS_PAIR_QUEUES && !h->p.probe_enable;
+    const size_t apart = fused ? nl - 1 : nl; // lists with a pair kernel of their own
     const size_t e1 = h->prof ? prof_mark(h) : SIZE_MAX;
-    launch_pairs(h, energy, nl);
-    const size_t e2 = h->prof ? prof_mark(h) : SIZE_MAX;
-    launch_springs(h, true, energy);
+    launch_pairs(h, energy, apart);
+    const size_t e2 = h->prof && apart > 0 ? prof_mark(h) : e1;
+    if (fused)
+        launch_step_kernel(pair_args(h, apart, energy), spring_args(h, true, energy), elec_mode(h, h->lists[apart]),
+                           (h->lists[apart].terms & TERM_HYDRO) ? 1 : 0, h->stream);
+    else
+        launch_springs(h, true, energy);
     launch_bodies(h);
     launch_probe_step(h, true);
     if (h->prof)
     {
-        if (nl > 0)
+        if (apart > 0)
             prof_span(h, BS_PROF_PAIR, e1, e2);
         prof_span(h, BS_PROF_SPRING, e2, prof_mark(h));
     }

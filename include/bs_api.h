@@ -293,10 +293,14 @@ int bs_get_counters(const bs_handle *h, int64_t *out6);
 
 /* ---- profiling --------------------------------------------------------------- */
 
-/* Kernel classes timed with HIP events on the handle's stream. */
+/* Kernel classes timed with HIP events on the handle's stream.  A step in the
+ * queue layout (BS_PAIR_QUEUES, no probe) takes the last list's pairs, the
+ * springs and the integrator in one kernel: its time counts under
+ * BS_PROF_SPRING, and BS_PROF_PAIR has the earlier lists' kernels alone (no
+ * launches with one list). */
 #define BS_PROF_REBUILD 0  /* neighbour-upkeep chain (box, binning, list build) */
-#define BS_PROF_PAIR    1  /* non-bonded pair kernels */
-#define BS_PROF_SPRING  2  /* spring gather + integrator (or force epilogue) */
+#define BS_PROF_PAIR    1  /* non-bonded pair kernels of their own */
+#define BS_PROF_SPRING  2  /* spring gather + integrator, with the last list's pairs in the queue layout */
 #define BS_PROF_ADJ_PAIR   3  /* bs_adjoint: pair part of H w and dL/dq */
 #define BS_PROF_ADJ_SPRING 4  /* bs_adjoint: spring part, parameter gradients, reverse update */
 #define BS_PROF_TOPO_COUNT 5  /* bs_springs_from_cutoff: binning and the count pass */
@@ -304,7 +308,8 @@ int bs_get_counters(const bs_handle *h, int64_t *out6);
 #define BS_PROF_NUM     7
 
 /* Turns per-kernel-class event timing of bs_step and bs_adjoint on (1) or off
- * (0) and resets the totals.  Counterpart of the reference's wall-clock timeit::Profiler
+ * (0) and resets the totals.  The steps' kernels and results are the same
+ * either way; a graph (graph_steps) is not replayed while it is on.  Counterpart of the reference's wall-clock timeit::Profiler
  * (src/timeit.hpp:16-168; "Average framerate", SpringNetwork.cpp:305-308). */
 int bs_profile(bs_handle *h, int32_t enable);
 

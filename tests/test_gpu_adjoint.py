@@ -262,3 +262,23 @@ def test_every_spring_gets_its_own_gradient(spokes):
     along = ((g[ends[:, 0]] - g[ends[:, 1]]) * d).sum(1) / r * c  # dL per unit of the pull on the first end
     for got, want in ((dk, along * (r - l0)), (dl, -along * k.astype(np.float64))):
         assert np.abs(got - want).max() <= 4e-7 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("recorded,swept", [(False, True), (True, False)])
+def test_event_timing_changes_no_bit(recorded, swept):
+    """A run, and a record swept with event timing switched in between (its
+    segments are recomputed on the recorded rebuilds), against the same
+    without timing."""
+    s = workloads.generate(1, seed=16, n=3000)
+    y = _target(s)
+    got = []
+    for rec, swp in ((False, False), (recorded, swept)):
+        net = SpringNetwork.from_system(s)
+        net.profile(rec)
+        net.run(15)
+        net.adjointForward(16, 5)
+        x, v = net.getState()
+        net.profile(swp)
+        got.append((x, v) + tuple(net.adjointBackward(2.0 * (x.astype(np.float64) - y) / s.n)))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

@@ -459,3 +459,38 @@ def test_autotune_layout_switch(hostcheck_lib):
         print("switched, leak", L.hc_live_allocations() - base)
         ''', hostcheck_lib)
     assert "switched, leak 0" in out, out
+
+
+def test_profiling_leaves_the_launches_alone(hostcheck_lib):
+    """Event timing on or off, a step and a gradient launch the same kernels:
+    the step kernel in the queue layout, whose time is the spring class's."""
+    out = _run('''
+        s = workloads.generate(1, seed=3, n=3000)
+        def launches():
+            v = (ctypes.c_int64 * 4)()
+            L.hc_take_launches(v)
+            return list(v)
+        for layout in (_abi.PAIR_QUEUES, _abi.PAIR_CLUSTERS):
+            for cutoffs in ((12.0, 12.0), (6.0, 9.0)):
+                p = s.params.copy()
+                p.pair_layout = layout
+                p.steric_cutoff, p.electrostatic_cutoff = cutoffs
+                got = []
+                for on in (False, True):
+                    net = SpringNetwork.from_system(s, params=p, library=L)
+                    net.setup()
+                    net.profile(on)
+                    launches()
+                    net.run(4)
+                    prof = net.getProfile()
+                    net.computeForces()
+                    net.adjoint(6, s.x, 2)
+                    got.append(launches())
+                    assert prof["spring"]["launches"] == (4 if on else 0), prof
+                    own = layout == _abi.PAIR_CLUSTERS or cutoffs[0] != cutoffs[1]
+                    assert prof["pair"]["launches"] == (4 if on and own else 0), prof
+                    net.close()
+                assert got[0] == got[1], (layout, cutoffs, got)
+        print("same launches")
+        ''', hostcheck_lib)
+    assert "same launches" in out, out
