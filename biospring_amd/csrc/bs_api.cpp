@@ -1204,14 +1204,19 @@ int regrow_lists(bs_handle *h)
     return BS_OK;
 }
 
+// Whether a step takes the last list's pairs, the springs and the integrator
+// in one kernel (the probe's block sums need them apart).
+bool step_fused(const bs_handle *h, int32_t layout)
+{
+    return !h->lists.empty() && layout == BS_PAIR_QUEUES && !h->p.probe_enable;
+}
+
 // A step's forces and integration, lists in place: the pair forces, springs,
-// rigid bodies and probe.  In the queue layout the last list's pairs, the
-// springs and the integrator are one kernel; the probe's block sums need them
-// apart.  Event timing changes nothing that is launched.
+// rigid bodies and probe.  Event timing changes nothing that is launched.
 void launch_forces(bs_handle *h, bool energy)
 {
     const size_t nl = h->lists.size();
-    const bool fused = nl > 0 && h->p.pair_layout == BS_PAIR_QUEUES && !h->p.probe_enable;
+    const bool fused = step_fused(h, h->p.pair_layout);
     const size_t apart = fused ? nl - 1 : nl; // lists with a pair kernel of their own
     const size_t e1 = h->prof ? prof_mark(h) : SIZE_MAX;
     launch_pairs(h, energy, apart);
@@ -3642,27 +3647,35 @@ int bs_autotune(bs_handle *h, int32_t steps, int32_t *group_out, int32_t *graph_
     rc = springs_host(h); // the trials copy the host spring table
     if (rc)
         return rc;
-    // first the pair layout (at the current lanes and graph setting), then
-    // lanes per spring row x graph replay with that layout
+    // First the pair layout, at the current lanes and graph setting (the row
+    // layout stays), then graph replay with that layout, and with it the lanes
+    // per spring row where the step's springs have a kernel of their own.
     struct Trial
     {
         int32_t layout, group, graph;
     };
     std::vector<Trial> trials;
-    for (int32_t lay : {BS_PAIR_CLUSTERS, BS_PAIR_QUEUES})
-        trials.push_back({lay, h->group, h->p.graph_steps});
-    for (int32_t gs : {0, 16})
-        for (int32_t g : {4, 8, 16, 32})
-            trials.push_back({-1, g, gs});
+    int32_t bg = h->group, bgr = h->p.graph_steps, blay = h->p.pair_layout;
+    if (blay != BS_PAIR_ROWS)
+        for (int32_t lay : {BS_PAIR_CLUSTERS, BS_PAIR_QUEUES})
+            trials.push_back({lay, h->group, h->p.graph_steps});
+    const size_t layouts = trials.size();
     double best = INFINITY;
-    int32_t bg = h->group, bgr = h->p.graph_steps, blay = h->p.pair_layout == BS_PAIR_ROWS ? BS_PAIR_CLUSTERS
-                                                                                        : h->p.pair_layout;
-    for (size_t ti = 0; ti < trials.size(); ++ti)
+    for (size_t ti = 0;; ++ti)
     {
-        if (ti == 2)
-            best = INFINITY; // second phase: compare among itself
-        const int32_t lay = trials[ti].layout >= 0 ? trials[ti].layout : blay;
-        const int32_t g = trials[ti].group, gs = trials[ti].graph;
+        if (ti == layouts)
+        { // second phase: compare among itself
+            best = INFINITY;
+            for (int32_t gs : {0, 16})
+                if (step_fused(h, blay)) // its lanes follow from the cluster count
+                    trials.push_back({blay, h->group, gs});
+                else
+                    for (int32_t g : {4, 8, 16, 32})
+                        trials.push_back({blay, g, gs});
+        }
+        if (ti == trials.size())
+            break;
+        const int32_t lay = trials[ti].layout, g = trials[ti].group, gs = trials[ti].graph;
         {
             bs_handle *t = nullptr;
             bs_params p = h->p;
@@ -3708,7 +3721,7 @@ int bs_autotune(bs_handle *h, int32_t steps, int32_t *group_out, int32_t *graph_
                     hipEventElapsedTime(&ms, e0, e1) == hipSuccess && ms < best)
                 {
                     best = ms;
-                    if (ti < 2)
+                    if (ti < layouts)
                         blay = lay;
                     else
                     {
@@ -3733,7 +3746,7 @@ int bs_autotune(bs_handle *h, int32_t steps, int32_t *group_out, int32_t *graph_
     if (h->p.graph_steps != bgr || h->p.pair_layout != blay)
         drop_graph(h);
     h->p.graph_steps = bgr;
-    if (h->p.pair_layout != BS_PAIR_ROWS && h->p.pair_layout != blay) // row buffers are sized at setup
+    if (h->p.pair_layout != blay)
     {
         rc = set_pair_layout(h, blay);
         if (rc)

@@ -209,6 +209,7 @@ extern "C" void hc_event_times(const float *ms, int32_t n)
     g_event_ms.assign(ms, ms + n);
     g_event_next = 0;
 }
+extern "C" int64_t hc_event_times_used() { return (int64_t)g_event_next; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
 {
     *ms = g_event_next < g_event_ms.size() ? g_event_ms[g_event_next++] : 0.0f;

@@ -595,8 +595,10 @@ int bs_adjoint_backward_noalloc(bs_handle *h, const double *dl_dx3, const double
 /* Times `steps` steps of a copy of the current system for each launch
  * configuration and keeps the fastest for h; h's state is not advanced.
  * First the pair layout (BS_PAIR_CLUSTERS or BS_PAIR_QUEUES; a handle set to
- * BS_PAIR_ROWS keeps it), then lanes per spring row (4/8/16/32) x direct
- * launches or a 16-step graph.  The chosen values go to *group_out,
+ * BS_PAIR_ROWS keeps it), then direct launches or a 16-step graph, and with
+ * them the lanes per spring row (4/8/16/32) where the step's springs have a
+ * kernel of their own: any layout but BS_PAIR_QUEUES, the probe, or no
+ * neighbour list.  Otherwise the lanes stay as they are.  The chosen values go to *group_out,
  * *graph_out, *layout_out (nullable).  No reference counterpart. */
 int bs_autotune(bs_handle *h, int32_t steps, int32_t *group_out, int32_t *graph_out, int32_t *layout_out);
 

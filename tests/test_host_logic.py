@@ -494,3 +494,47 @@ def test_profiling_leaves_the_launches_alone(hostcheck_lib):
         print("same launches")
         ''', hostcheck_lib)
     assert "same launches" in out, out
+
+
+def test_autotune_tries_what_the_step_uses(hostcheck_lib):
+    """Lanes per spring row are tried and set only where the step's springs
+    have a kernel of their own; the row layout is tuned as it is.  A clock
+    makes the last trial of each phase the fastest; the number of trials is
+    the number of setups (allocations)."""
+    out = _run('''
+        s = workloads.generate(1, seed=3, n=500)
+        L.hc_event_times.argtypes = [ctypes.POINTER(ctypes.c_float), ctypes.c_int32]
+        L.hc_event_times_used.restype = ctypes.c_int64
+        C, Q, R = _abi.PAIR_CLUSTERS, _abi.PAIR_QUEUES, _abi.PAIR_ROWS
+        def tune(first, terms=1, probe=0, **kw):
+            p = s.params.copy()
+            p.steric_enable = p.electrostatic_enable = terms
+            p.probe_enable = probe
+            for k, v in kw.items():
+                setattr(p, k, v)
+            net = SpringNetwork.from_system(s, params=p, library=L)
+            net.adjointForward(2, 1) if not probe else net.setup()
+            ms = list(first) + [10.0 - k for k in range(8)]
+            L.hc_event_times((ctypes.c_float * len(ms))(*ms), len(ms))
+            got = net.autotune(2)
+            used = L.hc_event_times_used()
+            kept = None
+            if not probe:
+                try:
+                    net.adjointBackward(np.ones((s.n, 3)))
+                    kept = True
+                except _abi.EngineError as e:
+                    assert e.code == _abi.BS_ERR_STATE
+                    kept = False
+            net.run(2)
+            net.close()
+            return got, used, kept
+        # the queue layout with a list: two graph settings, lanes as they were, the record kept
+        assert tune((2.0, 1.0)) == ((16, 16, Q), 4, True)
+        assert tune((1.0, 2.0)) == ((32, 16, C), 10, False)
+        assert tune((2.0, 1.0), probe=1)[:2] == ((32, 16, Q), 10)
+        assert tune((2.0, 1.0), terms=0)[:2] == ((32, 16, Q), 10)
+        assert tune((), pair_layout=R) == ((32, 16, R), 8, False)
+        print("tuned")
+        ''', hostcheck_lib)
+    assert "tuned" in out, out
