@@ -1444,15 +1444,16 @@ __global__ void k_edge_fill(const uint32_t *sa, const uint32_t *sb, int64_t m, c
 }
 
 constexpr int32_t EDGE_WAVES = BLOCK / 64;
-constexpr int32_t EDGE_KEYS = 4;             // keys per lane held in registers
-constexpr int32_t EDGE_LDS = 64 * EDGE_KEYS; // longer rows rank from global memory
+constexpr int32_t EDGE_KEYS = 4;   // keys per lane held in registers
+constexpr int32_t EDGE_LDS = 1024; // partners of a row held in LDS; longer rows rank from global memory
 
 // One wave per row: each key's rank is the number of smaller partners in the
 // row (partners are distinct).  Writes the edge words and stiffnesses in rank
-// order, then the null edges.  Rows up to EDGE_LDS keep their keys in
-// registers and compare all of them with each partner read from LDS: 3.4
-// reads of four partners per key instead of one 64-bit key per pair (1.81 ->
-// 0.32 ms at 100,000 rows of 182).
+// order, then the null edges.  Bound by VALU issue, every key against every
+// partner: a lane compares EDGE_KEYS keys with four partners per LDS read
+// (eight keys, with fewer waves for their registers, take as long).  40,000
+// rows of 172, 326 and 840: 0.12, 0.39 and 8.3 ms, the last for the rows past
+// EDGE_LDS among them; with 64-bit keys compared one by one 0.71, 2.3 and 19.8.
 __global__ void __launch_bounds__(BLOCK) k_edge_sort(const int32_t *ptr, const int32_t *cnt, int32_t n,
                                                      const uint2 *key, const float4 *jprm, const float *sl,
                                                      const float *sk, uint2 *rows, float *rk)
@@ -1469,30 +1470,33 @@ __global__ void __launch_bounds__(BLOCK) k_edge_sort(const int32_t *ptr, const i
         rows[b + rank] = make_uint2(st ? kv.x | 0x80000000u : kv.x, fbits(sl[kv.y]));
         rk[b + rank] = sk[kv.y];
     };
-    if (len <= EDGE_LDS)
+    if (len <= EDGE_LDS) // wave-uniform
     {
-        uint2 kv[EDGE_KEYS];
-        int32_t rank[EDGE_KEYS];
-#pragma unroll
-        for (int q = 0; q < EDGE_KEYS; ++q)
-        {
-            const int32_t t = lane + 64 * q;
-            kv[q] = t < len ? key[b + t] : make_uint2(0xffffffffu, 0u); // past the end: larger than any partner
-            rank[q] = 0;
-            lj[w][t] = kv[q].x;
-        }
+        for (int32_t t = lane; t < ((len + 3) & ~3); t += 64)
+            lj[w][t] = t < len ? key[b + t].x : 0xffffffffu; // past the end: larger than any partner
         wave_lds_sync();
-        for (int32_t t = 0; t < len; t += 4)
+        for (int32_t e0 = lane; e0 - lane < len; e0 += 64 * EDGE_KEYS)
         {
-            const uint4 o = *reinterpret_cast<const uint4 *>(&lj[w][t]);
+            uint2 kv[EDGE_KEYS];
+            int32_t rank[EDGE_KEYS];
 #pragma unroll
             for (int q = 0; q < EDGE_KEYS; ++q)
-                rank[q] += (o.x < kv[q].x) + (o.y < kv[q].x) + (o.z < kv[q].x) + (o.w < kv[q].x);
-        }
+            {
+                kv[q] = e0 + 64 * q < len ? key[b + e0 + 64 * q] : make_uint2(0u, 0u);
+                rank[q] = 0;
+            }
+            for (int32_t t = 0; t < len; t += 4)
+            {
+                const uint4 o = *reinterpret_cast<const uint4 *>(&lj[w][t]);
 #pragma unroll
-        for (int q = 0; q < EDGE_KEYS; ++q)
-            if (lane + 64 * q < len)
-                put(kv[q], rank[q]);
+                for (int q = 0; q < EDGE_KEYS; ++q)
+                    rank[q] += (o.x < kv[q].x) + (o.y < kv[q].x) + (o.z < kv[q].x) + (o.w < kv[q].x);
+            }
+#pragma unroll
+            for (int q = 0; q < EDGE_KEYS; ++q)
+                if (e0 + 64 * q < len)
+                    put(kv[q], rank[q]);
+        }
     }
     else
         for (int32_t e = lane; e < len; e += 64)
@@ -1526,20 +1530,22 @@ template <class Row> __device__ inline int32_t row_lower_bound(const Row &partne
     return lo;
 }
 
-constexpr int32_t EX_STAGE = 2048; // partners of a cluster's rows held in LDS
+constexpr int32_t EX_STAGE = 8192; // partners of a cluster's rows held in LDS
 
-// One wave per i-cluster: the words j << 8 | 1 << k of its rows k = 0..7
+// One block per i-cluster: the words j << 8 | 1 << k of its rows k = 0..7
 // merged in j order (stable in k) from merged[EDGE_PAD ptr[8c]] on, then the
-// number of distinct j.  The binary searches run on a copy of the rows in LDS
-// when they fit (0.96 -> 0.55 ms at 100,000 rows of 182).
+// number of distinct j.  Bound by the binary searches' dependent reads, so
+// they run on a copy of the rows' partners in LDS where it fits.  5,000
+// clusters of rows of 172, 326 and 840: 0.20, 0.40 and 1.9 ms (a wave per
+// cluster with 2,048 partners each: 0.27, 1.5, 5.4; all from global memory, 4
+// bytes a partner: 0.49, 1.0, 3.3).
 __global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n,
                                                     int32_t ncl, uint32_t *merged, int32_t *ucount)
 {
-    __shared__ int32_t stage[EDGE_WAVES][EX_STAGE];
-    const int32_t lane = (int32_t)(threadIdx.x & 63u), w = (int32_t)(threadIdx.x >> 6);
-    const int32_t c = (int32_t)blockIdx.x * EDGE_WAVES + w;
-    if (c >= ncl)
-        return; // whole wave
+    __shared__ int32_t stage[EX_STAGE];
+    __shared__ int32_t part[EDGE_WAVES];
+    const int32_t tid = (int32_t)threadIdx.x;
+    const int32_t c = (int32_t)blockIdx.x;
     // row k: edges from[k] on, words off[k] to off[k + 1] of the cluster
     size_t from[CLUSTER];
     int32_t off[CLUSTER + 1];
@@ -1553,16 +1559,16 @@ __global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const in
     }
     const int32_t total = off[CLUSTER];
     const size_t base = from[0];
-    const bool staged = total <= EX_STAGE;
+    const bool staged = total <= EX_STAGE; // block-uniform
     if (staged)
     {
 #pragma unroll
         for (int k = 0; k < CLUSTER; ++k)
-            for (int32_t t = lane; t < off[k + 1] - off[k]; t += 64)
-                stage[w][off[k] + t] = (int32_t)(rows[from[k] + t].x & 0x7fffffffu);
-        wave_lds_sync();
+            for (int32_t t = tid; t < off[k + 1] - off[k]; t += BLOCK)
+                stage[off[k] + t] = (int32_t)(rows[from[k] + t].x & 0x7fffffffu);
+        __syncthreads();
     }
-    for (int32_t e = lane; e < total; e += 64)
+    for (int32_t e = tid; e < total; e += BLOCK)
     {
         int32_t k = 0, start = 0;
         size_t row = from[0];
@@ -1573,32 +1579,35 @@ __global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const in
             start = e >= off[q] ? off[q] : start;
             row = e >= off[q] ? from[q] : row;
         }
-        const int32_t j = staged ? stage[w][e] : (int32_t)(rows[row + (e - start)].x & 0x7fffffffu);
+        const int32_t j = staged ? stage[e] : (int32_t)(rows[row + (e - start)].x & 0x7fffffffu);
         // rank: its place in its own row, plus the smaller words of the
         // other rows (for rows before its own, the equal ones too)
         int32_t r = e - start;
 #pragma unroll
         for (int q = 0; q < CLUSTER; ++q)
             if (q != k)
-                r += staged ? row_lower_bound([&](int32_t t) { return stage[w][off[q] + t]; }, off[q + 1] - off[q], j,
-                                              q < k)
+                r += staged ? row_lower_bound([&](int32_t t) { return stage[off[q] + t]; }, off[q + 1] - off[q], j, q < k)
                             : row_lower_bound([&](int32_t t) { return (int32_t)(rows[from[q] + t].x & 0x7fffffffu); },
                                               off[q + 1] - off[q], j, q < k);
         merged[base + r] = (uint32_t)j << 8 | 1u << k;
     }
-    // the wave reads back what its own lanes stored (one CU)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    __syncthreads(); // the block reads back what it stored
     int32_t u = 0;
-    for (int32_t t0 = 0; t0 < total; t0 += 64)
+    for (int32_t t0 = 0; t0 < total; t0 += BLOCK)
     {
-        const int32_t t = t0 + lane;
+        const int32_t t = t0 + tid;
         const bool first = t < total && (t == 0 || (merged[base + t - 1] >> 8) != (merged[base + t] >> 8));
         u += (int32_t)__popcll(__ballot(first));
     }
-    if (lane == 0)
+    if ((tid & 63) == 0)
+        part[tid >> 6] = u;
+    __syncthreads();
+    if (tid == 0)
+    {
+        for (int w = 1; w < EDGE_WAVES; ++w)
+            u += part[w];
         ucount[c] = u;
+    }
 }
 
 // The distinct words of each cluster, masks of equal j or-ed, at ex_ptr[c].
@@ -1993,7 +2002,7 @@ void launch_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, 
                      uint32_t *merged, int32_t *ucount, hipStream_t s)
 {
     if (ncl > 0)
-        k_ex_merge<<<(ncl + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, cnt, rows, n, ncl, merged, ucount);
+        k_ex_merge<<<ncl, BLOCK, 0, s>>>(ptr, cnt, rows, n, ncl, merged, ucount);
 }
 
 void launch_ex_fill(const int32_t *ptr, const int32_t *cnt, int32_t n, int32_t ncl, const uint32_t *merged,

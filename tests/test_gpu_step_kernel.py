@@ -84,7 +84,7 @@ def test_distant_beads_have_empty_lists():
     _compare(s)
 
 
-@pytest.mark.parametrize("spokes", [1, 7, 8, 255, 256, 257, 300])
+@pytest.mark.parametrize("spokes", [1, 7, 8, 255, 256, 257, 300, 512, 513, 1023, 1024, 1025])
 def test_row_lengths(spokes):
     """One hub with `spokes` springs, given in a shuffled order: its force is
     their sum, and every spoke's the opposite."""
@@ -114,3 +114,26 @@ def test_row_lengths(spokes):
     # FP64 sums rounded to FP32: half an ulp of each component
     assert np.abs(f - want).max() <= 1.2e-7 * np.abs(want).max()
     assert abs(e[_abi.E_SPRING] - (0.5 * k.astype(np.float64) * (r - l0) ** 2).sum()) <= 1e-9 * abs(e[_abi.E_SPRING])
+
+
+@pytest.mark.parametrize("n,cutoff", [(900, 7.0), (1100, 12.0), (1400, 40.0)])
+def test_exclusions_of_long_rows(n, cutoff):
+    """The listed pairs are those inside the cutoff without a spring, whether
+    a cluster's rows fit the exclusions' LDS copy (8,192 partners) or not:
+    rows of 15 to 100, of 85 to 520, and of 1,260."""
+    rng = np.random.default_rng(n)
+    x = (rng.random((n, 3)) * 24.0).astype(np.float32)
+    d = np.linalg.norm(x[:, None].astype(np.float64) - x[None], axis=2)
+    i, j = np.triu_indices(n, 1)
+    spring = (d[i, j] < cutoff) & (rng.random(len(i)) < 0.9)
+    near = d[i, j] < 12.0
+    order = rng.permutation(np.flatnonzero(spring))
+    p = _abi.default_params()
+    p.spring_enable, p.steric_enable, p.steric_mode, p.steric_cutoff = 1, 1, _abi.STERIC_LINEAR, 12.0
+    net = SpringNetwork(p)
+    net.setParticles(x.reshape(-1))
+    net.setSprings(i[order].astype(np.uint32), j[order].astype(np.uint32), d[i, j][order].astype(np.float32),
+                   np.ones(len(order), np.float32))
+    got = {tuple(sorted(v)) for v in net.getPairs(_abi.NS_STERIC).tolist()}
+    want = set(zip(i[near & ~spring].tolist(), j[near & ~spring].tolist()))
+    assert got == want, (len(got), len(want), len(got ^ want))
