@@ -72,7 +72,7 @@ struct EdgeRow
 {
     const char *eb, *kb; // kb null: every spring has stiffness k_uni
     float k_uni;
-    uint32_t off, last, step;
+    uint32_t off, last, step, self; // self: the row, partner of its null edges
 
     // G lanes per row, 64 / G rows from row0 on (wave-uniform) of the wave;
     // row0 < n.  Rows past n, static rows and disabled springs read the null
@@ -84,6 +84,7 @@ struct EdgeRow
         kb = a.sp_k ? reinterpret_cast<const char *>(a.sp_k + (size_t)c0 * EDGE_PAD) : nullptr;
         k_uni = a.k_uni;
         step = (uint32_t)G * sizeof(uint2);
+        self = (uint32_t)r;
         const uint32_t unit = EDGE_PAD * sizeof(uint2);
         last = (uint32_t)(a.sp_ptr[r + 1] - c0) * unit - (uint32_t)sizeof(uint2);
         off = on ? (uint32_t)(a.sp_ptr[r] - c0) * unit + (uint32_t)lane * (uint32_t)sizeof(uint2) : last;
@@ -237,7 +238,9 @@ __device__ inline void probe_pair(const ProbeArgs &p, const float4 q, float4 pi,
 
 // The springs of the wave's rows, D edges in flight per lane: the edge words
 // of the next D load while these gather and compute (two dependent loads per
-// edge: the word, then x_j).
+// edge: the word, then x_j).  A lane with null edges alone adds nothing, also
+// for a particle whose position is not finite (a null edge of a lane that has
+// a real one cannot make that one's sum worse).
 template <int D, bool COMP> __device__ inline void row_springs(const SpringArgs &a, EdgeRow &er, RowSum<COMP> &sum, bool energy)
 {
     uint32_t j[D], jn[D];
@@ -245,6 +248,7 @@ template <int D, bool COMP> __device__ inline void row_springs(const SpringArgs 
 #pragma unroll
     for (int u = 0; u < D; ++u)
         er.word(u, j[u], l[u], k[u]);
+    const bool real = j[0] != er.self;
     for (int32_t left = er.steps(); left > 0; left -= D) // wave-uniform
     {
         float4 p[D];
@@ -267,6 +271,8 @@ template <int D, bool COMP> __device__ inline void row_springs(const SpringArgs 
             l[u] = ln[u];
         }
     }
+    if (!real)
+        sum.fx = sum.fy = sum.fz = sum.e = 0.0;
 }
 
 // What a particle's row adds to the sums beside its force: energies, and the

@@ -137,3 +137,30 @@ def test_exclusions_of_long_rows(n, cutoff):
     got = {tuple(sorted(v)) for v in net.getPairs(_abi.NS_STERIC).tolist()}
     want = set(zip(i[near & ~spring].tolist(), j[near & ~spring].tolist()))
     assert got == want, (len(got), len(want), len(got ^ want))
+
+
+@pytest.mark.parametrize("layout", [_abi.PAIR_QUEUES, _abi.PAIR_CLUSTERS])
+@pytest.mark.parametrize("lost", [np.inf, np.nan])
+@pytest.mark.parametrize("comp", [0, 1])
+def test_a_fixed_bead_nowhere_adds_nothing(layout, lost, comp):
+    """A fixed bead without springs at a position that is not finite (an atom
+    that a structure lacks) leaves every force, energy and step as they are
+    without it."""
+    s = _perturbed(1, 1501, 9)
+    gone = 700
+    keep = (s.id1 != gone) & (s.id2 != gone)
+    s.id1, s.id2, s.l0, s.k = s.id1[keep], s.id2[keep], s.l0[keep], s.k[keep]
+    s.flags[gone] = _abi.FLAG_STATIC
+    got = []
+    for x in (1.0e4, lost):
+        s.x.reshape(-1, 3)[gone] = x
+        p = s.params.copy()
+        p.pair_layout, p.compensated_positions, p.electrostatic_enable = layout, comp, 0
+        net = SpringNetwork.from_system(s, p)
+        f, e = net.computeForces()
+        net.run(3)
+        x3, v3 = net.getState()
+        got.append((f, e, np.delete(x3, gone, 0), v3, net.getEnergies()))
+    for a, b in zip(*got):
+        assert np.isfinite(b).all()
+        assert np.abs(a - b).max() <= TOL * max(np.abs(a).max(), 1e-12)
