@@ -529,9 +529,19 @@ uint32_t particle_flags(const bs_handle *h, int64_t i)
 }
 
 // A particle's share of the steric size as the kernels take it: two factors'
-// product is R^2 (R = sqrt(r_i r_j) for Amber and Lewitt, r_i r_j for
-// Zacharias); the raw radius for the linear wall, which adds them.
-float radius_factor(int32_t steric_mode, float r) { return steric_mode == BS_STERIC_ZACHARIAS_8_6 ? r * r : r; }
+// product is R^2 (R = sqrt(r_i r_j) for Amber and Lewitt, where a negative
+// radius has no square root; r_i r_j for Zacharias, whose kernels any mode
+// past it gets); the raw radius for the linear wall, which adds them.
+float radius_factor(int32_t steric_mode, float r)
+{
+    switch (steric_mode)
+    {
+    case BS_STERIC_LINEAR: return r;
+    case BS_STERIC_AMBER_12_6:
+    case BS_STERIC_LEWITT_8_6: return r < 0.0f ? NAN : r;
+    default: return r * r;
+    }
+}
 
 float4 jprm_of(const bs_handle *h, int64_t i)
 {

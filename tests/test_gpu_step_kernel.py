@@ -164,3 +164,23 @@ def test_a_fixed_bead_nowhere_adds_nothing(layout, lost, comp):
     for a, b in zip(*got):
         assert np.isfinite(b).all()
         assert np.abs(a - b).max() <= TOL * max(np.abs(a).max(), 1e-12)
+
+
+@pytest.mark.parametrize("mode", [_abi.STERIC_AMBER_12_6, _abi.STERIC_LEWITT_8_6])
+@pytest.mark.parametrize("layout", [_abi.PAIR_QUEUES, _abi.PAIR_CLUSTERS])
+def test_a_negative_radius_is_not_a_number(mode, layout):
+    """sqrt(r_i r_j) of a negative and a positive radius is NaN, as in the
+    reference (energy/steric.hpp), and not a size with a sign: the bead's
+    forces and the steric energy say so, the beads out of its reach are as
+    they were."""
+    s = _perturbed(1, 1501, 4)
+    p = s.params.copy()
+    p.pair_layout, p.steric_mode, p.electrostatic_enable = layout, mode, 0
+    f0, e0 = SpringNetwork.from_system(s, p).computeForces()
+    bad = 17
+    s.radius[bad] = -s.radius[bad]
+    f, e = SpringNetwork.from_system(s, p).computeForces()
+    d = np.linalg.norm(s.x.reshape(-1, 3).astype(np.float64) - s.x.reshape(-1, 3)[bad], axis=1)
+    assert np.isnan(f[bad]).all() and np.isnan(e[_abi.E_STERIC]) and np.isfinite(e0).all()
+    far = d > 1.0001 * p.steric_cutoff
+    assert far.any() and np.array_equal(f[far], f0[far])
