@@ -345,7 +345,7 @@ __global__ void __launch_bounds__(BLOCK) k_spring(SpringArgs a)
     if (row0 < a.n && a.spring_enable) // wave-uniform
     {
         EdgeRow er(a, row0, row, lane, G, dyn);
-        row_springs<8, COMP>(a, er, sum, a.energy != 0);
+        row_springs<8, false, COMP>(a, er, sum, a.energy != 0, er.steps<G>());
     }
     const double cs = a.k.c_spring * (double)a.spring_scale;
     double fx = sum.fx * cs, fy = sum.fy * cs, fz = sum.fz * cs, espr = sum.e;
@@ -844,7 +844,7 @@ __global__ void __launch_bounds__(BLOCK) k_adj_spring(AdjSpringArgs a)
 #pragma unroll
         for (int u = 0; u < U; ++u)
             er.word(u, jr[u], ll[u], kk[u]);
-        for (int32_t it = (er.steps() + U - 1) / U; it > 0; --it)
+        for (int32_t it = (er.steps<G>() + U - 1) / U; it > 0; --it)
         {
             uint32_t jn[U];
             float kn[U], ln[U];

@@ -89,13 +89,16 @@ struct EdgeRow
         last = (uint32_t)(a.sp_ptr[r + 1] - c0) * unit - (uint32_t)sizeof(uint2);
         off = on ? (uint32_t)(a.sp_ptr[r] - c0) * unit + (uint32_t)lane * (uint32_t)sizeof(uint2) : last;
     }
-    // the longest row of the wave in steps (wave-uniform)
-    __device__ int32_t steps() const
+    // the longest row of the wave in steps (wave-uniform): a row's first lane
+    // takes the most, and rows start at lanes that STRIDE divides
+    template <int STRIDE> __device__ int32_t steps() const
     {
-        int32_t s = ((int32_t)(last - off) + (int32_t)(sizeof(uint2) + step) - 1) >> (31 - __builtin_clz(step));
-        for (int o = 1; o < 64; o <<= 1)
-            s = max(s, __shfl_xor(s, o, 64));
-        return __builtin_amdgcn_readfirstlane(s);
+        const int32_t s = ((int32_t)(last - off) + (int32_t)(sizeof(uint2) + step) - 1) >> (31 - __builtin_clz(step));
+        int32_t m = 0;
+#pragma unroll
+        for (int o = 0; o < 64; o += STRIDE)
+            m = max(m, __builtin_amdgcn_readlane(s, o));
+        return m;
     }
     __device__ void word(int u, uint32_t &j, float &l0, float &k) const
     {
@@ -236,29 +239,40 @@ __device__ inline void probe_pair(const ProbeArgs &p, const float4 q, float4 pi,
     f[2] += dz * inv * fm;
 }
 
-// The springs of the wave's rows, D edges in flight per lane: the edge words
-// of the next D load while these gather and compute (two dependent loads per
-// edge: the word, then x_j).  A lane with null edges alone adds nothing, also
-// for a particle whose position is not finite (a null edge of a lane that has
-// a real one cannot make that one's sum worse).
-template <int D, bool COMP> __device__ inline void row_springs(const SpringArgs &a, EdgeRow &er, RowSum<COMP> &sum, bool energy)
+// The springs of the wave's rows (at most `steps` edges a lane), D edges in
+// flight per lane: the edge words of the next D load while these gather and
+// compute (two dependent loads per edge: the word, then x_j).  A lane with null
+// edges alone adds nothing, also for a particle whose position is not finite
+// (a null edge of a lane that has a real one cannot make that one's sum worse).
+//
+// Every edge in flight costs a row its loads, needed or not: with ALL none is
+// skipped, which suits D = 4 beside the pair walk (skipped there: 71 -> 69 us
+// a step for chains of 250,000 beads, but 465 -> 467 for rows of 182); with D =
+// 8 and the springs alone the branches pay at every length (100,000 rows of 5,
+// 71 and 185 springs: 39.4, 43.5 and 59.8 us with all loads, 28.9, 37.2 and
+// 55.6 without the idle ones).
+template <int D, bool ALL, bool COMP>
+__device__ inline void row_springs(const SpringArgs &a, EdgeRow &er, RowSum<COMP> &sum, bool energy, int32_t steps)
 {
     uint32_t j[D], jn[D];
     float k[D], l[D], kn[D], ln[D];
 #pragma unroll
     for (int u = 0; u < D; ++u)
-        er.word(u, j[u], l[u], k[u]);
+        if (ALL || u < steps)
+            er.word(u, j[u], l[u], k[u]);
     const bool real = j[0] != er.self;
-    for (int32_t left = er.steps(); left > 0; left -= D) // wave-uniform
+    for (int32_t left = steps; left > 0; left -= D) // wave-uniform
     {
         float4 p[D];
 #pragma unroll
         for (int u = 0; u < D; ++u)
-            p[u] = partner(a.pos, j[u]);
+            if (ALL || u < left)
+                p[u] = partner(a.pos, j[u]);
         er.off += D * er.step;
 #pragma unroll
         for (int u = 0; u < D; ++u)
-            er.word(u, jn[u], ln[u], kn[u]);
+            if (ALL || D + u < left)
+                er.word(u, jn[u], ln[u], kn[u]);
 #pragma unroll
         for (int u = 0; u < D; ++u)
             if (u < left)

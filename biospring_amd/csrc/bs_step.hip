@@ -39,7 +39,7 @@ __device__ inline void spring_walk(const SpringArgs &a, int32_t first, int32_t r
     if (a.spring_enable)
     {
         EdgeRow er(a, min(first, a.n - 1), row, lane & (G - 1), G, live && !(fbits(a.jprm[row].w) & PF_STATIC));
-        row_springs<4, COMP>(a, er, sum, ENERGY);
+        row_springs<4, true, COMP>(a, er, sum, ENERGY, er.steps<CLUSTER>());
     }
     for (int off = G / 2; off > 0; off >>= 1)
     {
