@@ -2045,7 +2045,7 @@ int do_setup(bs_handle *h)
         const int32_t ncl = (int32_t)((n + CLUSTER - 1) / CLUSTER);
         uint32_t *merged = reinterpret_cast<uint32_t *>(key); // the keys are done with
         int32_t *ucnt = units;
-        launch_ex_merge(fptr, cnt, frow, (int32_t)n, ncl, merged, ucnt, st);
+        launch_ex_merge(fptr, cnt, frow, (int32_t)n, ncl, 2 * m, merged, ucnt, st);
         ALLOC(h->ex_ptr, int32_t, ncl + 1);
         launch_scan(ucnt, h->ex_ptr, ncl, nullptr, st);
         int32_t nex = 0;

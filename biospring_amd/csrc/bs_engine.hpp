@@ -452,8 +452,9 @@ void launch_edge_sort(const uint32_t *sa, const uint32_t *sb, int64_t m, const i
 // Exclusions of each i-cluster from its rows: merged (j << 8 | row bit, in
 // j order) from merged[EDGE_PAD ptr[8c]] on with the count of distinct j per
 // cluster, then the distinct words (row bits of equal j or-ed) at ex_ptr[c].
+// nedges: the rows' edges in all.
 void launch_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n, int32_t ncl,
-                     uint32_t *merged, int32_t *ucount, hipStream_t s);
+                     int64_t nedges, uint32_t *merged, int32_t *ucount, hipStream_t s);
 void launch_ex_fill(const int32_t *ptr, const int32_t *cnt, int32_t n, int32_t ncl, const uint32_t *merged,
                     const int32_t *ex_ptr, uint32_t *ex_w, hipStream_t s);
 // Rows without the edges joining two rigid members (rigid[i] != 0): krows

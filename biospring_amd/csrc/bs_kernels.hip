@@ -1472,18 +1472,25 @@ __global__ void __launch_bounds__(BLOCK) k_edge_sort(const int32_t *ptr, const i
     };
     if (len <= EDGE_LDS) // wave-uniform
     {
-        for (int32_t t = lane; t < ((len + 3) & ~3); t += 64)
-            lj[w][t] = t < len ? key[b + t].x : 0xffffffffu; // past the end: larger than any partner
-        wave_lds_sync();
-        for (int32_t e0 = lane; e0 - lane < len; e0 += 64 * EDGE_KEYS)
+        for (int32_t e0 = 0; e0 < len; e0 += 64 * EDGE_KEYS)
         {
             uint2 kv[EDGE_KEYS];
             int32_t rank[EDGE_KEYS];
 #pragma unroll
             for (int q = 0; q < EDGE_KEYS; ++q)
             {
-                kv[q] = e0 + 64 * q < len ? key[b + e0 + 64 * q] : make_uint2(0u, 0u);
+                const int32_t t = e0 + lane + 64 * q;
+                kv[q] = t < len ? key[b + t] : make_uint2(0xffffffffu, 0u); // past the end: larger than any partner
                 rank[q] = 0;
+            }
+            if (e0 == 0)
+            {
+#pragma unroll
+                for (int q = 0; q < EDGE_KEYS; ++q)
+                    lj[w][lane + 64 * q] = kv[q].x;
+                for (int32_t t = 64 * EDGE_KEYS + lane; t < ((len + 3) & ~3); t += 64)
+                    lj[w][t] = t < len ? key[b + t].x : 0xffffffffu;
+                wave_lds_sync();
             }
             for (int32_t t = 0; t < len; t += 4)
             {
@@ -1494,7 +1501,7 @@ __global__ void __launch_bounds__(BLOCK) k_edge_sort(const int32_t *ptr, const i
             }
 #pragma unroll
             for (int q = 0; q < EDGE_KEYS; ++q)
-                if (e0 + 64 * q < len)
+                if (e0 + lane + 64 * q < len)
                     put(kv[q], rank[q]);
         }
     }
@@ -1530,22 +1537,37 @@ template <class Row> __device__ inline int32_t row_lower_bound(const Row &partne
     return lo;
 }
 
-constexpr int32_t EX_STAGE = 8192; // partners of a cluster's rows held in LDS
+constexpr int32_t EX_STAGE = 2048; // partners per wave held in LDS
 
-// One block per i-cluster: the words j << 8 | 1 << k of its rows k = 0..7
-// merged in j order (stable in k) from merged[EDGE_PAD ptr[8c]] on, then the
-// number of distinct j.  Bound by the binary searches' dependent reads, so
-// they run on a copy of the rows' partners in LDS where it fits.  5,000
-// clusters of rows of 172, 326 and 840: 0.20, 0.40 and 1.9 ms (a wave per
-// cluster with 2,048 partners each: 0.27, 1.5, 5.4; all from global memory, 4
-// bytes a partner: 0.49, 1.0, 3.3).
+// W waves per i-cluster, a block's other waves for the next ones: the words
+// j << 8 | 1 << k of its rows k = 0..7 merged in j order (stable in k) from
+// merged[EDGE_PAD ptr[8c]] on, then the number of distinct j.  Bound by the
+// binary searches' dependent reads, so they run on a copy of the rows' partners
+// in LDS where it fits.
+template <int W>
 __global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n,
                                                     int32_t ncl, uint32_t *merged, int32_t *ucount)
 {
-    __shared__ int32_t stage[EX_STAGE];
+    constexpr int PER = EDGE_WAVES / W; // clusters per block
+    constexpr int32_t LANES = 64 * W;
+    __shared__ int32_t stages[PER][EX_STAGE * W];
     __shared__ int32_t part[EDGE_WAVES];
-    const int32_t tid = (int32_t)threadIdx.x;
-    const int32_t c = (int32_t)blockIdx.x;
+    const int32_t tid = (int32_t)threadIdx.x % LANES;
+    const int32_t c = (int32_t)blockIdx.x * PER + (int32_t)threadIdx.x / LANES;
+    int32_t *stage = stages[threadIdx.x / LANES];
+    if (PER > 1 && c >= ncl)
+        return; // whole wave; no block barrier below
+    // what a lane of the cluster wrote, its other lanes read
+    auto sync = [&]() {
+        if (W > 1)
+            __syncthreads();
+        else
+        {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        }
+    };
     // row k: edges from[k] on, words off[k] to off[k + 1] of the cluster
     size_t from[CLUSTER];
     int32_t off[CLUSTER + 1];
@@ -1559,16 +1581,16 @@ __global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const in
     }
     const int32_t total = off[CLUSTER];
     const size_t base = from[0];
-    const bool staged = total <= EX_STAGE; // block-uniform
+    const bool staged = total <= EX_STAGE * W; // the same for the cluster's lanes
     if (staged)
     {
 #pragma unroll
         for (int k = 0; k < CLUSTER; ++k)
-            for (int32_t t = tid; t < off[k + 1] - off[k]; t += BLOCK)
+            for (int32_t t = tid; t < off[k + 1] - off[k]; t += LANES)
                 stage[off[k] + t] = (int32_t)(rows[from[k] + t].x & 0x7fffffffu);
-        __syncthreads();
+        sync();
     }
-    for (int32_t e = tid; e < total; e += BLOCK)
+    for (int32_t e = tid; e < total; e += LANES)
     {
         int32_t k = 0, start = 0;
         size_t row = from[0];
@@ -1591,23 +1613,24 @@ __global__ void __launch_bounds__(BLOCK) k_ex_merge(const int32_t *ptr, const in
                                               off[q + 1] - off[q], j, q < k);
         merged[base + r] = (uint32_t)j << 8 | 1u << k;
     }
-    __syncthreads(); // the block reads back what it stored
+    sync();
     int32_t u = 0;
-    for (int32_t t0 = 0; t0 < total; t0 += BLOCK)
+    for (int32_t t0 = 0; t0 < total; t0 += LANES)
     {
         const int32_t t = t0 + tid;
         const bool first = t < total && (t == 0 || (merged[base + t - 1] >> 8) != (merged[base + t] >> 8));
         u += (int32_t)__popcll(__ballot(first));
     }
-    if ((tid & 63) == 0)
-        part[tid >> 6] = u;
-    __syncthreads();
-    if (tid == 0)
+    if (W > 1)
     {
-        for (int w = 1; w < EDGE_WAVES; ++w)
-            u += part[w];
-        ucount[c] = u;
+        if ((tid & 63) == 0)
+            part[tid >> 6] = u;
+        __syncthreads();
+        for (int w = 1; w < W; ++w)
+            u += tid == 0 ? part[w] : 0;
     }
+    if (tid == 0)
+        ucount[c] = u;
 }
 
 // The distinct words of each cluster, masks of equal j or-ed, at ex_ptr[c].
@@ -1999,10 +2022,19 @@ void launch_edge_sort(const uint32_t *sa, const uint32_t *sb, int64_t m, const i
 }
 
 void launch_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n, int32_t ncl,
-                     uint32_t *merged, int32_t *ucount, hipStream_t s)
+                     int64_t nedges, uint32_t *merged, int32_t *ucount, hipStream_t s)
 {
-    if (ncl > 0)
-        k_ex_merge<<<ncl, BLOCK, 0, s>>>(ptr, cnt, rows, n, ncl, merged, ucount);
+    if (ncl <= 0)
+        return;
+    // A block per cluster has LDS for four times the partners and wins where
+    // there is work for its lanes: 100,000 rows of 5, 71, 118 and 185 take 76,
+    // 229, 338 and 517 us with it, 26, 213, 349 and 577 with a wave per cluster;
+    // 40,000 rows of 326 and 840, past a wave's LDS, 0.40 and 1.9 ms against 1.5
+    // and 5.4 (1.0 and 3.3 with 4 bytes a partner in global memory).
+    if (nedges > 1024 * (int64_t)ncl)
+        k_ex_merge<EDGE_WAVES><<<ncl, BLOCK, 0, s>>>(ptr, cnt, rows, n, ncl, merged, ucount);
+    else
+        k_ex_merge<1><<<(ncl + EDGE_WAVES - 1) / EDGE_WAVES, BLOCK, 0, s>>>(ptr, cnt, rows, n, ncl, merged, ucount);
 }
 
 void launch_ex_fill(const int32_t *ptr, const int32_t *cnt, int32_t n, int32_t ncl, const uint32_t *merged,

@@ -1134,7 +1134,7 @@ void launch_edge_sort(const uint32_t *sa, const uint32_t *sb, int64_t m, const i
 }
 
 void launch_ex_merge(const int32_t *ptr, const int32_t *cnt, const uint2 *rows, int32_t n, int32_t ncl,
-                     uint32_t *merged, int32_t *ucount, hipStream_t)
+                     int64_t, uint32_t *merged, int32_t *ucount, hipStream_t)
 {
     need(ptr, sizeof(int32_t) * (n + 1), "ex_merge: ptr");
     need(rows, sizeof(uint2) * EDGE_PAD * (size_t)ptr[n], "ex_merge: rows");
