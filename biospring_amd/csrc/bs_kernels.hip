@@ -836,63 +836,91 @@ __global__ void __launch_bounds__(BLOCK) k_adj_spring(AdjSpringArgs a)
         const uint64_t gmask = ((1ull << G) - 1ull) << gbase; // G <= 32
         const bool own = a.dk && dyn;
         const double px = pi.x, py = pi.y, pz = pi.z;
-        constexpr int U = 4; // edges in flight per lane
-        // the edge words of the next iteration load while this one gathers
-        // and computes
-        uint32_t jr[U];
-        float kk[U], ll[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            er.word(u, jr[u], ll[u], kk[u]);
-        for (int32_t it = (er.steps<G>() + U - 1) / U; it > 0; --it)
+        auto edge = [&](uint32_t j, float kf, float lf, float4 pj, float4 wj) {
+            // a null edge's partner is the row itself: not owned
+            const bool owned = own && (int32_t)j != row && ((int32_t)j < 0 || (int32_t)j > row);
+            const uint64_t ob = __ballot(owned) & gmask;
+            const int32_t slot = next_slot + (int32_t)__popcll(ob & ((1ull << (threadIdx.x & 63u)) - 1ull));
+            next_slot += (int32_t)__popcll(ob);
+            const double dx = (double)pj.x - px, dy = (double)pj.y - py, dz = (double)pj.z - pz;
+            const double r2 = dx * dx + dy * dy + dz * dz;
+            if (!(r2 > 0.0))
+                return;
+            const double k = kf, l0 = lf;
+            const double ir = rsqrt_d(r2), r = r2 * ir;
+            const double phi = k * (r - l0) * C * ir, dphi = (k * C - phi) * ir;
+            const double wx = (double)wj.x - wi.x, wy = (double)wj.y - wi.y, wz = (double)wj.z - wi.z;
+            const double dd = dx * wx + dy * wy + dz * wz;
+            const double g = dphi * ir * dd;
+            hx = fma(phi, wx, fma(g, dx, hx));
+            hy = fma(phi, wy, fma(g, dy, hy));
+            hz = fma(phi, wz, fma(g, dz, hz));
+            if (owned)
+            {
+                const double wu = dd * ir * C;
+                a.dk[slot] -= (float)(wu * (r - l0));
+                a.dl0[slot] += (float)(wu * k);
+            }
+        };
+        // edges in flight per lane: S for rows of up to S steps, where more
+        // would load null edges (100,000 rows of 5, 18 and 31 springs: 73, 74
+        // and 80 us with U of them, 66, 67 and 74 with S), else U (rows of 118
+        // and 185: 112 and 162 us; with their idle loads skipped 118 and 191,
+        // as the branches part the loads)
+        constexpr int S = 2, U = 4;
+        const int32_t steps = er.steps<G>(); // wave-uniform
+        if (steps <= S)
         {
-            uint32_t jn[U];
-            float kn[U], ln[U];
-            float4 pj[U], wj[U];
+            uint32_t j[S];
+            float k[S], l[S];
+            float4 p[S], w[S];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
+            for (int u = 0; u < S; ++u)
+                er.word(u, j[u], l[u], k[u]);
+#pragma unroll
+            for (int u = 0; u < S; ++u)
             {
-                pj[u] = partner(a.pos, jr[u]);
-                wj[u] = partner(a.w, jr[u]);
+                p[u] = partner(a.pos, j[u]);
+                w[u] = partner(a.w, j[u]);
             }
-            er.off += U * er.step;
+#pragma unroll
+            for (int u = 0; u < S; ++u)
+                edge(j[u], k[u], l[u], p[u], w[u]);
+        }
+        else
+        {
+            // the edge words of the next iteration load while this one
+            // gathers and computes
+            uint32_t jr[U];
+            float kk[U], ll[U];
 #pragma unroll
             for (int u = 0; u < U; ++u)
-                er.word(u, jn[u], ln[u], kn[u]);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
+                er.word(u, jr[u], ll[u], kk[u]);
+            for (int32_t left = steps; left > 0; left -= U)
             {
-                // a null edge's partner is the row itself: not owned
-                const bool owned = own && (int32_t)jr[u] != row && ((int32_t)jr[u] < 0 || (int32_t)jr[u] > row);
-                const uint64_t ob = __ballot(owned) & gmask;
-                const int32_t slot = next_slot + (int32_t)__popcll(ob & ((1ull << (threadIdx.x & 63u)) - 1ull));
-                next_slot += (int32_t)__popcll(ob);
-                const double dx = (double)pj[u].x - px, dy = (double)pj[u].y - py, dz = (double)pj[u].z - pz;
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                if (!(r2 > 0.0))
-                    continue;
-                const double k = kk[u], l0 = ll[u];
-                const double ir = rsqrt_d(r2), r = r2 * ir;
-                const double phi = k * (r - l0) * C * ir, dphi = (k * C - phi) * ir;
-                const double wx = (double)wj[u].x - wi.x, wy = (double)wj[u].y - wi.y, wz = (double)wj[u].z - wi.z;
-                const double dd = dx * wx + dy * wy + dz * wz;
-                const double g = dphi * ir * dd;
-                hx = fma(phi, wx, fma(g, dx, hx));
-                hy = fma(phi, wy, fma(g, dy, hy));
-                hz = fma(phi, wz, fma(g, dz, hz));
-                if (owned)
+                uint32_t jn[U];
+                float kn[U], ln[U];
+                float4 pj[U], wj[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
                 {
-                    const double wu = dd * ir * C;
-                    a.dk[slot] -= (float)(wu * (r - l0));
-                    a.dl0[slot] += (float)(wu * k);
+                    pj[u] = partner(a.pos, jr[u]);
+                    wj[u] = partner(a.w, jr[u]);
                 }
-            }
+                er.off += U * er.step;
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-            {
-                jr[u] = jn[u];
-                kk[u] = kn[u];
-                ll[u] = ln[u];
+                for (int u = 0; u < U; ++u)
+                    er.word(u, jn[u], ln[u], kn[u]);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    edge(jr[u], kk[u], ll[u], pj[u], wj[u]);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                {
+                    jr[u] = jn[u];
+                    kk[u] = kn[u];
+                    ll[u] = ln[u];
+                }
             }
         }
     }
