@@ -331,12 +331,17 @@ struct ListSet
 
 // Blocks of one wave (a slot is free as soon as its cluster is done; clusters'
 // candidates differ by half) where the build is most of the launch, of four
-// where a gated-off launch is: at 31,250 clusters 67 against 77 us a step, at
-// two lists of 12,000 with few rebuilds 4.1 against 2.7 us a launch.  A
-// gated-off launch costs 0.16 ns a block, so above 65,536 clusters (10 us)
-// blocks are of four again: 2.1 M sparse beads, 262,000 clusters, 1.24 ms a
-// step with single waves, 1.18 with four.
-constexpr int32_t list_waves(int32_t ncl) { return ncl > 16384 && ncl <= 65536 ? 1 : 4; }
+// where a gated-off launch is, which costs 0.16 ns a block: at 31,250 clusters
+// of 2,500 entries, a build every 10 steps, 67 against 77 us a step; of 100
+// entries, hardly ever built, 108 against 103; at two lists of 12,000 with few
+// rebuilds 4.1 against 2.7 us a launch.  A build's gain goes with the entries
+// and is the launches' loss at about 1,000.  Above 65,536 clusters (10 us a
+// launch) four again: 2.1 M sparse beads, 262,000 clusters, 1.24 ms a step with
+// single waves, 1.18 with four.
+constexpr int32_t list_waves(int32_t ncl, int32_t cap)
+{
+    return ncl > 16384 && ncl <= 65536 && cap >= 1024 ? 1 : 4;
+}
 
 __global__ void __launch_bounds__(BLOCK) k_cluster_list(ListSet set)
 {
@@ -720,7 +725,10 @@ void launch_list_build(const ListArgs *a, int32_t nlists, hipStream_t s)
         set.list[l] = a[l];
     if (nlists > 0 && a[0].ncl > 0)
     {
-        const int32_t W = list_waves(a[0].ncl);
+        int32_t cap = 0; // of the longest list
+        for (int32_t l = 0; l < nlists; ++l)
+            cap = a[l].cap > cap ? a[l].cap : cap;
+        const int32_t W = list_waves(a[0].ncl, cap);
         k_cluster_list<<<dim3((a[0].ncl + W - 1) / W, nlists), 64 * W, W * EX_SLOTS * sizeof(uint32_t), s>>>(set);
     }
 }

@@ -184,3 +184,32 @@ def test_a_negative_radius_is_not_a_number(mode, layout):
     assert np.isnan(f[bad]).all() and np.isnan(e[_abi.E_STERIC]) and np.isfinite(e0).all()
     far = d > 1.0001 * p.steric_cutoff
     assert far.any() and np.array_equal(f[far], f0[far])
+
+
+@pytest.mark.parametrize("clusters", [16384, 65536])
+def test_list_build_blocks_change(clusters):
+    """Long lists on both sides of the cluster counts at which the build's
+    blocks change from four waves to one and back: eight beads far away add a
+    cluster and no force, so the others' are the same (FP64 sums in another
+    order, rounded once)."""
+    n = 8 * clusters
+    rng = np.random.default_rng(clusters)
+    per = int(np.ceil(n ** (1 / 3)))
+    site = np.stack(np.unravel_index(np.arange(n), (per, per, per)), 1)
+    x = ((site + rng.uniform(-0.2, 0.2, (n, 3))) * 3.0).astype(np.float32)
+    far = (np.full((8, 3), per * 3.0 + 100.0) + 40.0 * np.arange(8)[:, None]).astype(np.float32)
+    p = _abi.default_params()
+    p.steric_enable, p.steric_mode, p.steric_cutoff = 1, _abi.STERIC_LINEAR, 16.0
+    got = []
+    for beads in (x, np.concatenate([x, far])):
+        net = SpringNetwork(p)
+        net.setParticles(beads.reshape(-1), radius=np.full(len(beads), 5.0, np.float32))
+        print("n", len(beads), flush=True)
+        f, e = net.computeForces()
+        assert net.counters()["list_cap"] >= 1024
+        got.append((f[:n], e[_abi.E_STERIC], net.countPairs(_abi.NS_STERIC)))
+        assert not f[n:].any()
+        net.close()
+    (fa, ea, pa), (fb, eb, pb) = got
+    assert pa == pb and abs(ea - eb) <= 1e-9 * abs(ea)
+    assert np.abs(fa - fb).max() <= 1.2e-7 * np.abs(fa).max()
