@@ -243,7 +243,8 @@ __device__ inline void probe_pair(const ProbeArgs &p, const float4 q, float4 pi,
 // flight per lane: the edge words of the next D load while these gather and
 // compute (two dependent loads per edge: the word, then x_j).  A lane with null
 // edges alone adds nothing, also for a particle whose position is not finite
-// (a null edge of a lane that has a real one cannot make that one's sum worse).
+// (a null edge of a lane that has a real one cannot make that one's sum worse);
+// with ALL the caller sees to that, a row at a time (lost_row).
 //
 // Every edge in flight costs a row its loads, needed or not: with ALL none is
 // skipped, which suits D = 4 beside the pair walk (skipped there: 71 -> 69 us
@@ -285,8 +286,16 @@ __device__ inline void row_springs(const SpringArgs &a, EdgeRow &er, RowSum<COMP
             l[u] = ln[u];
         }
     }
-    if (!real)
+    if (!ALL && !real)
         sum.fx = sum.fy = sum.fz = sum.e = 0.0;
+}
+
+// Whether row's springs add nothing although its position, not being finite,
+// made its null edges' sums NaN: a static row, or one without springs.
+__device__ inline bool lost_row(const SpringArgs &a, int32_t row, float4 pi, uint32_t fli)
+{
+    return !(fabsf(pi.x) < INFINITY && fabsf(pi.y) < INFINITY && fabsf(pi.z) < INFINITY) &&
+           ((fli & PF_STATIC) || a.sp_e[(size_t)a.sp_ptr[row] * EDGE_PAD].x == (uint32_t)row);
 }
 
 // What a particle's row adds to the sums beside its force: energies, and the

@@ -113,6 +113,7 @@ __global__ void __launch_bounds__(BLOCK) k_step(PairArgs p, SpringArgs a)
     RowOut o;
     const float4 pi = a.pos[row];
     const uint32_t fli = fbits(a.jprm[row].w);
+    const bool lost = lost_row(a, row, pi, fli);
     if (!(fli & PF_STATIC))
     {
         float4 li = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -126,7 +127,13 @@ __global__ void __launch_bounds__(BLOCK) k_step(PairArgs p, SpringArgs a)
             fy += f.y;
             fz += f.z;
         }
-        finish_row<true, COMP>(a, row, pi, li, fli, spring[0] + fx, spring[1] + fy, spring[2] + fz, o);
+        if (!lost)
+        {
+            fx += spring[0];
+            fy += spring[1];
+            fz += spring[2];
+        }
+        finish_row<true, COMP>(a, row, pi, li, fli, fx, fy, fz, o);
     }
     if (ENERGY)
     {
@@ -139,7 +146,7 @@ __global__ void __launch_bounds__(BLOCK) k_step(PairArgs p, SpringArgs a)
             en.z += v.z;
         }
         p.epp[row] = en;
-        a.eps[row] = make_double4(spring[3], o.eke, o.eimp, o.efld);
+        a.eps[row] = make_double4(lost ? 0.0 : spring[3], o.eke, o.eimp, o.efld);
     }
 }
 
