@@ -282,3 +282,22 @@ def test_event_timing_changes_no_bit(recorded, swept):
         got.append((x, v) + tuple(net.adjointBackward(2.0 * (x.astype(np.float64) - y) / s.n)))
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+def test_gradients_above_forty_thousand_beads_match_fp64():
+    """One wave per cluster (above 5,120 clusters) in the adjoint pair kernel:
+    the gradients of two reversed steps against the oracle's.  The springs
+    start stretched: dL/dk goes with the extension, which the FP32 positions
+    hold to 4e-6 A (half an ulp of 77 A), 2e-5 of an extension of 0.2 A."""
+    s = workloads.generate(1, seed=17, n=40968)
+    y = _target(s)
+    rng = np.random.default_rng(17)
+    s.x = (s.x + rng.normal(scale=0.05, size=s.x.shape)).astype(np.float32)
+    net = SpringNetwork.from_system(s)
+    loss, dk, dl, dq = net.adjoint(2, y, 0)
+    o = po.Oracle(s)
+    lo, dko, dlo, dqo = o.adjoint(2, y.astype(np.float64))
+    o.close()
+    _log(f"n={s.n}: dk {_rel(dk, dko):.1e} dl0 {_rel(dl, dlo):.1e} dq {_rel(dq, dqo):.1e}")
+    assert abs(loss - lo) <= 1e-6 * lo
+    assert _rel(dk, dko) <= GRAD_RTOL and _rel(dl, dlo) <= GRAD_RTOL and _rel(dq, dqo) <= GRAD_RTOL

@@ -39,7 +39,9 @@ def _compare(s, **over):
     (xq, vq, eq), (xc, vc, ec) = got
     assert np.abs(vq - vc).max() <= TOL * max(np.abs(vc).max(), 1e-12)
     assert np.abs(xq - xc).max() <= TOL * max(np.abs(xc).max(), 1.0)
-    assert np.allclose(eq, ec, rtol=TOL, atol=TOL * np.abs(ec).max())
+    # every energy to its own size (sums whose terms nearly cancel: to 1e-9)
+    assert np.allclose(eq, ec, rtol=TOL, atol=1e-9)
+    return xq, vq, eq
 
 
 def _perturbed(config, n, seed):
@@ -71,8 +73,21 @@ def test_terms(over):
     if over.get("steric_mode") == _abi.STERIC_ZACHARIAS_8_6:
         s.radius = np.sqrt(s.radius).astype(np.float32)  # products of radii
     if over.get("hydrophobicity_enable"):
-        s.hydro = rng.uniform(-1.0, 1.0, s.n).astype(np.float32) * 1e-18
-    _compare(s, **over)
+        # the force goes with h_i h_j: 100 times that of h = 1, which changes the
+        # velocities (2e-3 at most) by 2e-7 in three steps
+        s.hydro = rng.uniform(-10.0, 10.0, s.n).astype(np.float32)
+    _, v, e = _compare(s, **over)
+    if over.get("hydrophobicity_enable"):
+        # the term is there to be compared: without it the energy is none and
+        # the velocities differ by far more than the comparison allows
+        assert abs(e[_abi.E_HYDROPHOBIC]) > 0.0
+        p = s.params.copy()
+        for k, w in over.items():
+            setattr(p, k, w)
+        p.hydrophobicity_enable = 0
+        _, v0, e0 = _state(s, p)
+        assert e0[_abi.E_HYDROPHOBIC] == 0.0
+        assert np.abs(v - v0).max() >= 1e3 * TOL * np.abs(v).max()
 
 
 def test_distant_beads_have_empty_lists():
