@@ -326,12 +326,15 @@ def main():
     layout = int(s.params.pair_layout) if tuned is None else tuned[2]
     if layout == _abi.PAIR_QUEUES:
         # one kernel takes the (last) list's pairs, the springs and the
-        # integrator; the pairs' operations and the springs' bytes are both its
+        # integrator: priced against the longer of its two floors, the springs'
+        # bytes and the pairs' operations
         step_ms = pair_ms + spring_ms
-        kernels = {"step": valu(step_ms)}
-        mem = hbm(step_ms)
-        kernels["step"].update({"alg_bytes": b_alg, "uniform_stiffness": k_uniform, "hbm_gbs": mem["achieved"],
-                                "hbm_frac": mem["frac"], "earlier_lists_pair_ms": pair_ms})
+        floors = sorted((hbm(step_ms), valu(step_ms)), key=lambda f: -f["frac"])
+        kernels = {"step": {**floors[1], **floors[0], "other_floor": {k: floors[1][k] for k in
+                                                                      ("bound", "achieved", "peak", "unit", "frac")},
+                            "earlier_lists_pair_ms": pair_ms,
+                            "note": "one kernel for pairs, springs and integrator; bound by VALU issue on dense "
+                                    "networks whatever the longer floor (profiles/pair_valu_250k.md)"}}
         dom = "step"
     else:
         kernels = {"spring_integrate": hbm(spring_ms), "pair": valu(pair_ms)}

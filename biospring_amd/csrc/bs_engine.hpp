@@ -89,6 +89,9 @@ constexpr int32_t EDGE_PAD = 8;
 // leave the chip's 1024 SIMDs idle or end in a tail: measured per step with 1,
 // 2 and 4 waves at 1,126 clusters 164, 126 and 118 us, at 3,752 clusters 119,
 // 108 and 112, at 6,250 (short lists) 49, 54 and 68, at 31,250 500, 507 and 598.
+// Where the line between one and two lies depends on the lists too: dense beads
+// (lists of 2,300) still gain at 6,250 clusters (132 -> 117), 12,500 (219 -> 207)
+// and 25,000 (383 -> 382), which a rule on the cluster count alone leaves.
 constexpr int32_t pair_waves(int32_t ncl) { return ncl <= 2048 ? 4 : ncl <= 5120 ? 2 : 1; }
 
 // A list's plan for the queue layout: one record per stretch of 64 words

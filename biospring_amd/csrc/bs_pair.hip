@@ -3,10 +3,12 @@
 // Particles are grouped into i-clusters of 8 consecutive internal indices
 // (the internal order is spatial).  A neighbour list holds, per i-cluster,
 // entries j | m << 24 where the 8-bit m marks which of the cluster's particles
-// have j within the list radius and not spring-bonded.  Kernels run one wave64
-// per i-cluster with lanes laid out as 8 i x 8 entries, so that every load of
-// a j's data serves 8 lanes, and accumulate forces on i only (each pair is
-// visited from both sides): no atomics, bitwise reproducible.
+// have j within the list radius and not spring-bonded.  The queue layout's
+// kernels run one to four wave64s per i-cluster (pair_waves), which evaluate
+// listed pairs from LDS queues; the cluster layout's run one, with lanes laid
+// out as 8 i x 8 entries, so that every load of a j's data serves 8 lanes.  All
+// accumulate forces on i only (each pair is visited from both sides): no
+// atomics, bitwise reproducible.
 #include "bs_pairterm.hpp"
 
 #include <cmath>

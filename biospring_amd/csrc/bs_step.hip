@@ -5,9 +5,10 @@
 // gather waits on memory (its edge words are read once a step, from HBM) and
 // the pair walk keeps the VALU busy, so waves in one phase run beside waves
 // in the other, and the pair forces never leave the chip.  At 250,000 dense
-// beads a step takes 0.50 ms, against 0.56 ms with the two as kernels of their
-// own before the pair walk was planned and 0.53 ms after.  Measured and left
-// out: one spring edge per lane between the stretches of the pair walk (its
+// beads a step takes 0.46 ms, 0.40 of it here.  When the kernels were joined a
+// step took 0.50 ms, against 0.56 ms with the two as kernels of their own before
+// the pair walk was planned and 0.53 ms after (list builds have become shorter
+// since).  Measured then and left out: one spring edge per lane between the stretches of the pair walk (its
 // partner in flight meanwhile: 0.53 ms; 8-lane rows read a line in two halves,
 // a stretch apart); half the blocks taking their pairs first (0.51 ms; the
 // second copy's registers cost a wave per SIMD); six or eight spring edges in
