@@ -633,6 +633,22 @@ void plan_lists(bs_handle *h)
         l.radius = l.rc + std::max(p.list_skin, 0.0f);
 }
 
+// Whether one workgroup bins this system (k_bin).  It saves the launches of
+// the chain on steps that do not rebuild, and is slower than the chain's
+// workgroups on steps that do: rebuilding every step, 40 steps of 2,000, 9,001
+// and 16,384 sparse beads with one list take 2.3, 2.9 and 4.0 ms with it, 1.9,
+// 2.1 and 2.8 without; every 10 steps 0.71, 0.83 and 1.05 against 1.19, 1.30 and
+// 1.40.  It bins all lists in one launch, so with three it is the faster one
+// either way (9,001 dense beads, every step: 10.9 against 13.8 ms; 16,384:
+// 15.5, 15.7), with two up to half that size (sparse, every step: 6,000 beads
+// 3.5 against 3.6 ms, 9,001 4.1 against 3.8).
+bool bins_small(const bs_handle *h)
+{
+    const bool every_step = h->p.rebuild_interval == 1 || !(h->p.list_skin > 0.0f);
+    const size_t nl = h->lists.size();
+    return h->n <= BIN_MAX && (!every_step || nl > 2 || (nl == 2 && h->n <= BIN_MAX / 2));
+}
+
 // Engine grid dimensions of a list from the current host positions.
 void plan_grid(bs_handle *h, List &l, const std::vector<float4> &shift)
 {
@@ -664,23 +680,14 @@ void plan_grid(bs_handle *h, List &l, const std::vector<float4> &shift)
         l.dims[c] = (int32_t)d;
         total *= d;
     }
-    // a small system is binned by one workgroup, its cell counts in LDS
-    while (h->n <= BIN_MAX && total > BIN_CELLS)
+    // A small system's cell counts are held in LDS.  Otherwise no more cells
+    // than particles: in sparse or spread-out systems finer ones are mostly
+    // empty, and the scan reads every one (coarse-grained beads with a 5 A
+    // radius: 205,000 cells for 50,000 beads).
+    const int64_t most = bins_small(h) ? BIN_CELLS : std::max<int64_t>(h->n, 4096);
+    while (total > most)
     {
-        const double f = std::cbrt((double)BIN_CELLS / (double)total) * 0.999;
-        total = 1;
-        for (int c = 0; c < 3; ++c)
-        {
-            l.dims[c] = std::max(1, (int)(l.dims[c] * f));
-            total *= l.dims[c];
-        }
-    }
-    // no more cells than particles: in sparse or spread-out systems finer ones
-    // are mostly empty, and the scan reads every one (coarse-grained beads with
-    // a 5 A radius: 205,000 cells for 50,000 beads)
-    while (h->n > BIN_MAX && total > h->n)
-    {
-        const double f = std::cbrt((double)h->n / (double)total) * 0.999;
+        const double f = std::cbrt((double)most / (double)total) * 0.999;
         total = 1;
         for (int c = 0; c < 3; ++c)
         {
@@ -2262,7 +2269,7 @@ int do_setup(bs_handle *h)
     for (auto &l : h->lists)
     {
         ALLOC(l.cln, int32_t, h->ncl);
-        if (n <= BIN_MAX)
+        if (bins_small(h))
         {
             ALLOC(l.bstart, int32_t, l.ncells + 1);
             ALLOC(l.bxs, float4, n);

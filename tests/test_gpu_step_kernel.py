@@ -228,3 +228,22 @@ def test_list_build_blocks_change(clusters):
     (fa, ea, pa), (fb, eb, pb) = got
     assert pa == pb and abs(ea - eb) <= 1e-9 * abs(ea)
     assert np.abs(fa - fb).max() <= 1.2e-7 * np.abs(fa).max()
+
+
+@pytest.mark.parametrize("n", [63, 1001, 8192, 8193, 16384])
+@pytest.mark.parametrize("cutoffs", [(12.0, 12.0), (10.0, 12.0)], ids=["one_list", "two_lists"])
+def test_rebuilding_every_step(n, cutoffs):
+    """Systems that rebuild in every step (an interval of 1, or no skin) leave
+    the one-workgroup binning: the same steps as with the lists kept."""
+    s = _perturbed(1, n, 6)
+    got = []
+    for interval, skin in ((0, 0.25), (1, 0.25), (0, 0.0)):
+        p = s.params.copy()
+        p.rebuild_interval, p.list_skin = interval, skin
+        p.steric_cutoff, p.electrostatic_cutoff = cutoffs
+        got.append(_state(s, p, 4))
+    (x0, v0, e0) = got[0]
+    for x, v, e in got[1:]:
+        assert np.abs(v - v0).max() <= TOL * max(np.abs(v0).max(), 1e-12)
+        assert np.abs(x - x0).max() <= TOL * max(np.abs(x0).max(), 1.0)
+        assert np.allclose(e, e0, rtol=TOL, atol=1e-9)
